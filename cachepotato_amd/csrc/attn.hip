@@ -494,253 +494,390 @@ __device__ static inline int head_on_xcd(int b, int H, int KV) {
     return x * per_xcd + i;                    /* XCD x takes heads x*per_xcd .. +per_xcd-1 */
 }
 
-/* Many tokens on MFMA: grid (KV, ceil(T / (64/G))), 256 threads, HD == 128, G = H/KV
-   dividing 16. Workgroup (kh, b) takes 64 query rows, wavefront w rows 16w..16w+15, row r =
-   (token b*TB + r / G, head kh*G + r % G) with TB = 64/G tokens; all of them share each tile
-   of AMT key positions of kv head kh staged in LDS as hi/lo f16 halves (x = hi + lo, hi =
-   f16(x), lo = f16(x - hi): 22 significant bits). Per tile:
+/* The maximum and the sum over each half of the wavefront (lanes 0-31, 32-63), the same
+   bits in every lane of the half: DPP steps within rows of 16 lanes, then one exchange
+   between the two rows of the half. */
+__device__ static inline float half_max(float v) {
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_QUAD_1032, 0xf, 0xf, false)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_QUAD_2301, 0xf, 0xf, false)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_ROW_HALF_MIRROR, 0xf, 0xf, false)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_ROW_MIRROR, 0xf, 0xf, false)));
+    return fmaxf(v, __shfl_xor(v, 16));
+}
+__device__ static inline float half_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_QUAD_1032, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_QUAD_2301, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_ROW_HALF_MIRROR, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_ROW_MIRROR, 0xf, 0xf, false));
+    return v + __shfl_xor(v, 16);
+}
+
+/* Many tokens on MFMA: grid (KV, ceil(T / TB), splits), 256 threads, HD == 128, G = H/KV dividing
+   16. Workgroup (kh, b, z) takes ROWS = 64 * QS query rows, wavefront w the QS sets of 16 rows
+   from 16 * QS * w on, row r = (token b*TB + r / G, head kh*G + r % G) with TB = ROWS / G
+   tokens, over split z of the block's keys, of which there are at most ns (ns == 1: one split
+   with all of them; splits past the block's last leave at once). All rows share each tile of
+   AMT key positions of kv head kh staged in LDS as hi/lo f16 halves (x = hi + lo, hi = f16(x),
+   lo = f16(x - hi): 22 significant bits). Per tile:
      S^T = K . Q^T on v_mfma_f32_16x16x32_f16 (A = key rows, B = the wavefront's query rows,
        held in registers for the whole call), each product as hi.hi + lo.hi + hi.lo (the lo.lo
        term, below 2^-22 of the sum, is not formed); lane l then holds the scores of query
-       l%16 against keys 16kt + 4(l/16) + i (kt, i < 4), divided by sqrt(HD) and masked
-       (key j > the query's position, or past the cache: -inf);
-     online softmax per query (the 4 lanes of a query reduce by shuffles): running maximum m,
-       sum l of expf(s - m) with the reference's expf, the accumulators rescaled by
-       expf(m_old - m_new) when the maximum grows;
+       l%16 against keys 16kt + 4(l/16) + i (kt < 2, i < 4), masked where the tile reaches past
+       one of the wavefront's positions (key j > the query's position, or past the cache: -inf);
+     online softmax per query in powers of two: with c = log2(e) / sqrt(HD) and M = c * (the
+       largest score so far) the probabilities are exp2(c s - M), one fused multiply-add and
+       the hardware exponential (1 ulp); the 4 lanes of a query share the maximum by shuffles,
+       each adds its own part of the sum l, and the accumulators are rescaled by
+       exp2(M_old - M_new) in the tiles where some maximum of the wavefront grew;
      O += P . V, A = the lane's own probabilities (hi/lo, in the lane order above: slot 8g + j
-       of a 32-key step u is key 32u + 4g + j for j < 4 and 32u + 16 + 4g + j - 4 after), B =
-       value rows read in that key order from LDS, where a value tile is laid out as
-       [key / 4][dim][key % 4] so that a lane's four consecutive keys of one dimension are one
-       8-byte read.
-   out = O / l, written as ao (fp32) or, aoh not null, as the hi/lo planes of the output
-   projection. The sums run in another order than the reference's two-pass softmax
+       is key 4g + j for j < 4 and 16 + 4g + j - 4 after), B = value rows read in that key
+       order from LDS, where a value tile is laid out as [key / 4][dim][key % 4] so that a
+       lane's four consecutive keys of one dimension are one 8-byte read.
+   ns == 1: out = O / l, written as ao (fp32) or, aoh not null, as the hi/lo planes of the
+   output projection. ns > 1: split z's O, M and l are left in pacc / pml at row (z*T + t)*H + h
+   for k_attn_merge. The sums run in another order than the reference's two-pass softmax
    (qwen3_moe.c:127-157) and the products carry 22-bit operands, so the output agrees to
-   rounding. Dynamic LDS: amma_lds_bytes(). */
-#define AMT 64              /* k_attn_mma: key positions per tile */
-#define AMQ 64              /* k_attn_mma: query rows per workgroup (4 wavefronts of 16) */
-#define AMLK (128 + 8)      /* k_attn_mma: K row stride in halves (16 B of padding) */
-#define AMMA_MIN_T 2        /* k_attn_mma from this many tokens on (HD 128, G | 16) */
+   rounding. Dynamic LDS: amma_lds_bytes().
 
-#define AMMA_BUF (2 * AMT * AMLK + 2 * AMT * 128)   /* halves of one K/V tile buffer */
+   What bounds it, at 512 tokens over 4096 positions: per tile and 32 rows of a wavefront 96
+   MFMAs of 16 cycles, and beside them the operand reads from LDS and the softmax and staging
+   on the VALU. Two sets of rows per wavefront (QS = 2) use each key and value operand read
+   from LDS twice; tiles of 32 keys, double-buffered in 72 KiB, let two workgroups share a CU,
+   so that one's MFMAs run beside the other's softmax; the splits fill the chip where the
+   query blocks do not. That kernel 365 -> 120 us (MFMAs 32 % of it), and 67 -> 9 at 21 tokens
+   over 700 positions, against tiles of 64 keys over one set of rows, one workgroup per CU,
+   unsplit, and an exponential in double precision. */
+#define AMT 32              /* k_attn_mma: key positions per tile */
+#define AMLK (128 + 8)      /* k_attn_mma: K row stride in halves (16 B of padding) */
+#define AMLV (4 * 128 + 64) /* k_attn_mma: V stride of 4 keys in halves (128 B of padding: the
+                               lanes' 8-byte reads of two neighbouring key groups then fall in
+                               distinct banks) */
+#define AMMA_MIN_T 2        /* k_attn_mma from this many tokens on (attn_mma_shape) */
+#define AMMA_MAX_NS 32      /* k_attn_merge: splits, one per lane of a row's 32 */
+/* The launch (whole attention half of a layer, us):
+   AMMA_QS1_ROWS: rows per kv head up to which a wavefront takes one set of 16: few rows are
+     bound by the launch's length, which one set shortens (37 tokens over 4715 positions 65.4
+     with two sets, 61.4 with one; 96 tokens, whole layers with the MoE half, 209 and 207; at
+     100 tokens over 2000 positions the two are equal);
+   AMMA_WGS: workgroups that the key splits aim at, two per CU (512 tokens over 3584 positions:
+     256 workgroups 238, 512 214, 768 or 1024 224);
+   AMMA_MIN_KEYS: keys per split at least (138 tokens at position 0: 58.7 with 32, 60.0 with
+     64, 65.6 with 128). */
+#define AMMA_QS1_ROWS 1024
+#define AMMA_WGS 512
+#define AMMA_MIN_KEYS 32
+
+#define AMMA_BUF (2 * AMT * AMLK + 2 * (AMT / 4) * AMLV)   /* halves of one K/V tile buffer */
 
 static inline size_t amma_lds_bytes() { return sizeof(_Float16) * 2 * (size_t)AMMA_BUF; }
 
+/* the keys per split of a block that ends at key n: whole tiles */
+__device__ static inline int amma_split_keys(int n, int ns) {
+    return ((n + ns - 1) / ns + AMT - 1) / AMT * AMT;
+}
+
 /* k_attn_mma's staging of one key tile, in two halves so that the next tile's loads fly
-   while the current one is computed: thread tid takes items tid and tid + 256, item = (key
-   group kg of 4 keys, float4 column c4) of kv head kh, keys from j0 (clamped to n - 1) */
-__device__ __forceinline__ static void amma_load(float4 (&kv)[2][4], float4 (&vv)[2][4],
+   while the current one is computed: thread tid takes 4 keys of key group tid / 32 and the
+   float4 column tid % 32 of kv head kh, keys from j0 (clamped to n - 1) */
+__device__ __forceinline__ static void amma_load(float4 (&kv)[4], float4 (&vv)[4],
                                                  const float *__restrict__ kc,
                                                  const float *__restrict__ vc, int kvw, int kh,
                                                  int j0, int n) {
+    const int kg = threadIdx.x >> 5, c4 = threadIdx.x & 31;
 #pragma unroll
-    for (int it = 0; it < 2; it++) {
-        const int item = threadIdx.x + 256 * it, kg = item >> 5, c4 = item & 31;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int jj = min(j0 + 4 * kg + e, n - 1);
-            const size_t off = (size_t)jj * kvw + (size_t)kh * 128 + 4 * c4;
-            kv[it][e] = *(const float4 *)(kc + off);
-            vv[it][e] = *(const float4 *)(vc + off);
-        }
+    for (int e = 0; e < 4; e++) {
+        const int jj = min(j0 + 4 * kg + e, n - 1);
+        const size_t off = (size_t)jj * kvw + (size_t)kh * 128 + 4 * c4;
+        kv[e] = *(const float4 *)(kc + off);
+        vv[e] = *(const float4 *)(vc + off);
     }
 }
 
 /* the loaded items as hi/lo halves into buffer buf: K rows [key][AMLK], V as
-   [key / 4][dim][key % 4] */
-__device__ __forceinline__ static void amma_store(const float4 (&kv)[2][4],
-                                                  const float4 (&vv)[2][4], _Float16 *buf) {
-    typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+   [key / 4][dim][key % 4] with stride AMLV */
+__device__ __forceinline__ static void amma_store(const float4 (&kv)[4], const float4 (&vv)[4],
+                                                  _Float16 *buf) {
     _Float16 *kh_s = buf, *kl_s = kh_s + AMT * AMLK;
-    _Float16 *vh_s = kl_s + AMT * AMLK, *vl_s = vh_s + AMT * 128;
+    _Float16 *vh_s = kl_s + AMT * AMLK, *vl_s = vh_s + AMT / 4 * AMLV;
+    const int kg = threadIdx.x >> 5, c4 = threadIdx.x & 31;
 #pragma unroll
-    for (int it = 0; it < 2; it++) {
-        const int item = threadIdx.x + 256 * it, kg = item >> 5, c4 = item & 31;
+    for (int e = 0; e < 4; e++) {
+        const f16pair2 a = split_f16x2(kv[e].x, kv[e].y), b = split_f16x2(kv[e].z, kv[e].w);
+        *(uint2 *)(kh_s + (4 * kg + e) * AMLK + 4 * c4) = make_uint2(a.hi, b.hi);
+        *(uint2 *)(kl_s + (4 * kg + e) * AMLK + 4 * c4) = make_uint2(a.lo, b.lo);
+    }
+    const float v[4][4] = {{vv[0].x, vv[1].x, vv[2].x, vv[3].x},
+                           {vv[0].y, vv[1].y, vv[2].y, vv[3].y},
+                           {vv[0].z, vv[1].z, vv[2].z, vv[3].z},
+                           {vv[0].w, vv[1].w, vv[2].w, vv[3].w}};
+    _Float16 *ph = vh_s + kg * AMLV + 16 * c4, *pl = vl_s + kg * AMLV + 16 * c4;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float x[4] = {kv[it][e].x, kv[it][e].y, kv[it][e].z, kv[it][e].w};
-            half4_t h, lo;
+    for (int d = 0; d < 4; d += 2) {
+        const f16pair2 a = split_f16x2(v[d][0], v[d][1]), b = split_f16x2(v[d][2], v[d][3]);
+        const f16pair2 e = split_f16x2(v[d + 1][0], v[d + 1][1]),
+                       f = split_f16x2(v[d + 1][2], v[d + 1][3]);
+        *(uint4 *)(ph + 4 * d) = make_uint4(a.hi, b.hi, e.hi, f.hi);
+        *(uint4 *)(pl + 4 * d) = make_uint4(a.lo, b.lo, e.lo, f.lo);
+    }
+}
+
+template <int QS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_mma(
+    const float *__restrict__ q, const float *__restrict__ kc, const float *__restrict__ vc, int H,
+    int KV, int T, int pos0_arg, const int *__restrict__ pos_dev, int lim,
+    int ns, float *__restrict__ pacc, float2 *__restrict__ pml, float *__restrict__ ao,
+    _Float16 *__restrict__ aoh, _Float16 *__restrict__ aol) {
+    constexpr int HD = 128;
+    extern __shared__ __align__(16) _Float16 smh[];   /* two tile buffers (amma_store) */
+    const int tid = threadIdx.x, l = tid & 63, g = l >> 4, c = l & 15;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int G = H / KV, TB = 64 * QS / G, kh = blockIdx.x, t0 = blockIdx.y * TB;
+    const int z = blockIdx.z;
+    const int kvw = KV * HD;
+    const int pos0 = pos_dev ? *pos_dev : pos0_arg;
+    const int tl = min(T, t0 + TB) - 1;          /* the last token of the block */
+    auto put = [&](int t, int h, int d, float v) {
+        const size_t e = ((size_t)t * H + h) * HD + d;
+        if (aoh) {
+            const f16pair p = split_f16(v);
+            aoh[e] = p.hi;
+            aol[e] = p.lo;
+        } else {
+            ao[e] = v;
+        }
+    };
+    if (pos0 < 0 || pos0 + t0 >= lim) {          /* no position of the block is in the cache */
+        if (ns == 1)
+            for (int i = tid; i < (tl - t0 + 1) * G * HD; i += 256)
+                put(t0 + i / (G * HD), kh * G + i / HD % G, i % HD, __int_as_float(0x7fc00000));
+        return;
+    }
+    const int n = min(pos0 + tl + 1, lim);       /* keys 0 .. n-1 */
+    const int per = amma_split_keys(n, ns), jb = z * per, je = min(n, jb + per);
+    if (jb >= je) return;
+    /* this lane's queries (scores, softmax state): rows 16 (QS w + s) + c; rows past the
+       block's last token compute with its query and are not stored; a wavefront with no row
+       of the block only stages */
+    const bool active = 16 * QS * w < (tl - t0 + 1) * G;
+    int pq[QS];                                  /* their last keys */
+    half8_t qh[QS][4], ql[QS][4];                /* B operand: dims 32s4 + 8g .. + 7 */
 #pragma unroll
-            for (int d = 0; d < 4; d++) {
-                const f16pair p = split_f16(x[d]);
-                h[d] = p.hi;
-                lo[d] = p.lo;
+    for (int s = 0; s < QS; s++) {
+        const int r = 16 * (QS * w + s) + c, tq = min(t0 + r / G, tl);
+        pq[s] = pos0 + tq;
+        const float *qr = q + ((size_t)tq * H + kh * G + r % G) * HD + 8 * g;
+#pragma unroll
+        for (int s4 = 0; s4 < 4; s4++)
+            split_hilo8(*(const float4 *)(qr + 32 * s4), *(const float4 *)(qr + 32 * s4 + 4),
+                        qh[s][s4], ql[s][s4]);
+    }
+    const int pfirst = pos0 + min(t0 + 16 * QS * w / G, tl);   /* the wavefront's first position */
+    const float cs = 1.44269504088896341f * 0.08838834764831845f;   /* log2(e) / sqrt(128) */
+    float m[QS], M[QS], lsum[QS];
+    f32x4_t o[QS][HD / 16];
+#pragma unroll
+    for (int s = 0; s < QS; s++) {
+        m[s] = -INFINITY;
+        M[s] = 0.0f;
+        lsum[s] = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; dt++) o[s][dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    float4 kv[4], vv[4];
+    amma_load(kv, vv, kc, vc, kvw, kh, jb, n);
+    amma_store(kv, vv, smh);
+    __syncthreads();
+    for (int j0 = jb, cur = 0; j0 < je; j0 += AMT, cur ^= 1) {
+        /* the next tile's loads fly while this one is computed */
+        const bool more = j0 + AMT < je;
+        if (more) amma_load(kv, vv, kc, vc, kvw, kh, j0 + AMT, n);
+        if (active) {
+            const _Float16 *kh_s = smh + cur * AMMA_BUF, *kl_s = kh_s + AMT * AMLK;
+            const _Float16 *vh_s = kl_s + AMT * AMLK, *vl_s = vh_s + AMT / 4 * AMLV;
+            /* scores: st[s][kt][i] = S[query c of set s][key j0 + 16kt + 4g + i] */
+            f32x4_t st[QS][2];
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++) {
+#pragma unroll
+                for (int s = 0; s < QS; s++) st[s][kt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                const _Float16 *kr = kh_s + (16 * kt + c) * AMLK + 8 * g;
+                const _Float16 *kl = kl_s + (16 * kt + c) * AMLK + 8 * g;
+#pragma unroll
+                for (int s4 = 0; s4 < 4; s4++) {
+                    const half8_t ah = *(const half8_t *)(kr + 32 * s4);
+                    const half8_t al = *(const half8_t *)(kl + 32 * s4);
+#pragma unroll
+                    for (int s = 0; s < QS; s++)
+                        st[s][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, qh[s][s4], st[s][kt], 0, 0, 0);
+#pragma unroll
+                    for (int s = 0; s < QS; s++)
+                        st[s][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, qh[s][s4], st[s][kt], 0, 0, 0);
+#pragma unroll
+                    for (int s = 0; s < QS; s++)
+                        st[s][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, ql[s][s4], st[s][kt], 0, 0, 0);
+                }
             }
-            *(half4_t *)(kh_s + (4 * kg + e) * AMLK + 4 * c4) = h;
-            *(half4_t *)(kl_s + (4 * kg + e) * AMLK + 4 * c4) = lo;
+            if (j0 + AMT - 1 > pfirst) {         /* some query of the wavefront ends in the tile */
+#pragma unroll
+                for (int s = 0; s < QS; s++)
+#pragma unroll
+                    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const int j = j0 + 16 * kt + 4 * g + i;
+                            st[s][kt][i] = j <= pq[s] && j < n ? st[s][kt][i] : -INFINITY;
+                        }
+            }
+            half8_t ph[QS], pl[QS];
+#pragma unroll
+            for (int s = 0; s < QS; s++) {
+                float mn = m[s];
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) mn = fmaxf(mn, st[s][kt][i]);
+                mn = fmaxf(mn, __shfl_xor(mn, 16));
+                mn = fmaxf(mn, __shfl_xor(mn, 32));
+                if (__any(mn > m[s])) {
+                    /* a query without a key yet (m = -inf): its sums are zero, and M stays 0
+                       so that its masked scores give exp2(-inf) = 0 */
+                    const float Mn = mn == -INFINITY ? 0.0f : cs * mn;
+                    const float f = m[s] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M[s] - Mn);
+                    m[s] = mn;
+                    M[s] = Mn;
+                    lsum[s] *= f;
+                    /* the accumulators hold queries 4g + i: their factors from lanes 4g + i */
+                    float fi[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) fi[i] = __shfl(f, 4 * g + i);
+#pragma unroll
+                    for (int dt = 0; dt < HD / 16; dt++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) o[s][dt][i] *= fi[i];
+                }
+                float p[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    p[j] = __builtin_amdgcn_exp2f(fmaf(st[s][j >> 2][j & 3], cs, -M[s]));
+                    lsum[s] += p[j];
+                }
+                uint4 hi, lo;
+                f16pair2 a = split_f16x2(p[0], p[1]);
+                hi.x = a.hi;
+                lo.x = a.lo;
+                a = split_f16x2(p[2], p[3]);
+                hi.y = a.hi;
+                lo.y = a.lo;
+                a = split_f16x2(p[4], p[5]);
+                hi.z = a.hi;
+                lo.z = a.lo;
+                a = split_f16x2(p[6], p[7]);
+                hi.w = a.hi;
+                lo.w = a.lo;
+                ph[s] = __builtin_bit_cast(half8_t, hi);
+                pl[s] = __builtin_bit_cast(half8_t, lo);
+            }
+            /* O += P . V over the tile */
+#pragma unroll
+            for (int dt = 0; dt < HD / 16; dt++) {
+                const int d = 16 * dt + c;
+                const uint2 h0 = *(const uint2 *)(vh_s + g * AMLV + 4 * d);
+                const uint2 h1 = *(const uint2 *)(vh_s + (4 + g) * AMLV + 4 * d);
+                const uint2 l0 = *(const uint2 *)(vl_s + g * AMLV + 4 * d);
+                const uint2 l1 = *(const uint2 *)(vl_s + (4 + g) * AMLV + 4 * d);
+                const half8_t bh = __builtin_bit_cast(half8_t, make_uint4(h0.x, h0.y, h1.x, h1.y));
+                const half8_t bl = __builtin_bit_cast(half8_t, make_uint4(l0.x, l0.y, l1.x, l1.y));
+#pragma unroll
+                for (int s = 0; s < QS; s++)
+                    o[s][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[s], bh, o[s][dt], 0, 0, 0);
+#pragma unroll
+                for (int s = 0; s < QS; s++)
+                    o[s][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[s], bh, o[s][dt], 0, 0, 0);
+#pragma unroll
+                for (int s = 0; s < QS; s++)
+                    o[s][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[s], bl, o[s][dt], 0, 0, 0);
+            }
+        }
+        /* the other buffer was last read before the previous barrier */
+        if (more) amma_store(kv, vv, smh + (cur ^ 1) * AMMA_BUF);
+        __syncthreads();
+    }
+    if (!active) return;
+    /* out: o[s][dt][i] is query row 16 (QS w + s) + 4g + i, dimension 16dt + c */
+#pragma unroll
+    for (int s = 0; s < QS; s++) {
+        lsum[s] += __shfl_xor(lsum[s], 16);
+        lsum[s] += __shfl_xor(lsum[s], 32);
+        if (ns > 1 && g == 0) {
+            const int r = 16 * (QS * w + s) + c, t = t0 + r / G;
+            if (t <= tl)
+                pml[((size_t)z * T + t) * H + kh * G + r % G] =
+                    make_float2(m[s] == -INFINITY ? -INFINITY : M[s], lsum[s]);
         }
 #pragma unroll
-        for (int d = 0; d < 4; d++) {
-            half4_t h, lo;
+        for (int i = 0; i < 4; i++) {
+            const float li = __shfl(lsum[s], 4 * g + i);
+            const int r = 16 * (QS * w + s) + 4 * g + i, t = t0 + r / G, h = kh * G + r % G;
+            if (t > tl) continue;
+            if (ns > 1) {
+                float *pa = pacc + (((size_t)z * T + t) * H + h) * HD + c;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float4 v = vv[it][e];
-                const f16pair p = split_f16(d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w);
-                h[e] = p.hi;
-                lo[e] = p.lo;
+                for (int dt = 0; dt < HD / 16; dt++) pa[16 * dt] = o[s][dt][i];
+            } else {
+#pragma unroll
+                for (int dt = 0; dt < HD / 16; dt++) put(t, h, 16 * dt + c, __fdiv_rn(o[s][dt][i], li));
             }
-            *(half4_t *)(vh_s + ((size_t)kg * 128 + 4 * c4 + d) * 4) = h;
-            *(half4_t *)(vl_s + ((size_t)kg * 128 + 4 * c4 + d) * 4) = lo;
         }
     }
 }
 
-__global__ __launch_bounds__(256) void k_attn_mma(const float *__restrict__ q,
-                                                  const float *__restrict__ kc,
-                                                  const float *__restrict__ vc, int H, int KV,
-                                                  int T, int pos0_arg,
-                                                  const int *__restrict__ pos_dev, int lim,
-                                                  float *__restrict__ ao,
-                                                  _Float16 *__restrict__ aoh,
-                                                  _Float16 *__restrict__ aol) {
-    constexpr int HD = 128;
-    typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-    extern __shared__ __align__(16) _Float16 smh[];   /* two tile buffers (amma_store) */
-    __shared__ uint64_t tab[32];
-    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, g = l >> 4, c = l & 15;
-    const int G = H / KV, TB = AMQ / G, kh = blockIdx.x, t0 = blockIdx.y * TB;
-    const int kvw = KV * HD;
+/* grid ceil(T * H / 8), 256 threads: row (t, h) of k_attn_mma's ns splits (the same H, KV, T,
+   position, lim and TB) merged by 32 threads, a float4 of the head each: with M the largest
+   M_z, w_z = exp2(M_z - M) and L = sum_z w_z l_z, out = (sum_z w_z O_z) / L, splits in order.
+   Written as ao or, aoh not null, as hi/lo planes; NaN for a block past the cache. */
+__global__ __launch_bounds__(256) void k_attn_merge(
+    const float *__restrict__ pacc, const float2 *__restrict__ pml, int H, int T, int TB, int ns,
+    int pos0_arg, const int *__restrict__ pos_dev, int lim, float *__restrict__ ao,
+    _Float16 *__restrict__ aoh, _Float16 *__restrict__ aol) {
+    const int row = blockIdx.x * 8 + (threadIdx.x >> 5), l32 = threadIdx.x & 31;
+    if (row >= T * H) return;
+    const int t0 = row / H / TB * TB;
     const int pos0 = pos_dev ? *pos_dev : pos0_arg;
-    if (pos0 < 0 || pos0 + t0 >= lim) return;
-    const int tl = min(T, t0 + TB) - 1;          /* the last token of the block */
-    const int n = min(pos0 + tl + 1, lim);       /* keys 0 .. n-1 */
-    if (tid < 32) tab[tid] = cpg_exp2f_tab[tid];
-    /* this lane's query (scores, softmax state): row 16w + c; rows past the block's last
-       token compute with its query and are not stored */
-    const int rq = 16 * w + c, tq = min(t0 + rq / G, tl), hq = kh * G + rq % G;
-    const int pq = pos0 + tq;                    /* its last key */
-    half8_t qh[4], ql[4];                        /* B operand: dims 32s + 8g .. + 7 */
-    {
-        const float *qr = q + ((size_t)tq * H + hq) * HD + 8 * g;
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float L = 1.0f;
+    if (pos0 < 0 || pos0 + t0 >= lim) {
+        a.x = a.y = a.z = a.w = __int_as_float(0x7fc00000);
+    } else {
+        const int n = min(pos0 + min(T, t0 + TB), lim), per = amma_split_keys(n, ns);
+        const int used = (n + per - 1) / per;
+        const size_t zs = (size_t)T * H;
+        const float2 ml = pml[(size_t)min(l32, used - 1) * zs + row];
+        const float Mz = l32 < used ? ml.x : -INFINITY;
+        const float M = half_max(Mz);
+        const float wz = l32 < used && ml.x != -INFINITY ? __builtin_amdgcn_exp2f(ml.x - M) : 0.0f;
+        L = half_sum(l32 < used ? wz * ml.y : 0.0f);
+        for (int z0 = 0; z0 < used; z0 += 8) {
+            float4 v[8];
 #pragma unroll
-        for (int s4 = 0; s4 < 4; s4++) {
-            const float4 a = *(const float4 *)(qr + 32 * s4), b = *(const float4 *)(qr + 32 * s4 + 4);
-            const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            for (int u = 0; u < 8; u++)          /* clamped, unconditional: in flight together */
+                v[u] = *(const float4 *)(pacc + ((size_t)min(z0 + u, used - 1) * zs + row) * 128 + 4 * l32);
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const f16pair p = split_f16(v[j]);
-                qh[s4][j] = p.hi;
-                ql[s4][j] = p.lo;
+            for (int u = 0; u < 8; u++) {        /* a split past the last: its weight is 0 */
+                const float wu = __shfl(wz, (threadIdx.x & 32) + min(z0 + u, 31));
+                if (z0 + u < used)
+                    a = make_float4(fmaf(wu, v[u].x, a.x), fmaf(wu, v[u].y, a.y),
+                                    fmaf(wu, v[u].z, a.z), fmaf(wu, v[u].w, a.w));
             }
         }
     }
-    const float rs = cpg_sqrt_rn((float)HD);
-    float m = -INFINITY, lsum = 0.0f;
-    f32x4_t o[HD / 16];
-#pragma unroll
-    for (int dt = 0; dt < HD / 16; dt++) o[dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    float4 kv[2][4], vv[2][4];
-    amma_load(kv, vv, kc, vc, kvw, kh, 0, n);
-    amma_store(kv, vv, smh);
-    __syncthreads();
-    for (int j0 = 0; j0 < n; j0 += AMT) {
-        /* the next tile's loads fly while this one is computed */
-        const bool more = j0 + AMT < n;
-        if (more) amma_load(kv, vv, kc, vc, kvw, kh, j0 + AMT, n);
-        const _Float16 *buf = smh + ((j0 / AMT) & 1) * AMMA_BUF;
-        const _Float16 *kh_s = buf, *kl_s = kh_s + AMT * AMLK;
-        const _Float16 *vh_s = kl_s + AMT * AMLK, *vl_s = vh_s + AMT * HD;
-        /* scores: st[kt][i] = S[query c][key j0 + 16kt + 4g + i] */
-        float st[4][4];
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++) {
-            f32x4_t a = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            const _Float16 *kr = kh_s + (16 * kt + c) * AMLK + 8 * g;
-            const _Float16 *kl = kl_s + (16 * kt + c) * AMLK + 8 * g;
-#pragma unroll
-            for (int s4 = 0; s4 < 4; s4++) {
-                const half8_t ah = *(const half8_t *)(kr + 32 * s4);
-                const half8_t al = *(const half8_t *)(kl + 32 * s4);
-                a = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, qh[s4], a, 0, 0, 0);
-                a = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, qh[s4], a, 0, 0, 0);
-                a = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, ql[s4], a, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {   /* computed unconditionally, then masked: no branch */
-                const int j = j0 + 16 * kt + 4 * g + i;
-                const float sv = __fdiv_rn(a[i], rs);
-                st[kt][i] = j <= pq && j < n ? sv : -INFINITY;
-            }
-        }
-        float mt = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) mt = fmaxf(mt, st[kt][i]);
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float mn = fmaxf(m, mt);
-        float psum = 0.0f;
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                /* a masked score is -inf, whose expf is 0 (mn is finite: key 0 is every
-                   query's and comes first) */
-                const float e = cpg_expf_tab(__fsub_rn(st[kt][i], mn), tab);
-                st[kt][i] = e;
-                psum += e;
-            }
-        psum += __shfl_xor(psum, 16);
-        psum += __shfl_xor(psum, 32);
-        const float f = m == -INFINITY ? 0.0f : cpg_expf_tab(__fsub_rn(m, mn), tab);
-        lsum = fmaf(lsum, f, psum);
-        m = mn;
-        /* the accumulators hold queries 4g + i: their factors from lanes 4g + i */
-        float fi[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) fi[i] = __shfl(f, 4 * g + i);
-#pragma unroll
-        for (int dt = 0; dt < HD / 16; dt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) o[dt][i] *= fi[i];
-        /* O += P . V over the tile, two steps of 32 keys */
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            half8_t ph, pl;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float pv = j < 4 ? st[2 * u][j] : st[2 * u + 1][j - 4];
-                const f16pair p = split_f16(pv);
-                ph[j] = p.hi;
-                pl[j] = p.lo;
-            }
-            const int kg0 = 8 * u + g, kg1 = 8 * u + 4 + g;
-#pragma unroll
-            for (int dt = 0; dt < HD / 16; dt++) {
-                const int d = 16 * dt + c;
-                const half4_t h0 = *(const half4_t *)(vh_s + ((size_t)kg0 * HD + d) * 4);
-                const half4_t h1 = *(const half4_t *)(vh_s + ((size_t)kg1 * HD + d) * 4);
-                const half4_t l0 = *(const half4_t *)(vl_s + ((size_t)kg0 * HD + d) * 4);
-                const half4_t l1 = *(const half4_t *)(vl_s + ((size_t)kg1 * HD + d) * 4);
-                const half8_t bh = {h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
-                const half8_t bl = {l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3]};
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, bh, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, bh, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, bl, o[dt], 0, 0, 0);
-            }
-        }
-        /* the other buffer was last read before the previous barrier */
-        if (more) amma_store(kv, vv, smh + ((j0 / AMT + 1) & 1) * AMMA_BUF);
-        __syncthreads();
-    }
-    /* out: o[dt][i] is query row 16w + 4g + i, dimension 16dt + c */
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float li = __shfl(lsum, 4 * g + i);
-        const int r = 16 * w + 4 * g + i, t = t0 + r / G, h = kh * G + r % G;
-        if (t > tl) continue;
-        const size_t e0 = ((size_t)t * H + h) * HD + c;
-#pragma unroll
-        for (int dt = 0; dt < HD / 16; dt++) {
-            const float v = __fdiv_rn(o[dt][i], li);
-            if (aoh) {
-                const f16pair p = split_f16(v);
-                aoh[e0 + 16 * dt] = p.hi;
-                aol[e0 + 16 * dt] = p.lo;
-            } else {
-                ao[e0 + 16 * dt] = v;
-            }
-        }
+    a = make_float4(__fdiv_rn(a.x, L), __fdiv_rn(a.y, L), __fdiv_rn(a.z, L), __fdiv_rn(a.w, L));
+    const size_t e = (size_t)row * 128 + 4 * l32;
+    if (aoh) {
+        const f16pair2 p = split_f16x2(a.x, a.y), r = split_f16x2(a.z, a.w);
+        *(uint2 *)(aoh + e) = make_uint2(p.hi, r.hi);
+        *(uint2 *)(aol + e) = make_uint2(p.lo, r.lo);
+    } else {
+        *(float4 *)(ao + e) = a;
     }
 }
 
@@ -1052,24 +1189,6 @@ __global__ __launch_bounds__(ADT) void k_attn_decode(const float *__restrict__ q
     }
     attn_softmax_av<ADT, AV_DEPTH>(vc, kvw, kh, HD, n, pos, vq, v0, v1, sc, mx, red, part, etab,
                          ao + (size_t)h * HD);
-}
-
-/* The maximum and the sum over each half of the wavefront (lanes 0-31, 32-63), the same
-   bits in every lane of the half: DPP steps within rows of 16 lanes, then one exchange
-   between the two rows of the half. */
-__device__ static inline float half_max(float v) {
-    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_QUAD_1032, 0xf, 0xf, false)));
-    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_QUAD_2301, 0xf, 0xf, false)));
-    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_ROW_HALF_MIRROR, 0xf, 0xf, false)));
-    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_ROW_MIRROR, 0xf, 0xf, false)));
-    return fmaxf(v, __shfl_xor(v, 16));
-}
-__device__ static inline float half_sum(float v) {
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_QUAD_1032, 0xf, 0xf, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_QUAD_2301, 0xf, 0xf, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_ROW_HALF_MIRROR, 0xf, 0xf, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP_ROW_MIRROR, 0xf, 0xf, false));
-    return v + __shfl_xor(v, 16);
 }
 
 /* The reference's per-head RMSNorm and RoPE (qwen3_moe.c:137-143, kernels.c:408-413, 430-447)
@@ -1407,8 +1526,10 @@ extern "C" int cpg_gemv_norm(int enc, const void *w, int n_in, int n_out, const 
 struct cpg_attn_ws {
     int D, H, KV, HD, max_T;
     float *qkv, *q, *ao;
-    float *pacc;            /* k_attn_split: (H, ASPLIT_MAX_POS / AP, HD), or null */
-    float2 *pml;            /* k_attn_split: (H, ASPLIT_MAX_POS / AP) */
+    float *pacc;            /* k_attn_split: (H, ASPLIT_MAX_POS / AP, HD); k_attn_mma: mma_rows
+                               of 128; or null */
+    float2 *pml;            /* the same rows' maxima and sums */
+    size_t mma_rows;
     int *ctr;               /* k_attn_split: KV arrival counters, zero between launches */
     int *stat;              /* 1 once a kernel saw a position outside the cache */
     void *dense;            /* cpg_dense_mfma for T >= DENSE_MIN_T, or null */
@@ -1435,6 +1556,11 @@ static bool attn_split_shape(int H, int KV, int HD) {
     return HD == AHD && KV > 0 && H == AG * KV;
 }
 
+/* the shapes k_attn_mma is written for */
+static bool attn_mma_shape(int H, int KV, int HD) {
+    return HD == 128 && KV > 0 && H / KV <= 16 && 16 % (H / KV) == 0;
+}
+
 extern "C" cpg_attn_ws *cpg_attn_ws_create(int D, int H, int KV, int HD, int max_T) {
     if (!g_cpg.ready) { cpg_set_error("cpg_init has not been called"); return nullptr; }
     if (D <= 0 || H <= 0 || KV <= 0 || H % KV || HD <= 0 || HD > 128 || HD % 4 || max_T <= 0) {
@@ -1446,6 +1572,13 @@ extern "C" cpg_attn_ws *cpg_attn_ws_create(int D, int H, int KV, int HD, int max
     ws->D = D; ws->H = H; ws->KV = KV; ws->HD = HD; ws->max_T = max_T;
     const size_t T = (size_t)max_T, smax = ASPLIT_MAX_POS / AP;
     const bool split = attn_split_shape(H, KV, HD);
+    /* partial rows: (head, split) of one token in k_attn_split; (split, token, head) in
+       k_attn_mma, whose AMMA_WGS workgroups leave at most 128 rows each */
+    ws->mma_rows = attn_mma_shape(H, KV, HD) && max_T >= AMMA_MIN_T
+                       ? (size_t)AMMA_WGS * 128 : 0;
+    if (ws->mma_rows > AMMA_MAX_NS * T * H) ws->mma_rows = AMMA_MAX_NS * T * H;
+    const size_t srows = split ? H * smax : 0;
+    const size_t rows = srows > ws->mma_rows ? srows : ws->mma_rows;
     const int nqkv = (H + 2 * KV) * HD;
     size_t dense = 0;
     if (cpg_dense_shape_ok(D, nqkv) && cpg_dense_shape_ok(H * HD, D))
@@ -1456,7 +1589,7 @@ extern "C" cpg_attn_ws *cpg_attn_ws_create(int D, int H, int KV, int HD, int max
             dense = b > dense ? b : dense;
         }
     const size_t sz[8] = {T * nqkv * 4, T * H * HD * 4, T * H * HD * 4,
-                          split ? H * smax * HD * 4 : 0, split ? H * smax * 8 : 0, dense,
+                          rows * HD * 4, rows * 8, dense,
                           split ? (size_t)KV * 4 : 0, 4};
     size_t total = 0;
     for (int i = 0; i < 8; i++) total += cpg_round256(sz[i]);
@@ -1489,6 +1622,45 @@ extern "C" void cpg_attn_ws_destroy(cpg_attn_ws *ws) {
     if (!ws) return;
     cpg_free(ws->block);
     free(ws);
+}
+
+/* k_attn_mma over the T tokens whose q heads are in ws->q and whose keys are in the cache, and
+   k_attn_merge where the keys are split */
+static int launch_attn_mma(const cpg_attn_layer *A, cpg_attn_ws *ws, int T, int pos0,
+                           const int *pos_dev, int lim, float *kc, float *vc, _Float16 *aoh,
+                           _Float16 *aol) {
+    const int H = A->H, KV = A->KV, G = H / KV;
+    const int qs = T * G > AMMA_QS1_ROWS ? 2 : 1, TB = 64 * qs / G;
+    const int blocks = KV * ((T + TB - 1) / TB);
+    /* the splits are set by the cache's length and not by the position, so that a position
+       given by the host and one read on the device give the same bits */
+    int ns = AMMA_WGS / blocks;
+    ns = ns < lim / AMMA_MIN_KEYS ? ns : lim / AMMA_MIN_KEYS;
+    const size_t cap = ws->mma_rows / ((size_t)T * H);       /* k_attn_merge's partial rows */
+    ns = ns < AMMA_MAX_NS ? ns : AMMA_MAX_NS;
+    ns = (size_t)ns < cap ? ns : (int)cap;
+    ns = ns > 1 ? ns : 1;
+    /* a known position: no more splits than tiles, and with one tile the split that holds it
+       writes the result (the bits that merging one split gives) */
+    const int tiles = pos_dev ? ns : (pos0 + T + AMT - 1) / AMT;
+    if (tiles == 1) ns = 1;
+    const size_t sm = amma_lds_bytes();
+    const void *kf = qs == 2 ? (const void *)k_attn_mma<2> : (const void *)k_attn_mma<1>;
+    CPG_HIP(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
+    const dim3 grid(KV, (T + TB - 1) / TB, ns < tiles ? ns : tiles);
+    if (qs == 2)
+        hipLaunchKernelGGL(k_attn_mma<2>, grid, dim3(256), sm, g_cpg.stream, ws->q, kc, vc, H, KV,
+                           T, pos0, pos_dev, lim, ns, ws->pacc, ws->pml, ws->ao, aoh, aol);
+    else
+        hipLaunchKernelGGL(k_attn_mma<1>, grid, dim3(256), sm, g_cpg.stream, ws->q, kc, vc, H, KV,
+                           T, pos0, pos_dev, lim, ns, ws->pacc, ws->pml, ws->ao, aoh, aol);
+    CPG_LAUNCH_CHECK("k_attn_mma");
+    if (ns > 1) {
+        hipLaunchKernelGGL(k_attn_merge, dim3((T * H + 7) / 8), dim3(256), 0, g_cpg.stream,
+                           ws->pacc, ws->pml, H, T, TB, ns, pos0, pos_dev, lim, ws->ao, aoh, aol);
+        CPG_LAUNCH_CHECK("k_attn_merge");
+    }
+    return 0;
 }
 
 /* pos0 >= 0: the position as a value; pos_dev: read on the device (pos0 is then the largest
@@ -1537,7 +1709,7 @@ static int attn_forward(const cpg_attn_layer *A, const float *x, int T, int pos0
     const int nmax = pos_dev ? lim : pos0 + T;
     const size_t smem = sizeof(float) * (size_t)nmax;
     bool planes = false;                         /* the output projection's planes written */
-    if (T == 1 && g_attn_mode == CPG_ATTN_SPLIT && ws->pacc && lim <= ASPLIT_MAX_POS) {
+    if (T == 1 && g_attn_mode == CPG_ATTN_SPLIT && ws->ctr && lim <= ASPLIT_MAX_POS) {
         const int smax = (lim + AP - 1) / AP;
         /* while the few attention workgroups run, the output projection's rows are read into
            the L2 of the XCD whose workgroups will read them */
@@ -1562,16 +1734,9 @@ static int attn_forward(const cpg_attn_layer *A, const float *x, int T, int pos0
         CPG_LAUNCH_CHECK("k_qk_norm_rope");
         const int G = H / KV;
         _Float16 *aoh = dense ? ph : nullptr, *aol = dense ? ph + (size_t)T * H * HD : nullptr;
-        if (HD == 128 && G <= 16 && 16 % G == 0 && T >= AMMA_MIN_T) {
-            /* on MFMA: 64 query rows per workgroup share every key tile */
-            const size_t sm = amma_lds_bytes();
-            if (sm > 64 * 1024)
-                CPG_HIP(hipFuncSetAttribute((const void *)k_attn_mma,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
-            const int TB = AMQ / G;
-            hipLaunchKernelGGL(k_attn_mma, dim3(KV, (T + TB - 1) / TB), dim3(256), sm, s, ws->q,
-                               kc, vc, H, KV, T, pos0, pos_dev, lim, ws->ao, aoh, aol);
-            CPG_LAUNCH_CHECK("k_attn_mma");
+        if (attn_mma_shape(H, KV, HD) && T >= AMMA_MIN_T) {
+            rc = launch_attn_mma(A, ws, T, pos0, pos_dev, lim, kc, vc, aoh, aol);
+            if (rc) return rc;
             planes = dense;
         } else if (G <= 32 && 32 % G == 0 && HD <= 128) {
             /* the kv head's rows read once per block of tokens (k_attn_blk): 16 query rows

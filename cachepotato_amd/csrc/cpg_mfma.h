@@ -31,6 +31,24 @@ __device__ static inline f16pair split_f16(float x) {
     return {h, (_Float16)(x - (float)h)};
 }
 
+/* split_f16 of two floats, the f16 pairs in one word each (x in the low half): four
+   instructions, v_cvt_pk_f16_f32 for hi, x - hi exact in v_fma_mix_f32, v_cvt_pk_f16_f32 */
+struct f16pair2 {
+    uint32_t hi, lo;
+};
+__device__ static inline f16pair2 split_f16x2(float x, float y) {
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    asm("" : "+v"(x), "+v"(y));
+    const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{x, y}), half2_t));
+    f32x2_t r;
+    float rx, ry;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(rx) : "v"(h), "v"(x));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(ry) : "v"(h), "v"(y));
+    r.x = rx;
+    r.y = ry;
+    return {h, __builtin_bit_cast(uint32_t, __builtin_convertvector(r, half2_t))};
+}
+
 __device__ static inline half8_t pairs_to_half8(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3,
                                                _Float16 bias) {
     /* each p holds two 16-bit values 0x6400 | u, i.e. the f16 numbers 1024 + u; subtracting

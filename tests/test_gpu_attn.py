@@ -148,6 +148,34 @@ def test_attn_prefill_gqa_groups_vs_oracle(cpg, oracle, H, KV):
         dev.close()
 
 
+@pytest.mark.parametrize("T,pos0,cap", [(2, 31, 64), (2, 300, 400), (21, 700, 800), (40, 992, 1100),
+                                        (128, 0, 256), (129, 415, 600), (12, 20, 2000)])
+def test_attn_prefill_key_splits_vs_oracle(cpg, oracle, T, pos0, cap):
+    """The MFMA attention core with its keys split over workgroups: one key past a tile of 32 and
+    a tile's end, ragged last splits, both row counts per wavefront (128 tokens of 8 heads is
+    the last call with one set), a cache longer than the positions (splits without keys); over
+    a random history, against the oracle. The position read on the device gives the same bits."""
+    from tests.attn_helpers import attn_layer, inputs, DeviceAttn
+    a = attn_layer(enc=8, D=2048, H=32, KV=4, HD=128)
+    kvw = a["KV"] * a["HD"]
+    dev = DeviceAttn(a, cap=cap, max_T=T)
+    X = inputs(a["D"], 103, T)
+    rng = np.random.default_rng(T + pos0)
+    kc_o, vc_o = np.zeros((cap, kvw), np.float32), np.zeros((cap, kvw), np.float32)
+    kc_o[:pos0], vc_o[:pos0] = rng.normal(size=(2, pos0, kvw))
+    dev.set_cache(kc_o, vc_o)
+    try:
+        got = dev.forward(X, pos0)
+        again = dev.forward_at(X, pos0)
+        want = oracle.attn(a, X, pos0, kc_o, vc_o, threads=8)
+        e = max(rel_err(got[t], want[t]) for t in range(T))
+        say(f"attn splits T={T} pos0={pos0}: worst token {e:.2e}")
+        assert e <= PREFILL_TOL
+        assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+    finally:
+        dev.close()
+
+
 def test_attn_device_position_equals_host_position(cpg):
     """cpg_attn_forward_at (position read on the device, as in a replayed graph) computes the
     same bits as cpg_attn_forward at the same positions, cache included; a position whose rows
