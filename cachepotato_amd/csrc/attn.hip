@@ -518,14 +518,16 @@ __device__ static inline float half_sum(float v) {
    tokens, over split z of the block's keys, of which there are at most ns (ns == 1: one split
    with all of them; splits past the block's last leave at once). All rows share each tile of
    AMT key positions of kv head kh staged in LDS as hi/lo f16 halves (x = hi + lo, hi = f16(x),
-   lo = f16(x - hi): 22 significant bits). Per tile:
+   lo = f16(x - hi): 22 significant bits), the query rows scaled by 8 log2(e) / sqrt(HD) in
+   double before the split (a scale of the scores rounded to fp32 would bend every softmax by the
+   same 2^-24; 8 keeps the halves of a normed query's size). Per tile:
      S^T = K . Q^T on v_mfma_f32_16x16x32_f16 (A = key rows, B = the wavefront's query rows,
        held in registers for the whole call), each product as hi.hi + lo.hi + hi.lo (the lo.lo
        term, below 2^-22 of the sum, is not formed); lane l then holds the scores of query
        l%16 against keys 16kt + 4(l/16) + i (kt < 2, i < 4), masked where the tile reaches past
        one of the wavefront's positions (key j > the query's position, or past the cache: -inf);
-     online softmax per query in powers of two: with c = log2(e) / sqrt(HD) and M = c * (the
-       largest score so far) the probabilities are exp2(c s - M), one fused multiply-add and
+     online softmax per query in powers of two: with M = (the largest score so far) / 8 the
+       probabilities are exp2(s / 8 - M), one fused multiply-add and
        the hardware exponential (1 ulp); the 4 lanes of a query share the maximum by shuffles,
        each adds its own part of the sum l, and the accumulators are rescaled by
        exp2(M_old - M_new) in the tiles where some maximum of the wavefront grew;
@@ -659,6 +661,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
        block's last token compute with its query and are not stored; a wavefront with no row
        of the block only stages */
     const bool active = 16 * QS * w < (tl - t0 + 1) * G;
+    const double c8 = 8.0 * 1.4426950408889634 * 0.08838834764831845;   /* 8 log2(e) / sqrt(128) */
+    auto scaled = [&](float4 v) {
+        return make_float4((float)(c8 * v.x), (float)(c8 * v.y), (float)(c8 * v.z), (float)(c8 * v.w));
+    };
     int pq[QS];                                  /* their last keys */
     half8_t qh[QS][4], ql[QS][4];                /* B operand: dims 32s4 + 8g .. + 7 */
 #pragma unroll
@@ -668,11 +674,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         const float *qr = q + ((size_t)tq * H + kh * G + r % G) * HD + 8 * g;
 #pragma unroll
         for (int s4 = 0; s4 < 4; s4++)
-            split_hilo8(*(const float4 *)(qr + 32 * s4), *(const float4 *)(qr + 32 * s4 + 4),
-                        qh[s][s4], ql[s][s4]);
+            split_hilo8(scaled(*(const float4 *)(qr + 32 * s4)),
+                        scaled(*(const float4 *)(qr + 32 * s4 + 4)), qh[s][s4], ql[s][s4]);
     }
     const int pfirst = pos0 + min(t0 + 16 * QS * w / G, tl);   /* the wavefront's first position */
-    const float cs = 1.44269504088896341f * 0.08838834764831845f;   /* log2(e) / sqrt(128) */
+    const float cs = 0.125f;                     /* the scores are 8 times the exponents of 2 */
     float m[QS], M[QS], lsum[QS];
     f32x4_t o[QS][HD / 16];
 #pragma unroll
