@@ -19,7 +19,7 @@
  *                    weighted sum over positions; the sums run in another order than the
  *                    reference's serial loops (fp32, ~1e-7 to 1e-6 relative).
  *   k_gemv           attn = Wo . ao.
- * From DENSE_MIN_T tokens on, both projections run as MFMA GEMMs instead (k_mfma_dense and
+ * From DENSE_MIN_T tokens on, both projections run as MFMA GEMMs instead (k_dense and
  * k_sum_parts of prefill.hip): k_rmsnorm_rows_hilo writes ln1's output as the hi + lo f16
  * planes of the q|k|v product, k_qk_norm_rope adds that product's k parts as it reads them,
  * and the attention core writes the planes of the Wo product; exact f16 weight integers, fp32
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float *__restrict__ 
 }
 
 /* the same rows as k_rmsnorm_rows, written as the hi/lo f16 planes of the dense MFMA
-   product (hi = f16(v), lo = f16(v - hi), the arithmetic of k_split_hilo) instead of fp32 */
+   product (split_f16_up: hi = f16(v), lo = f16((v - hi) 2^11)) instead of fp32 */
 __global__ __launch_bounds__(256) void k_rmsnorm_rows_hilo(const float *__restrict__ x,
                                                            const float *__restrict__ g, int D,
                                                            float eps, _Float16 *__restrict__ hi,
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows_hilo(const float *__restri
         half4_t h, l;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const f16pair p = split_f16(o[j]);
+            const f16pair p = split_f16_up(o[j]);
             h[j] = p.hi;
             l[j] = p.lo;
         }
@@ -254,7 +254,13 @@ __global__ __launch_bounds__(64) void k_qk_norm_rope(const float *__restrict__ q
     /* the projection's ks k-parts (pstride floats apart) added in part order, as k_sum_parts */
     auto val = [&](int i) {
         float a = src[i];
-        for (int z = 1; z < ks; z++) a = __fadd_rn(a, src[(size_t)z * pstride + i]);
+        for (int z0 = 1; z0 < ks; z0 += 8) {     /* the loads of eight parts in flight together */
+            float p[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) p[u] = src[(size_t)min(z0 + u, ks - 1) * pstride + i];
+#pragma unroll
+            for (int u = 0; u < 8; u++) a = z0 + u < ks ? __fadd_rn(a, p[u]) : a;
+        }
         return a;
     };
     if (hh >= H + KV) {                          /* value head: to the cache unchanged */
@@ -641,7 +647,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     auto put = [&](int t, int h, int d, float v) {
         const size_t e = ((size_t)t * H + h) * HD + d;
         if (aoh) {
-            const f16pair p = split_f16(v);
+            const f16pair p = split_f16_up(v);
             aoh[e] = p.hi;
             aol[e] = p.lo;
         } else {
@@ -879,7 +885,7 @@ __global__ __launch_bounds__(256) void k_attn_merge(
     a = make_float4(__fdiv_rn(a.x, L), __fdiv_rn(a.y, L), __fdiv_rn(a.z, L), __fdiv_rn(a.w, L));
     const size_t e = (size_t)row * 128 + 4 * l32;
     if (aoh) {
-        const f16pair2 p = split_f16x2(a.x, a.y), r = split_f16x2(a.z, a.w);
+        const f16pair2 p = split_f16x2_up(a.x, a.y), r = split_f16x2_up(a.z, a.w);
         *(uint2 *)(aoh + e) = make_uint2(p.hi, r.hi);
         *(uint2 *)(aol + e) = make_uint2(p.lo, r.lo);
     } else {
@@ -1043,7 +1049,7 @@ __global__ __launch_bounds__(256) void k_attn_blk(const float *__restrict__ q,
                     half4_t hv, lv;
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
-                        const f16pair p = split_f16(r4[j]);
+                        const f16pair p = split_f16_up(r4[j]);
                         hv[j] = p.hi;
                         lv[j] = p.lo;
                     }
@@ -1542,9 +1548,11 @@ struct cpg_attn_ws {
     void *block;
 };
 
-/* from this many tokens on the q|k|v and output projections run on MFMA (cpg_dense_mfma)
-   instead of k_gemv, whose passes of MT tokens each re-stream the matrix */
-#define DENSE_MIN_T 32
+/* from this many tokens on the q|k|v and output projections run on MFMA (k_dense) instead of
+   k_gemv, whose passes of four tokens each convert the whole matrix again. With the norm and the
+   sums of the parts, which k_gemv has inside, over 700 positions, Q4_0, us: 2 tokens 17.0 in four
+   launches against 16.2 in two, 3 tokens 17.3 against 21.2, 21 tokens (Q8_0) 21.1 against 96.2 */
+#define DENSE_MIN_T 3
 
 static int g_attn_mode = CPG_ATTN_SPLIT;     /* the per-head kernel where split does not apply */
 

@@ -94,7 +94,7 @@ bool cpg_prefill_shape_ok(int D, int F);
    xn; otherwise they are formed here from grp_cnt and xn. */
 size_t cpg_prefill_scratch_bytes(int T, int D, int K, int F);
 /* prefill.hip: the dense MFMA product from hi/lo planes already at the start of scratch
-   (T rows of n_in halves each, hi then lo); with sum == 0 and more than one k part the parts
+   (T rows of n_in halves each, hi then lo as split_f16_up forms them); with sum == 0 and more than one k part the parts
    are left in *parts (ks of them, T * n_out floats each, to be added in order) */
 int cpg_dense_from_planes(int enc, const void *w, int n_in, int n_out, int T, void *scratch,
                           float *out, int sum, const float **parts, int *ks);

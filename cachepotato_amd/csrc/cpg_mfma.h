@@ -49,6 +49,21 @@ __device__ static inline f16pair2 split_f16x2(float x, float y) {
     return {h, __builtin_bit_cast(uint32_t, __builtin_convertvector(r, half2_t))};
 }
 
+/* The same halves with lo kept 2^11 times larger, for products whose weights are scaled by
+   2^-11 where they meet lo (exact in f16): lo then has its 11 bits as long as hi is normal,
+   where f16(x - hi) loses them to f16's subnormals below |x| = 2^-2 (an attention output over
+   thousands of keys is about 2^-5). |lo| <= |x| / 2: no new overflow. */
+__device__ static inline f16pair split_f16_up(float x) {
+    asm("" : "+v"(x));
+    const _Float16 h = (_Float16)x;
+    return {h, (_Float16)((x - (float)h) * 0x1p11f)};
+}
+__device__ static inline f16pair2 split_f16x2_up(float x, float y) {
+    const f16pair a = split_f16_up(x), b = split_f16_up(y);
+    return {__builtin_bit_cast(uint32_t, half2_t{a.hi, b.hi}),
+            __builtin_bit_cast(uint32_t, half2_t{a.lo, b.lo})};
+}
+
 __device__ static inline half8_t pairs_to_half8(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3,
                                                _Float16 bias) {
     /* each p holds two 16-bit values 0x6400 | u, i.e. the f16 numbers 1024 + u; subtracting

@@ -34,24 +34,11 @@
  * twice the workgroups spread it over the CUs. The activations are split into
  * hi/lo f16 planes once per call (k_split_hilo for xn; the gate/up epilogue writes h split).
  * Both operands reach the MFMAs through a ring of stages in LDS filled by direct
- * global-to-LDS loads (k_pf_gemm); the dense projections keep a register-staged k loop
- * (gemm_k_loop).
+ * global-to-LDS loads (k_pf_gemm; k_dense for the dense projections).
  */
 #include "cpg_internal.h"
 #include "cpg_gemv.h"
 #include "cpg_mfma.h"
-
-/* The dense GEMM's tiling (gemm_k_loop): NW wavefronts of RW weight rows each, stages of KB
-   blocks of 32 in LDS with a row stride of KS + 8 halves (16 B of padding against bank
-   conflicts), and PIECES 16-byte pieces of a stage's activations per thread. */
-template <int NW_, int KB_, int RW_ = 16> struct PfGeo {
-    static constexpr int NW = NW_, NT = NW_ * 64, RW = RW_, ROWS = NW_ * RW_, KB = KB_,
-                         KS = KB_ * 32, LDA = KB_ * 32 + 8,
-                         PIECES = PF_CHUNK * (KB_ * 32 / 8) / (NW_ * 64);
-    static_assert(PIECES >= 1 && PF_CHUNK * (KB_ * 32 / 8) % (NW_ * 64) == 0, "stage pieces");
-    static_assert(RW_ % 16 == 0, "whole B tiles");
-};
-typedef PfGeo<4, 1> PfDown;
 
 /* ---------------------------------------------------------------- chunk list */
 
@@ -70,7 +57,8 @@ __global__ __launch_bounds__(64) void k_chunks(const int *__restrict__ grp_cnt, 
 }
 
 /* grid rows, 256 threads: hi[r] = f16(x[r]), lo[r] = f16(x[r] - hi[r]) for rows of n floats
-   (n % 8 == 0) */
+   (n % 8 == 0); UP: lo is kept 2^11 times larger, as the dense product takes it (split_f16_up) */
+template <bool UP>
 __global__ __launch_bounds__(256) void k_split_hilo(const float *__restrict__ x, int n,
                                                     _Float16 *__restrict__ hi,
                                                     _Float16 *__restrict__ lo) {
@@ -82,139 +70,12 @@ __global__ __launch_bounds__(256) void k_split_hilo(const float *__restrict__ x,
         half8_t h, l;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const f16pair p = split_f16(v[j]);
+            const f16pair p = UP ? split_f16_up(v[j]) : split_f16(v[j]);
             h[j] = p.hi;
             l[j] = p.lo;
         }
         *(half8_t *)(hi + r * n + 8 * c) = h;
         *(half8_t *)(lo + r * n + 8 * c) = l;
-    }
-}
-
-/* One stage of activations: G::KS halves of each of the chunk's 64 rows, hi and lo, as
-   16-byte pieces; thread tid moves pieces tid, tid + G::NT, ... (G::PIECES each of hi and
-   lo). */
-template <class G> struct AStage {
-    half8_t h[G::PIECES], l[G::PIECES];
-};
-
-template <class G, typename Row>
-__device__ static inline void stage_load(AStage<G> &a, int m, int k0, Row row_of,
-                                         const _Float16 *__restrict__ hi,
-                                         const _Float16 *__restrict__ lo, size_t ld) {
-    /* unconditional loads (a load under a branch makes the compiler wait for every load in
-       flight where the branches join): rows past m repeat row m-1, whose MFMA output rows
-       are never stored (an MFMA output row depends on its own A row only) */
-#pragma unroll
-    for (int p = 0; p < G::PIECES; p++) {
-        const int idx = threadIdx.x + G::NT * p, i = idx / (G::KS / 8), c = idx % (G::KS / 8);
-        const size_t off = (size_t)row_of(min(i, m - 1)) * ld + k0 + 8 * c;
-        a.h[p] = *(const half8_t *)(hi + off);
-        a.l[p] = *(const half8_t *)(lo + off);
-    }
-}
-
-template <class G>
-__device__ static inline void stage_store(const AStage<G> &a, _Float16 *ah, _Float16 *al) {
-#pragma unroll
-    for (int p = 0; p < G::PIECES; p++) {
-        const int idx = threadIdx.x + G::NT * p, i = idx / (G::KS / 8), c = idx % (G::KS / 8);
-        *(half8_t *)(ah + i * G::LDA + 8 * c) = a.h[p];
-        *(half8_t *)(al + i * G::LDA + 8 * c) = a.l[p];
-    }
-}
-
-/* One block (index kb of the LDS stage) for NMT token tiles and NB weight operands b[n]
-   with scales d[n]: acc[n][mt] += d[n] * (A_hi + A_lo)[mt] . b[n]. The A fragments are read
-   once and feed every B operand; for each n the NMT hi products are independent chains that
-   issue back to back, then the lo products accumulate onto them. */
-template <class G, int NMT, int NB>
-__device__ static inline void mma_block(const _Float16 *ah, const _Float16 *al, int kb,
-                                        const half8_t *b, const float *d,
-                                        f32x4_t (*acc)[PF_CHUNK / 16]) {
-    const int l = threadIdx.x & 63;
-    half8_t a_hi[NMT], a_lo[NMT];
-#pragma unroll
-    for (int mt = 0; mt < NMT; mt++) {
-        const int off = (mt * 16 + (l & 15)) * G::LDA + kb * 32 + 8 * (l >> 4);
-        a_hi[mt] = *(const half8_t *)(ah + off);
-        a_lo[mt] = *(const half8_t *)(al + off);
-    }
-#pragma unroll
-    for (int n = 0; n < NB; n++) {
-        f32x4_t t[NMT];
-#pragma unroll
-        for (int mt = 0; mt < NMT; mt++) {
-            const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-            t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_hi[mt], b[n], z, 0, 0, 0);
-        }
-#pragma unroll
-        for (int mt = 0; mt < NMT; mt++)
-            t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_lo[mt], b[n], t[mt], 0, 0, 0);
-#pragma unroll
-        for (int mt = 0; mt < NMT; mt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[n][mt][i] = fmaf(d[n], t[mt][i], acc[n][mt][i]);
-    }
-}
-
-/* The k loop shared by the GEMMs: NB B operands, operand n being 16 rows of matrix M[n]
-   (this lane's row rows[n], nb blocks per row), S stages of G::KB blocks from block b0; the
-   A operand rows come from planes hi/lo (row stride ld) through row_of(i). Software
-   pipeline: LDS double-buffered, next stage's activations loaded during the current stage's
-   MFMAs, weights two stages ahead in three register sets named per stage of a 3-way unrolled
-   loop (no register copies of loads in flight, which would make the compiler wait for
-   them). */
-template <int ENC, class G, int NMT, int NB, typename Row>
-__device__ static inline void gemm_k_loop(const uint8_t *const *M, size_t payload_plane,
-                                          const int (&rows)[NB], int nb, int g, int S, int m,
-                                          Row row_of, const _Float16 *__restrict__ hi,
-                                          const _Float16 *__restrict__ lo, size_t ld,
-                                          _Float16 (*ah)[PF_CHUNK * G::LDA],
-                                          _Float16 (*al)[PF_CHUNK * G::LDA],
-                                          f32x4_t (*acc)[PF_CHUNK / 16], int b0 = 0) {
-    WRaw w0[NB][G::KB], w1[NB][G::KB], w2[NB][G::KB];
-    auto wload = [&](WRaw (&wr)[NB][G::KB], int st) {
-        st = min(st, S - 1);                     /* past the end: a valid block, unused */
-#pragma unroll
-        for (int n = 0; n < NB; n++)
-#pragma unroll
-            for (int kb = 0; kb < G::KB; kb++)
-                wr[n][kb] = weight_raw<ENC>(M[n], payload_plane, rows[n], b0 + st * G::KB + kb,
-                                            nb, g);
-    };
-    wload(w0, 0);
-    wload(w1, 1);
-    /* activations two stages ahead as well, in three register sets named per stage of the
-       same unrolled loop: stage s loads stage s+2 and stores stage s+1 (loaded one stage
-       earlier) into the other LDS buffer */
-    AStage<G> a0, a1, a2;
-    stage_load(a0, m, 0, row_of, hi, lo, ld);
-    stage_load(a1, m, min(1, S - 1) * G::KS, row_of, hi, lo, ld);
-    stage_store(a0, ah[0], al[0]);
-    __syncthreads();
-    auto stage = [&](int s, WRaw (&wc)[NB][G::KB], WRaw (&wn)[NB][G::KB], AStage<G> &anext,
-                     AStage<G> &astore) {
-        stage_load(anext, m, min(s + 2, S - 1) * G::KS, row_of, hi, lo, ld);
-        wload(wn, s + 2);
-#pragma unroll
-        for (int kb = 0; kb < G::KB; kb++) {
-            half8_t b[NB];
-            float d[NB];
-#pragma unroll
-            for (int n = 0; n < NB; n++) {
-                b[n] = weight_half8<ENC>(wc[n][kb], g);
-                d[n] = scale_f32(wc[n][kb].d);
-            }
-            mma_block<G, NMT, NB>(ah[s & 1], al[s & 1], kb, b, d, acc);
-        }
-        if (s + 1 < S) stage_store(astore, ah[(s + 1) & 1], al[(s + 1) & 1]);
-        __syncthreads();
-    };
-    for (int s = 0; s < S; s += 3) {
-        stage(s, w0, w2, a2, a1);
-        if (s + 1 < S) stage(s + 1, w1, w0, a0, a2);
-        if (s + 2 < S) stage(s + 2, w2, w1, a1, a0);
     }
 }
 
@@ -277,7 +138,7 @@ struct PfRing {
        Chunks of one token tile (batches of up to 16 tokens) compute little per stage and
        wait for its loads: their ring is deeper (pf_small_ring). */
     static constexpr int P = P_;
-    static_assert((RW == 64 || RW == 128) && P >= 2 && WB % 16 == 0 && SB % 16 == 0 && SB <= 1024 && PP <= 16 &&
+    static_assert(RW % 64 == 0 && P >= 2 && WB % 16 == 0 && SB % 16 == 0 && SB <= 1024 && PP <= 16 &&
                       TT >= 1 && TT <= PF_CHUNK / 16 && R_Q_FITS(2 * KB + WI + 1, P),
                   "ring geometry");
     /* the position of logical piece c of A row r: rows 16 * 4 / PP apart share banks, so the
@@ -337,8 +198,10 @@ __device__ static inline half8_t weight_q(uint2 pw, int g) {
    blocks in order. Measured against the B operand w = q * d as an exact f16 pair hi + lo
    (three MFMAs accumulating across blocks, 22 instructions per lane to form hi and lo from
    a block's 8 weights, against 12 for q here plus 4 fused multiply-adds per token tile):
-   gate/up 112.7 -> 103.5 us, down 60.2 -> 57.6 us at 512 tokens. */
-template <class R, int NMT>
+   gate/up 112.7 -> 103.5 us, down 60.2 -> 57.6 us at 512 tokens.
+   UP: the lo plane is 2^11 times larger (split_f16_up), and is multiplied by q * 2^-11, exact
+   in f16: four more instructions per B tile and block. */
+template <class R, int NMT, bool UP = false>
 __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *const (&asrc_h)[R::KB],
                                const _Float16 *const (&asrc_l)[R::KB],
                                const uint8_t *wsrc, size_t wstep, const uint8_t *ssrc,
@@ -408,6 +271,8 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *const (&asr
                 r.w = *(const uint2 *)(wl + boff[n] + kb * 64 * R::PB);
                 r.d = *(const uint16_t *)((const uint8_t *)sl + soff[n] + kb * 128);
                 const half8_t q = weight_q<ENC>(r.w, g);
+                half8_t ql = q;
+                if (UP) ql *= (_Float16)0x1p-11f;
                 const float d = scale_f32(r.d);
                 f32x4_t t[NMT];
 #pragma unroll
@@ -417,7 +282,7 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *const (&asr
                 }
 #pragma unroll
                 for (int mt = 0; mt < NMT; mt++)
-                    t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_lo[mt], q, t[mt], 0, 0, 0);
+                    t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_lo[mt], ql, t[mt], 0, 0, 0);
 #pragma unroll
                 for (int mt = 0; mt < NMT; mt++)
 #pragma unroll
@@ -613,53 +478,99 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
 
 /* ---------------------------------------------------------------- dense */
 
-/* grid (n_out/PfDown::ROWS, ceil(T/PF_CHUNK), ks), PfDown::NT threads: one row-tiled matrix W
-   (n_out rows of n_in) times the tokens m0..m0+m-1 (m0 = blockIdx.y * PF_CHUNK) of the hi/lo
-   planes xh/xl (T rows of n_in), over the nbs blocks of 32 from b0 = blockIdx.z * nbs; written
-   to out[(blockIdx.z * T + t) * n_out + row], one part per blockIdx.z. */
-template <int ENC>
-__global__ __launch_bounds__(PfDown::NT) void k_mfma_dense(
-    const uint8_t *__restrict__ W, size_t payload_plane, int n_in, int n_out, int T, int nbs,
-    const _Float16 *__restrict__ xh, const _Float16 *__restrict__ xl, float *__restrict__ out) {
-    __shared__ __align__(16) _Float16 ah[2][PF_CHUNK * PfDown::LDA], al[2][PF_CHUNK * PfDown::LDA];
-    const int m0 = blockIdx.y * PF_CHUNK, m = min(PF_CHUNK, T - m0), nmt = (m + 15) / 16;
+#define DENSE_RW 64         /* rows per workgroup. Measured at 64, 128 and 256 (q|k|v, output
+                               projection with the sums of their parts, us): 512 tokens Q4_0 77.8,
+                               80.1, 87.1; 96 tokens 38, 39, 41; 21 tokens Q8_0 21.9, 22.7, - */
+
+/* grid (n_out / DENSE_RW, chunks, ks), PF_NT threads, dynamic LDS PfRing::P * PfRing::STAGE: one
+   row-tiled matrix W (n_out rows of n_in) times the ct <= 16 TT tokens from blockIdx.y * ct of
+   the hi/lo planes xh/xl (T rows of n_in, lo 2^11 times larger), over the nbs blocks of 32 from
+   blockIdx.z * nbs (nbs a multiple of KB); written to out[(blockIdx.z * T + t) * n_out + row],
+   one part per blockIdx.z.
+
+   The expert GEMMs' k loop over a ring of stages in LDS (pf_loop), each wavefront 16 rows for
+   the chunk's token tiles. Few tokens are bound by the launch and one trip through the ring (up
+   to 32 tokens a ring of four stages, all of a part's loads in flight at once), many by the MFMAs
+   and the LDS reads of their operands (per block and wavefront 2 token-tile operands for 2 MFMAs).
+   Against a k loop through registers (weights two stages ahead, a barrier a block): q|k|v and
+   output projection, Q4_0, us: 512 tokens 49.2 + 35.2 -> 36.6 + 26.8, 96 tokens 18.0 + 14.5 ->
+   14.7 + 12.6; and against k_gemv's passes of four tokens: 21 tokens Q8_0 46.8 + 49.4 -> 7.5 +
+   6.3, 4 tokens Q4_0 12.0 + 13.6 -> 6.0 + 5.2. */
+template <int ENC, int TT, int P, int KB>
+__global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ? 3 : 1))) void k_dense(
+    const uint8_t *__restrict__ W, size_t payload_plane, int n_in, int n_out, int T, int ct,
+    int nbs, const _Float16 *__restrict__ xh, const _Float16 *__restrict__ xl,
+    float *__restrict__ out) {
+    constexpr int RW = DENSE_RW;
+    using R = PfRing<ENC, false, TT, P, RW, KB>;
+    extern __shared__ __align__(16) uint8_t ring[];
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, g = l >> 4;
-    const int row = blockIdx.x * PfDown::ROWS + w * 16 + (l & 15);
-    const int b0 = blockIdx.z * nbs, S = nbs / PfDown::KB, nb = n_in / 32;
-    f32x4_t acc[1][PF_CHUNK / 16];
+    const int m0 = blockIdx.y * ct, m = min(ct, T - m0), nmt = (m + 15) / 16;
+    const int r0 = blockIdx.x * RW, nb = n_in / 32, b0 = blockIdx.z * nbs;
+    const _Float16 *ash[KB], *asl[KB];
 #pragma unroll
-    for (int mt = 0; mt < PF_CHUNK / 16; mt++)
-        for (int i = 0; i < 4; i++) acc[0][mt][i] = 0.0f;
-    auto row_of = [&](int i) { return m0 + i; };
-    const uint8_t *M[1] = {W};
-    const int rows[1] = {row};
-    /* the activation planes from block b0 on: stage k0 offsets then count from there */
-    const _Float16 *hi = xh + (size_t)b0 * 32, *lo = xl + (size_t)b0 * 32;
-    switch (nmt) {
-    case 1: gemm_k_loop<ENC, PfDown, 1, 1>(M, payload_plane, rows, nb, g, S, m, row_of, hi, lo, (size_t)n_in, ah, al, acc, b0); break;
-    case 2: gemm_k_loop<ENC, PfDown, 2, 1>(M, payload_plane, rows, nb, g, S, m, row_of, hi, lo, (size_t)n_in, ah, al, acc, b0); break;
-    case 3: gemm_k_loop<ENC, PfDown, 3, 1>(M, payload_plane, rows, nb, g, S, m, row_of, hi, lo, (size_t)n_in, ah, al, acc, b0); break;
-    default: gemm_k_loop<ENC, PfDown, 4, 1>(M, payload_plane, rows, nb, g, S, m, row_of, hi, lo, (size_t)n_in, ah, al, acc, b0); break;
+    for (int i = 0; i < KB; i++) {
+        const int ar = 16 * w + i * (64 / R::PP) + l / R::PP;
+        const size_t ao = (size_t)(m0 + min(ar, m - 1)) * n_in + 32 * b0 + 8 * R::apos(ar, l % R::PP);
+        ash[i] = xh + ao;
+        asl[i] = xl + ao;
     }
-    float *o = out + ((size_t)blockIdx.z * T + m0) * n_out + row;
+    const int wseg = w * R::WB / (KB * 64 * R::PB), wofs = w * R::WB % (KB * 64 * R::PB);
+    const int sseg = w * R::SB / (KB * 128), sofs = w * R::SB % (KB * 128);
+    const uint8_t *wsrc = W + ((size_t)((r0 >> 6) + wseg) * nb + b0) * 64 * R::PB + wofs;
+    const uint8_t *ssrc = W + payload_plane + ((size_t)((r0 >> 6) + sseg) * nb + b0) * 128 + sofs;
+    f32x4_t acc[R::NBT][TT];
 #pragma unroll
-    for (int mt = 0; mt < PF_CHUNK / 16; mt++)
+    for (int n = 0; n < R::NBT; n++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int r = mt * 16 + 4 * g + i;
-            if (r < m) o[(size_t)r * n_out] = acc[0][mt][i];
+        for (int mt = 0; mt < TT; mt++)
+            for (int i = 0; i < 4; i++) acc[n][mt][i] = 0.0f;
+    const size_t wstep = (size_t)KB * 64 * R::PB;
+    const int S = nbs / KB;
+    if constexpr (TT == 1) {
+        pf_loop<R, 1, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc);
+    } else if constexpr (TT == 2) {
+        if (nmt == 1) pf_loop<R, 1, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc);
+        else pf_loop<R, 2, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc);
+    } else {
+        switch (nmt) {
+        case 1: pf_loop<R, 1, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
+        case 2: pf_loop<R, 2, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
+        case 3: pf_loop<R, 3, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
+        default: pf_loop<R, 4, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
         }
+    }
+    float *o = out + ((size_t)blockIdx.z * T + m0) * n_out + r0 + RW / 4 * w + (l & 15);
+#pragma unroll
+    for (int n = 0; n < R::NBT; n++)
+#pragma unroll
+        for (int mt = 0; mt < TT; mt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int r = mt * 16 + 4 * g + i;
+                if (r < m) o[(size_t)r * n_out + 16 * n] = acc[n][mt][i];
+            }
 }
 
-/* grid ceil(n/256), 256 threads: out[i] = ((part[0][i] + part[1][i]) + part[2][i]) + ...,
-   ks parts of n floats, in part order */
-__global__ __launch_bounds__(256) void k_sum_parts(const float *__restrict__ part, int ks,
+/* grid ceil(n/512), 128 threads, n % 4 == 0: out[i] = ((part[0][i] + part[1][i]) + part[2][i]) +
+   ..., ks parts of n floats, in part order; the loads of eight parts in flight together (one
+   round trip each had been most of the launch with 16 parts) */
+__global__ __launch_bounds__(128) void k_sum_parts(const float *__restrict__ part, int ks,
                                                    size_t n, float *__restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t i = 4 * ((size_t)blockIdx.x * 128 + threadIdx.x);
     if (i >= n) return;
-    float a = part[i];
-    for (int z = 1; z < ks; z++) a = __fadd_rn(a, part[(size_t)z * n + i]);
-    out[i] = a;
+    float4 a = *(const float4 *)(part + i);
+    for (int z0 = 1; z0 < ks; z0 += 8) {
+        float4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = *(const float4 *)(part + (size_t)min(z0 + u, ks - 1) * n + i);
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (z0 + u < ks)
+                a = make_float4(__fadd_rn(a.x, v[u].x), __fadd_rn(a.y, v[u].y),
+                                __fadd_rn(a.z, v[u].z), __fadd_rn(a.w, v[u].w));
+    }
+    *(float4 *)(out + i) = a;
 }
 
 /* ---------------------------------------------------------------- combine */
@@ -739,7 +650,7 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
         if (!sel)
             LAUNCH(CPG_KT_SELECT, k_chunks, dim3(1), dim3(64), 0, grp_cnt, E, mc, chunk_grp,
                    chunk_m0);
-        LAUNCH(CPG_KT_SELECT, k_split_hilo, dim3(T), dim3(256), 0, xn, D, xh, xl);
+        LAUNCH(CPG_KT_SELECT, k_split_hilo<false>, dim3(T), dim3(256), 0, xn, D, xh, xl);
     }
     const uint8_t *ex = (const uint8_t *)L->experts;
     const size_t es = cpg_expert_bytes(ENC, D, F), mg = cpg_matrix_bytes(ENC, F, D);
@@ -787,22 +698,42 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
     return 0;
 }
 
-/* split of the k range of a dense product over T tokens: halved while every part keeps at
-   least 8 blocks of 32 and the grid stays within 1024 workgroups (four per CU) */
-static int dense_ksplit(int T, int n_in, int n_out) {
-    const int nb = n_in / 32, base = n_out / PfDown::ROWS * ((T + PF_CHUNK - 1) / PF_CHUNK);
-    int ks = 1;
-    while (ks < 16 && nb % (2 * ks) == 0 && nb / (2 * ks) >= 8 && base * 2 * ks <= 1024) ks *= 2;
-    return ks;
+/* The dense product's launch for T tokens: blocks of 32 per stage (two where the row has an
+   even number), token tiles of 16 and chunks (a workgroup's tokens, spread evenly: 96 tokens are
+   two chunks of 48, not 64 and 32), and the split of the k range, doubled while every part keeps
+   at least 8 blocks and the grid stays within 1024 workgroups. */
+struct dense_geo {
+    int kb, tt, tpc, chunks, ks;                 /* tt: the kernel's tiles; tpc: a chunk's */
+};
+static dense_geo dense_geometry(int T, int n_in, int n_out) {
+    const int nb = n_in / 32, tiles = (T + 15) / 16;
+    dense_geo d;
+    d.kb = nb % 2 ? 1 : 2;
+    d.tt = d.kb == 1 || T > 32 ? 4 : T > 16 ? 2 : 1;
+    d.chunks = (tiles + d.tt - 1) / d.tt;
+    d.tpc = (tiles + d.chunks - 1) / d.chunks;
+    d.chunks = (tiles + d.tpc - 1) / d.tpc;
+    const int base = n_out / DENSE_RW * d.chunks;
+    d.ks = 1;
+    while (d.ks < 16 && nb % (2 * d.ks * d.kb) == 0 && nb / (2 * d.ks) >= 8 &&
+           base * 2 * d.ks <= 1024)
+        d.ks *= 2;
+    return d;
 }
+static int dense_ksplit(int T, int n_in, int n_out) { return dense_geometry(T, n_in, n_out).ks; }
 
 bool cpg_dense_shape_ok(int n_in, int n_out) {
-    return n_in > 0 && n_out > 0 && n_in % PfDown::KS == 0 && n_out % PfDown::ROWS == 0;
+    return n_in > 0 && n_out > 0 && n_in % 32 == 0 && n_out % 64 == 0;
 }
 
 size_t cpg_dense_scratch_bytes(int T, int n_in, int n_out) {
     const int ks = dense_ksplit(T, n_in, n_out);
     return cpg_round256((size_t)4 * T * n_in) + (ks > 1 ? (size_t)4 * ks * T * n_out : 0);
+}
+
+template <int ENC, int TT, int P, int KB> static size_t dense_lds() {
+    using R = PfRing<ENC, false, TT, P, DENSE_RW, KB>;
+    return (size_t)R::P * R::STAGE;
 }
 
 /* the products from the hi/lo planes already in scratch: out directly (ks == 1) or ks parts
@@ -815,16 +746,30 @@ static int dense_from_planes(const void *w, int n_in, int n_out, int T, void *sc
     float *part = ks > 1 ? (float *)((uint8_t *)scratch + cpg_round256((size_t)4 * T * n_in))
                          : out;
     hipStream_t s = g_cpg.stream;
-    hipLaunchKernelGGL(k_mfma_dense<ENC>, dim3(n_out / PfDown::ROWS, (T + PF_CHUNK - 1) / PF_CHUNK, ks),
-                       dim3(PfDown::NT), 0, s, (const uint8_t *)w,
-                       cpg_payload_plane(ENC, n_out, n_in), n_in, n_out, T, n_in / 32 / ks, xh,
-                       xl, part);
-    CPG_LAUNCH_CHECK("k_mfma_dense");
+    const dense_geo d = dense_geometry(T, n_in, n_out);
+    auto go = [&](auto kernel, size_t lds) {
+        if (lds > 64 * 1024)
+            CPG_HIP(hipFuncSetAttribute((const void *)kernel,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, dim3(n_out / DENSE_RW, d.chunks, ks), dim3(PF_NT), lds, s,
+                           (const uint8_t *)w, cpg_payload_plane(ENC, n_out, n_in), n_in, n_out,
+                           T, 16 * d.tpc, n_in / 32 / ks, xh, xl, part);
+        CPG_LAUNCH_CHECK("k_dense");
+        return 0;
+    };
+#define DENSE_GO(TT, DEPTH, KB) go(k_dense<ENC, TT, DEPTH, KB>, dense_lds<ENC, TT, DEPTH, KB>())
+    int rc;
+    if (d.kb == 1) rc = DENSE_GO(4, 2, 1);
+    else if (d.tt == 1) rc = DENSE_GO(1, 4, 2);
+    else if (d.tt == 2) rc = DENSE_GO(2, 4, 2);
+    else rc = DENSE_GO(4, 2, 2);
+#undef DENSE_GO
+    if (rc) return rc;
     if (parts) *parts = part;
     if (ks_out) *ks_out = ks;
     if (ks > 1 && sum) {
         const size_t n = (size_t)T * n_out;
-        hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, part,
+        hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((n + 511) / 512)), dim3(128), 0, s, part,
                            ks, n, out);
         CPG_LAUNCH_CHECK("k_sum_parts");
     }
@@ -835,7 +780,7 @@ template <int ENC>
 static int dense_mfma(const void *w, int n_in, int n_out, const float *x, int T, void *scratch,
                       float *out) {
     _Float16 *xh = (_Float16 *)scratch, *xl = xh + (size_t)T * n_in;
-    hipLaunchKernelGGL(k_split_hilo, dim3(T), dim3(256), 0, g_cpg.stream, x, n_in, xh, xl);
+    hipLaunchKernelGGL(k_split_hilo<true>, dim3(T), dim3(256), 0, g_cpg.stream, x, n_in, xh, xl);
     CPG_LAUNCH_CHECK("k_split_hilo");
     return dense_from_planes<ENC>(w, n_in, n_out, T, scratch, out, true, nullptr, nullptr);
 }

@@ -68,7 +68,7 @@ def test_attn_vs_oracle(cpg, oracle, enc, geom):
 
 @pytest.mark.parametrize("enc,geom", [(4, "small"), (8, "small"), (4, "qwen3"), (8, "qwen3")])
 def test_attn_prefill_dense_vs_oracle(cpg, oracle, enc, geom):
-    """Prefill calls of 32 tokens and more, whose q|k|v and output projections run as MFMA
+    """Prefill calls of 33 tokens and more, whose q|k|v and output projections run as MFMA
     GEMMs with the k range split into parts: ragged token counts (70 = one full tile of 64 and
     6 more, 33, 40) between single-token calls, against the oracle with its cache."""
     from tests.attn_helpers import attn_layer, inputs, DeviceAttn
@@ -172,6 +172,33 @@ def test_attn_prefill_key_splits_vs_oracle(cpg, oracle, T, pos0, cap):
         say(f"attn splits T={T} pos0={pos0}: worst token {e:.2e}")
         assert e <= PREFILL_TOL
         assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+    finally:
+        dev.close()
+
+
+@pytest.mark.parametrize("enc,D,T", [(8, 2048, 2), (8, 2048, 3), (4, 2048, 16), (8, 2048, 17),
+                                     (4, 2048, 32), (8, 2048, 49), (4, 2048, 97), (8, 256, 3),
+                                     (4, 256, 70)])
+def test_attn_dense_token_edges_vs_oracle(cpg, oracle, enc, D, T):
+    """The MFMA projections at the edges of their token tiles and chunks (16, 32, 48 = two
+    chunks, 97 = chunks of 64 and 33), on both sides of the switch from k_gemv (2, 3), and with
+    an odd number of blocks of 32 per row of Wo (D = 256: two heads of 48, stages of one block),
+    against the oracle."""
+    from tests.attn_helpers import attn_layer, inputs, DeviceAttn
+    kw = dict(D=2048, H=32, KV=4, HD=128) if D == 2048 else dict(D=D, H=2, KV=1, HD=48)
+    a = attn_layer(enc=enc, **kw)
+    cap, kvw = T + 5, a["KV"] * a["HD"]
+    dev = DeviceAttn(a, cap=cap, max_T=T)
+    X = inputs(a["D"], 105, T)
+    kc_o, vc_o = np.zeros((cap, kvw), np.float32), np.zeros((cap, kvw), np.float32)
+    try:
+        got = dev.forward(X, 0)
+        want = oracle.attn(a, X, 0, kc_o, vc_o, threads=8)
+        kc, vc = dev.cache()
+        e = max(rel_err(got[t], want[t]) for t in range(T))
+        say(f"attn dense enc={enc} D={D} T={T}: worst token {e:.2e} k {rel_err(kc, kc_o):.2e}")
+        assert e <= PREFILL_TOL and rel_err(kc, kc_o) <= PREFILL_TOL
+        assert rel_err(vc, vc_o) <= PREFILL_TOL
     finally:
         dev.close()
 
