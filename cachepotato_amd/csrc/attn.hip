@@ -45,8 +45,11 @@
 #define AP 32               /* k_attn_split: positions per workgroup */
 #define AG 8                /* k_attn_split: query heads per kv head */
 #define AHD 128             /* k_attn_split: head dimension */
-#define ASPLIT_MAX_POS 32768 /* k_attn_split: positions its workspace holds */
-#define AMG 16              /* k_attn_split: splits merged per group of loads */
+#define ASPLIT_MAX_POS 32768 /* k_attn_split: cache rows up to which it is used */
+#define AMG 16              /* k_attn_split: partial results merged at once, one round of loads */
+#define AGS 8               /* k_attn_split: splits merged first, where there are more than AMG */
+#define ASPLIT_NS (AMG * AGS) /* k_attn_split: splits of a kv head's positions at most */
+#define ASPLIT_ROWS (ASPLIT_NS + AMG) /* k_attn_split: a head's partial rows (splits, groups) */
 
 /* grid T, 256 threads: out[t] = (x[t] * inv) * g with inv = rms_inv_row(x[t]) */
 __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float *__restrict__ x,
@@ -1219,24 +1222,67 @@ __device__ static inline void norm_rope_128(float *v, float g0, float g1, float2
     v[lane + 64] = __fadd_rn(__fmul_rn(b, cs.x), __fmul_rn(a, cs.y));
 }
 
-/* One new token (T = 1) at position pos, the AG = 8 query heads of one kv head over one split
-   of AP = 32 positions per workgroup: grid (KV, smax), 256 threads, HD == AHD, H == AG * KV.
-   Workgroup (kh, s) takes positions s*AP .. min(s*AP + AP, pos + 1) - 1; splits past pos + 1
-   leave at once. Every load is issued first: the split's cached key and value rows (one
-   float4 of each per thread and row group, clamped rows, coalesced), the 8 query heads, the
-   new key and value, the norm weights and this position's rotation pairs. Then the query
-   heads (and, in the split holding row pos, the new key) are normalised and rotated
-   (norm_rope_128), the split holding row pos writes the new key and value to the cache, the
-   rows are staged in LDS (row pos from the new key and value), thread (h, j) takes the score
-   s_hj = (q_h . k_j) / sqrtf(HD) (four partial sums over the float4 columns mod 4), and for
-   each head the split's maximum m, e_j = expf(s_hj - m), their sum l and acc = sum_j e_j v_j
-   are left in pml / pacc (agent-scope stores) for head h, split s at (h * smax + s).
-   The last of the ns = ceil((pos + 1) / AP) splits of kv head kh to count itself in at
-   ctr[kh] (which it resets for the next launch) merges them, thread (h, c) float4 c of head h:
-   M the largest m_s, w_s = expf(m_s - M) formed once per split, L = sum_s w_s l_s (a fixed
-   shuffle tree per group of AMG splits, the groups in order), o = sum_s w_s acc_s in split
-   order; ao = o / L. Up to AMG splits (positions <= AMG * AP) every load is issued at once.
-   qwen3_moe.c:144-160 in fp32, in another order (within rounding of k_attn_decode). */
+/* Up to NU partial results (m, l, acc) at rows row0 .. row0 + cnt - 1 of pml / pacc merged by the
+   32 threads of a head, thread c the float4 c of acc: M the largest m, w_u = expf(m_u - M),
+   L = sum w_u l_u (a fixed shuffle tree), o = sum w_u acc_u in row order. Every load is issued at
+   once (clamped rows, w = 0 past cnt). wsp: NU floats of LDS of the head's own. */
+template <int NU>
+__device__ __forceinline__ static void asplit_merge(const float *pacc, const float2 *pml, size_t row0,
+                                                    int cnt, int c, const uint64_t *etab, float *wsp,
+                                                    float4 &o, float &M, float &L) {
+    const unsigned long long mlb = __hip_atomic_load((unsigned long long *)(pml + row0 + min(c, cnt - 1)),
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    float4 aa[NU];
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+        const size_t hs = row0 + min(u, cnt - 1);
+        const v4i_t r = ld_agent16(pacc, (uint32_t)((hs * AHD + 4 * c) * sizeof(float)));
+        aa[u] = make_float4(__int_as_float(r.x), __int_as_float(r.y), __int_as_float(r.z),
+                            __int_as_float(r.w));
+    }
+    const float ms = __uint_as_float((uint32_t)mlb), ls = __uint_as_float((uint32_t)(mlb >> 32));
+    const bool mine = c < cnt;
+    M = half_max(mine ? ms : -INFINITY);
+    const float wgt = mine ? cpg_expf_tab(__fsub_rn(ms, M), etab) : 0.0f;
+    L = half_sum(mine ? __fmul_rn(wgt, ls) : 0.0f);
+    if (c < NU) wsp[c] = wgt;
+    wave_lds_sync();
+    o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int u = 0; u < NU; u++) {               /* w = 0 past cnt (its acc a valid row's) */
+        const float wg = wsp[u];
+        o = make_float4(fmaf(wg, aa[u].x, o.x), fmaf(wg, aa[u].y, o.y), fmaf(wg, aa[u].z, o.z),
+                        fmaf(wg, aa[u].w, o.w));
+    }
+    wave_lds_sync();                             /* wsp may be written again */
+}
+
+/* One new token (T = 1) at position pos, the AG = 8 query heads of one kv head over one split of
+   whole tiles of AP = 32 positions per workgroup: grid KV * nsp workgroups and the warming ones,
+   256 threads, HD == AHD, H == AG * KV. The ceil((pos + 1) / AP) tiles are dealt to at most
+   ASPLIT_NS splits of tps tiles each (one each up to ASPLIT_NS * AP positions); workgroup (kh, s)
+   takes tiles s * tps .., and those without a tile leave at once. The loads of the query heads,
+   the new key and value, the norm weights and the rotation pairs are issued first, then the
+   first tile's cached key and value rows (one float4 of each per thread and row group, clamped
+   rows, coalesced), which fly while the query heads (and, in the split holding row pos, the
+   new key) are normalised and rotated (norm_rope_128). The split holding row pos writes the new
+   key and value to the cache. Per tile: the rows are staged in LDS (row pos from the new key and
+   value) and the next tile's loads issued, thread (h, j) takes the score s_hj = (q_h . k_j) /
+   sqrtf(HD) (four partial sums over the float4 columns mod 4), and for each head the running
+   maximum m, l = sum expf(s_hj - m) and acc = sum_j expf(s_hj - m) v_j are carried on (rescaled
+   by expf(m_old - m) from the second tile on). m, l and acc are left in pml / pacc (agent-scope
+   stores) at row h * ASPLIT_ROWS + s.
+   Up to AMG splits: the last of a kv head's splits to count itself in at ctr[kh] (which it resets
+   for the next launch) merges them (asplit_merge) and ao = o / L. More: the last of each group of
+   AGS splits, counted at ctr[KV + kh * AMG + group], merges the group into row ASPLIT_NS + group,
+   and the last of the groups, counted at ctr[kh], merges those.
+   qwen3_moe.c:144-160 in fp32, in another order (within rounding of k_attn_decode).
+
+   What bounds it: at few positions the chain of launch, loads, norm, softmax, arrival and merge,
+   at many the reads of the cache. Before, one workgroup per kv head merged its splits of one tile
+   in groups of 16, a round trip each: 6000 positions 32.5 -> 15.6 us, 1900 15.8 -> 11.2, 200 8.0
+   -> 7.4 (the norm while the rows fly). With 64 splits (groups of 4) or 256 (of 16) at most:
+   8000 positions 19.1 and 18.4 against 16.9, 3500 13.8 and 13.8 against 13.3. */
 __global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ qkv,
                                                     const float *__restrict__ qn,
                                                     const float *__restrict__ kn,
@@ -1244,7 +1290,7 @@ __global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ qk
                                                     int KV, float eps, int pos_arg,
                                                     const int *__restrict__ pos_dev, int lim,
                                                     float *__restrict__ kc, float *__restrict__ vc,
-                                                    float *pacc, float2 *pml, int smax, int *ctr,
+                                                    float *pacc, float2 *pml, int *ctr,
                                                     float *__restrict__ ao, int *stat, int nsp,
                                                     l2_warm_t warm) {
     __shared__ __align__(16) float qs[AG][AHD];
@@ -1273,178 +1319,141 @@ __global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ qk
         }
         return;
     }
-    const int n = pos + 1, j0 = sp * AP;
-    if (j0 >= n) return;
-    const int cnt = min(AP, n - j0), kvw = KV * AHD, half = AHD / 2, ns = (n + AP - 1) / AP;
-    const bool has_new = pos < j0 + cnt;             /* this split holds the new row */
+    const int n = pos + 1, tiles = (n + AP - 1) / AP, tps = (tiles + ASPLIT_NS - 1) / ASPLIT_NS;
+    const int ns = (tiles + tps - 1) / tps, j0 = sp * tps * AP;
+    if (sp >= ns) return;
+    const int jend = min(n, j0 + tps * AP), kvw = KV * AHD, half = AHD / 2;
+    const bool has_new = pos < jend;             /* this split (the last) holds the new row */
     /* ---- every load first */
-    const int lastc = max(pos - 1, 0);
-    float4 kreg[4], vreg[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int idx = tid + 256 * r, jj = idx / (AHD / 4), c = idx % (AHD / 4);
-        const size_t o = (size_t)min(j0 + jj, lastc) * kvw + (size_t)kh * AHD + 4 * c;
-        kreg[r] = *(const float4 *)(kc + o);
-        vreg[r] = *(const float4 *)(vc + o);
-    }
     const float4 q4 = ((const float4 *)(qkv + (size_t)kh * AG * AHD))[tid];  /* [q | k | v] */
     const int tc = min(tid, AHD - 1);
     const float knew = qkv[(size_t)(H + kh) * AHD + tc], vnew = qkv[(size_t)(H + KV + kh) * AHD + tc];
     const float gq0 = qn[lane], gq1 = qn[lane + 64], gk0 = kn[lane], gk1 = kn[lane + 64];
     const float2 csl = rope[(size_t)pos * half + lane];
     const uint64_t et = cpg_exp2f_tab[tid & 31];
+    const int lastc = max(pos - 1, 0);
+    float4 kreg[4], vreg[4];
+    auto load_tile = [&](int jb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int idx = tid + 256 * r, jj = idx / (AHD / 4), c = idx % (AHD / 4);
+            const size_t o = (size_t)min(jb + jj, lastc) * kvw + (size_t)kh * AHD + 4 * c;
+            kreg[r] = *(const float4 *)(kc + o);
+            vreg[r] = *(const float4 *)(vc + o);
+        }
+    };
+    load_tile(j0);
+    __builtin_amdgcn_sched_barrier(0);           /* the tile's loads stay ahead of the waits below */
     ((float4 *)qs)[tid] = q4;
     if (tid < 32) etab[tid] = et;
     if (tid < AHD) {
         kr[tid] = knew;
         vr[tid] = vnew;
     }
-    __syncthreads();
+    lds_barrier();
     /* ---- wavefront w: query heads w and w + 4; wavefront 0 of the last split the new key */
     norm_rope_128(qs[w], gq0, gq1, csl, eps);
     norm_rope_128(qs[w + 4], gq0, gq1, csl, eps);
     if (w == 0 && has_new) norm_rope_128(kr, gk0, gk1, csl, eps);
-    __syncthreads();
+    lds_barrier();
     if (has_new && tid < AHD) {
         kc[(size_t)pos * kvw + (size_t)kh * AHD + tid] = kr[tid];
         vc[(size_t)pos * kvw + (size_t)kh * AHD + tid] = vr[tid];
     }
-    auto stage = [&](int r, float4 kv4, float4 vv4) {
-        const int idx = tid + 256 * r, jj = idx / (AHD / 4), c = idx % (AHD / 4), j = j0 + jj;
-        if (jj < cnt) {
-            if (j >= pos) {
-                kv4 = ((const float4 *)kr)[c];
-                vv4 = ((const float4 *)vr)[c];
+    /* thread (h, jj): the score; the 32 threads of a head are one half of a wavefront.
+       Thread (h, c): float4 c of the head's weighted sum of value rows. */
+    const int h = tid / AP, jj = tid % AP, c = jj;
+    float m = -INFINITY, l = 0.0f;
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int jb = j0; jb < jend; jb += AP) {
+        const int cnt = min(AP, jend - jb);
+        if (jb > j0) lds_barrier();              /* the previous tile's reads are done */
+        auto stage = [&](int r, float4 kv4, float4 vv4) __attribute__((always_inline)) {
+            const int idx = tid + 256 * r, sj = idx / (AHD / 4), sc = idx % (AHD / 4);
+            if (sj < cnt) {
+                if (jb + sj >= pos) {
+                    kv4 = ((const float4 *)kr)[sc];
+                    vv4 = ((const float4 *)vr)[sc];
+                }
+                *(float4 *)&ks[sj][4 * sc] = kv4;
+                vs[sj][sc] = vv4;
             }
-            *(float4 *)&ks[jj][4 * c] = kv4;
-            vs[jj][c] = vv4;
+        };
+        stage(0, kreg[0], vreg[0]);              /* constant indices keep kreg / vreg in registers */
+        stage(1, kreg[1], vreg[1]);
+        stage(2, kreg[2], vreg[2]);
+        stage(3, kreg[3], vreg[3]);
+        if (jb + AP < jend) load_tile(jb + AP);
+        lds_barrier();
+        float sc = -INFINITY;
+        if (jj < cnt) {
+            const float4 *qh = (const float4 *)qs[h], *kh4 = (const float4 *)ks[jj];
+            float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < AHD / 4; e++) {
+                const float4 qv = qh[e], kv = kh4[e];
+                a[e & 3] = fmaf(qv.x, kv.x, a[e & 3]);
+                a[e & 3] = fmaf(qv.y, kv.y, a[e & 3]);
+                a[e & 3] = fmaf(qv.z, kv.z, a[e & 3]);
+                a[e & 3] = fmaf(qv.w, kv.w, a[e & 3]);
+            }
+            sc = __fdiv_rn((a[0] + a[1]) + (a[2] + a[3]), cpg_sqrt_rn((float)AHD));
+        }
+        const float mt = half_max(sc);
+        if (jb > j0) {
+            const float mn = fmaxf(m, mt), f = cpg_expf_tab(__fsub_rn(m, mn), etab);
+            acc = make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f);
+            l *= f;
+            m = mn;
+        } else {
+            m = mt;
+        }
+        const float e = jj < cnt ? cpg_expf_tab(__fsub_rn(sc, m), etab) : 0.0f;
+        l += half_sum(e);
+        ps[h][jj] = e;
+        wave_lds_sync();                         /* read by the head's own half wavefront */
+        auto add = [&](int j) __attribute__((always_inline)) {
+            const float p = ps[h][j];
+            const float4 v = vs[j][c];
+            acc = make_float4(fmaf(p, v.x, acc.x), fmaf(p, v.y, acc.y), fmaf(p, v.z, acc.z),
+                              fmaf(p, v.w, acc.w));
+        };
+        if (cnt == AP) {
+#pragma unroll 8
+            for (int j = 0; j < AP; j++) add(j);
+        } else {
+            for (int j = 0; j < cnt; j++) add(j);
+        }
+    }
+    const size_t hb = (size_t)(kh * AG + h) * ASPLIT_ROWS;
+    auto put = [&](size_t row, float4 a, float mm, float ll) __attribute__((always_inline)) {
+        float *pa = pacc + row * AHD + 4 * c;
+        st_agent(pa + 0, a.x);
+        st_agent(pa + 1, a.y);
+        st_agent(pa + 2, a.z);
+        st_agent(pa + 3, a.w);
+        if (c == 0) {
+            st_agent((float *)(pml + row), mm);
+            st_agent((float *)(pml + row) + 1, ll);
         }
     };
-    stage(0, kreg[0], vreg[0]);       /* constant indices keep kreg / vreg in registers */
-    stage(1, kreg[1], vreg[1]);
-    stage(2, kreg[2], vreg[2]);
-    stage(3, kreg[3], vreg[3]);
-    __syncthreads();
-    /* ---- thread (h, jj): the score; the 32 threads of a head are one half of a wavefront */
-    const int h = tid / AP, jj = tid % AP;
-    float sc = -INFINITY;
-    if (jj < cnt) {
-        const float4 *qh = (const float4 *)qs[h], *kh4 = (const float4 *)ks[jj];
-        float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int e = 0; e < AHD / 4; e++) {
-            const float4 qv = qh[e], kv = kh4[e];
-            a[e & 3] = fmaf(qv.x, kv.x, a[e & 3]);
-            a[e & 3] = fmaf(qv.y, kv.y, a[e & 3]);
-            a[e & 3] = fmaf(qv.z, kv.z, a[e & 3]);
-            a[e & 3] = fmaf(qv.w, kv.w, a[e & 3]);
-        }
-        sc = __fdiv_rn((a[0] + a[1]) + (a[2] + a[3]), cpg_sqrt_rn((float)AHD));
+    put(hb + sp, acc, m, l);
+    float4 o;
+    float M, L;
+    size_t first = hb;
+    int parts = ns;
+    if (ns > AMG) {
+        const int g = sp / AGS, gn = min(AGS, ns - g * AGS);
+        if (!last_arriver(&ctr[KV + kh * AMG + g], gn - 1, &flag_s)) return;
+        asplit_merge<AGS>(pacc, pml, hb + g * AGS, gn, c, etab, wsp[h], o, M, L);
+        first = hb + ASPLIT_NS;
+        parts = (ns + AGS - 1) / AGS;
+        put(first + g, o, M, L);
     }
-    const float m = half_max(sc);
-    const float e = jj < cnt ? cpg_expf_tab(__fsub_rn(sc, m), etab) : 0.0f;
-    const float l = half_sum(e);
-    ps[h][jj] = e;
-    __syncthreads();
-    /* ---- thread (h, c): float4 c of the head's weighted sum of value rows */
-    const int c = tid % AP;
-    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int j = 0; j < cnt; j++) {
-        const float p = ps[h][j];
-        const float4 v = vs[j][c];
-        acc = make_float4(fmaf(p, v.x, acc.x), fmaf(p, v.y, acc.y), fmaf(p, v.z, acc.z),
-                          fmaf(p, v.w, acc.w));
-    }
-    const size_t hb = (size_t)(kh * AG + h) * smax;
-    float *pa = pacc + (hb + sp) * AHD + 4 * c;
-    st_agent(pa + 0, acc.x);
-    st_agent(pa + 1, acc.y);
-    st_agent(pa + 2, acc.z);
-    st_agent(pa + 3, acc.w);
-    if (c == 0) {
-        st_agent((float *)(pml + hb + sp), m);
-        st_agent((float *)(pml + hb + sp) + 1, l);
-    }
-    /* ---- the last split of this kv head merges */
-    if (!last_arriver(&ctr[kh], ns - 1, &flag_s)) return;
-    /* Thread (h, c): float4 c of head h. The weights w_s = expf(m_s - M) (M the largest m_s)
-       and L = sum_s w_s l_s are formed once per split by the head's 32 threads (split
-       s0 + lane32 each) and shared through LDS within the wavefront; each thread then adds
-       w_s acc_s over its splits in order, the loads of a group of AMG splits issued at once
-       with the (m, l) of the group. */
-    const int l32 = tid & 31;
-    if (ns <= AMG) {
-        /* one round of loads: split l32's (m, l), then every split's acc */
-        const unsigned long long mlb = __hip_atomic_load(
-            (unsigned long long *)(pml + hb + min(l32, ns - 1)), __ATOMIC_RELAXED,
-            __HIP_MEMORY_SCOPE_AGENT);
-        float4 aa[AMG];
-#pragma unroll
-        for (int u = 0; u < AMG; u++) {
-            const size_t hs = hb + min(u, ns - 1);
-            const v4i_t r = ld_agent16(pacc, (uint32_t)((hs * AHD + 4 * c) * sizeof(float)));
-            aa[u] = make_float4(__int_as_float(r.x), __int_as_float(r.y), __int_as_float(r.z),
-                                __int_as_float(r.w));
-        }
-        const float ms = __uint_as_float((uint32_t)mlb), ls = __uint_as_float((uint32_t)(mlb >> 32));
-        const bool mine = l32 < ns;
-        const float M1 = half_max(mine ? ms : -INFINITY);
-        const float wgt = mine ? cpg_expf_tab(__fsub_rn(ms, M1), etab) : 0.0f;
-        const float L1 = half_sum(mine ? __fmul_rn(wgt, ls) : 0.0f);
-        if (l32 < AMG) wsp[h][l32] = wgt;
-        wave_lds_sync();
-        float4 o1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-        for (int u = 0; u < AMG; u++) {          /* w = 0 past ns (its acc a valid split's) */
-            const float wg = wsp[h][u];
-            o1 = make_float4(fmaf(wg, aa[u].x, o1.x), fmaf(wg, aa[u].y, o1.y),
-                             fmaf(wg, aa[u].z, o1.z), fmaf(wg, aa[u].w, o1.w));
-        }
-        *(float4 *)(ao + (size_t)(kh * AG + h) * AHD + 4 * c) =
-            make_float4(__fdiv_rn(o1.x, L1), __fdiv_rn(o1.y, L1), __fdiv_rn(o1.z, L1),
-                        __fdiv_rn(o1.w, L1));
-        return;
-    }
-    float M = -INFINITY;
-    for (int s0 = 0; s0 < ns; s0 += 32) {
-        const int sidx = min(s0 + l32, ns - 1);
-        M = fmaxf(M, ld_agent((const float *)(pml + hb + sidx)));
-    }
-    for (int o = 16; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
-    float L = 0.0f;
-    float4 o4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int s0 = 0; s0 < ns; s0 += AMG) {
-        float4 aa[AMG];
-#pragma unroll
-        for (int u = 0; u < AMG; u++) {          /* clamped, unconditional: in flight together */
-            const size_t hs = hb + min(s0 + u, ns - 1);
-            const v4i_t r = ld_agent16(pacc, (uint32_t)((hs * AHD + 4 * c) * sizeof(float)));
-            aa[u] = make_float4(__int_as_float(r.x), __int_as_float(r.y), __int_as_float(r.z),
-                                __int_as_float(r.w));
-        }
-        /* the group's weights: lane l32 < AMG of head h takes split s0 + l32 */
-        {
-            const bool mine = l32 < AMG && s0 + l32 < ns;
-            const size_t hs = hb + min(s0 + (l32 < AMG ? l32 : 0), ns - 1);
-            const float ms = ld_agent((const float *)(pml + hs));
-            const float ls = ld_agent((const float *)(pml + hs) + 1);
-            const float wgt = mine ? cpg_expf_tab(__fsub_rn(ms, M), etab) : 0.0f;
-            float lw = mine ? __fmul_rn(wgt, ls) : 0.0f;
-            for (int o = 1; o < 32; o <<= 1) lw += __shfl_xor(lw, o);
-            L = __fadd_rn(L, lw);
-            if (l32 < AMG) wsp[h][l32] = wgt;
-            wave_lds_sync();
-        }
-#pragma unroll
-        for (int u = 0; u < AMG; u++) {          /* w = 0 past ns (its acc a valid split's) */
-            const float wg = wsp[h][u];
-            o4 = make_float4(fmaf(wg, aa[u].x, o4.x), fmaf(wg, aa[u].y, o4.y),
-                             fmaf(wg, aa[u].z, o4.z), fmaf(wg, aa[u].w, o4.w));
-        }
-        wave_lds_sync();                         /* wsp is rewritten by the next group */
-    }
+    if (!last_arriver(&ctr[kh], parts - 1, &flag_s)) return;
+    asplit_merge<AMG>(pacc, pml, first, parts, c, etab, wsp[h], o, M, L);
     *(float4 *)(ao + (size_t)(kh * AG + h) * AHD + 4 * c) =
-        make_float4(__fdiv_rn(o4.x, L), __fdiv_rn(o4.y, L), __fdiv_rn(o4.z, L), __fdiv_rn(o4.w, L));
+        make_float4(__fdiv_rn(o.x, L), __fdiv_rn(o.y, L), __fdiv_rn(o.z, L), __fdiv_rn(o.w, L));
 }
 
 /* ================================================================ host side */
@@ -1538,11 +1547,11 @@ extern "C" int cpg_gemv_norm(int enc, const void *w, int n_in, int n_out, const 
 struct cpg_attn_ws {
     int D, H, KV, HD, max_T;
     float *qkv, *q, *ao;
-    float *pacc;            /* k_attn_split: (H, ASPLIT_MAX_POS / AP, HD); k_attn_mma: mma_rows
+    float *pacc;            /* k_attn_split: (H, ASPLIT_ROWS, HD); k_attn_mma: mma_rows
                                of 128; or null */
     float2 *pml;            /* the same rows' maxima and sums */
     size_t mma_rows;
-    int *ctr;               /* k_attn_split: KV arrival counters, zero between launches */
+    int *ctr;               /* k_attn_split: KV (1 + AMG) arrival counters, zero between launches */
     int *stat;              /* 1 once a kernel saw a position outside the cache */
     void *dense;            /* cpg_dense_mfma for T >= DENSE_MIN_T, or null */
     void *block;
@@ -1584,14 +1593,14 @@ extern "C" cpg_attn_ws *cpg_attn_ws_create(int D, int H, int KV, int HD, int max
     cpg_attn_ws *ws = (cpg_attn_ws *)calloc(1, sizeof *ws);
     if (!ws) { cpg_set_error("out of host memory"); return nullptr; }
     ws->D = D; ws->H = H; ws->KV = KV; ws->HD = HD; ws->max_T = max_T;
-    const size_t T = (size_t)max_T, smax = ASPLIT_MAX_POS / AP;
+    const size_t T = (size_t)max_T;
     const bool split = attn_split_shape(H, KV, HD);
     /* partial rows: (head, split) of one token in k_attn_split; (split, token, head) in
        k_attn_mma, whose AMMA_WGS workgroups leave at most 128 rows each */
     ws->mma_rows = attn_mma_shape(H, KV, HD) && max_T >= AMMA_MIN_T
                        ? (size_t)AMMA_WGS * 128 : 0;
     if (ws->mma_rows > AMMA_MAX_NS * T * H) ws->mma_rows = AMMA_MAX_NS * T * H;
-    const size_t srows = split ? H * smax : 0;
+    const size_t srows = split ? (size_t)H * ASPLIT_ROWS : 0;
     const size_t rows = srows > ws->mma_rows ? srows : ws->mma_rows;
     const int nqkv = (H + 2 * KV) * HD;
     size_t dense = 0;
@@ -1604,7 +1613,7 @@ extern "C" cpg_attn_ws *cpg_attn_ws_create(int D, int H, int KV, int HD, int max
         }
     const size_t sz[8] = {T * nqkv * 4, T * H * HD * 4, T * H * HD * 4,
                           rows * HD * 4, rows * 8, dense,
-                          split ? (size_t)KV * 4 : 0, 4};
+                          split ? (size_t)KV * (1 + AMG) * 4 : 0, 4};
     size_t total = 0;
     for (int i = 0; i < 8; i++) total += cpg_round256(sz[i]);
     uint8_t *p = (uint8_t *)cpg_malloc(total);
@@ -1724,14 +1733,14 @@ static int attn_forward(const cpg_attn_layer *A, const float *x, int T, int pos0
     const size_t smem = sizeof(float) * (size_t)nmax;
     bool planes = false;                         /* the output projection's planes written */
     if (T == 1 && g_attn_mode == CPG_ATTN_SPLIT && ws->ctr && lim <= ASPLIT_MAX_POS) {
-        const int smax = (lim + AP - 1) / AP;
+        const int tiles = (lim + AP - 1) / AP, nsp = tiles < ASPLIT_NS ? tiles : ASPLIT_NS;
         /* while the few attention workgroups run, the output projection's rows are read into
            the L2 of the XCD whose workgroups will read them */
         const l2_warm_t warm = l2_warm_rows(A->enc, A->wo, D, H * HD);
-        hipLaunchKernelGGL(k_attn_split, dim3(KV * smax + NXCD * warm.parts), dim3(256), 0, s,
+        hipLaunchKernelGGL(k_attn_split, dim3(KV * nsp + NXCD * warm.parts), dim3(256), 0, s,
                            ws->qkv, A->q_norm, A->k_norm, (const float2 *)A->rope, H, KV, A->eps,
-                           pos0, pos_dev, lim, kc, vc, ws->pacc, ws->pml, ASPLIT_MAX_POS / AP,
-                           ws->ctr, ws->ao, ws->stat, smax, warm);
+                           pos0, pos_dev, lim, kc, vc, ws->pacc, ws->pml, ws->ctr, ws->ao, ws->stat,
+                           nsp, warm);
         CPG_LAUNCH_CHECK("k_attn_split");
     } else if (T == 1) {
         if (smem > 32 * 1024)

@@ -279,6 +279,33 @@ def test_attn_decode_long_context_vs_oracle(cpg, oracle, pos, mode):
     assert np.array_equal(kc[:pos].view(np.uint32), kc0[:pos].view(np.uint32))
 
 
+@pytest.mark.parametrize("pos", [511, 512, 4095, 4096, 8191])
+def test_attn_decode_split_groups_vs_oracle(cpg, oracle, pos):
+    """The split one-token kernel where its merge changes form: 16 splits (merged at once) and 17
+    (in groups), 128 splits of one tile of 32 and 65 of two, and the last position of the
+    longest context; twice each (the arrival counters are left zero), the position given by
+    the host and read on the device, against the oracle."""
+    from tests.attn_helpers import attn_layer, inputs, DeviceAttn
+    a = attn_layer(enc=8, D=2048, H=32, KV=4, HD=128)
+    cap, kvw = max(pos + 1, 8192 if pos < 4096 else 0), a["KV"] * a["HD"]
+    rng = np.random.default_rng(pos)
+    kc0, vc0 = rng.standard_normal((2, cap, kvw), dtype=np.float32)
+    kc0[pos:], vc0[pos:] = 0.0, 0.0
+    x = inputs(a["D"], 600 + pos, 1)
+    dev = DeviceAttn(a, cap=cap, max_T=1)
+    try:
+        dev.set_cache(kc0, vc0)
+        got = dev.forward(x, pos)
+        again = dev.forward_at(x, pos)
+    finally:
+        dev.close()
+    want = oracle.attn(a, x, pos, kc0.copy(), vc0.copy(), threads=8)
+    e = rel_err(got, want)
+    say(f"decode attention at position {pos}: out {e:.2e}")
+    assert e <= PREFILL_TOL
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+
+
 @pytest.mark.parametrize("P0,N,cap", [(20, 100, 128), (222, 262, 320)])
 def test_attn_decode_splits_vs_oracle(cpg, oracle, P0, N, cap):
     """One token at a time from position P0 to N - 1 after a P0-token prefill: positions 20-99
