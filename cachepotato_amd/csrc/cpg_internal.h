@@ -88,6 +88,9 @@ hipEvent_t *cpg_timing_pair(int slot);
 
 /* prefill.hip: the MFMA grouped expert GEMMs for many tokens */
 int cpg_prefill_max_chunks(int T, int K, int E);
+/* the most chunks of any call of up to T tokens, and the tokens per chunk of a call of T */
+int cpg_prefill_chunks_upto(int T, int K, int E);
+int cpg_prefill_chunk(int T, int K, int E);
 bool cpg_prefill_shape_ok(int D, int F);
 /* scratch: cpg_prefill_scratch_bytes (the hi/lo f16 planes of xn, then those of h).
    prepared: the routing step has written the chunk list (pf_chunk_list) and the planes of

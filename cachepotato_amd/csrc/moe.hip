@@ -312,7 +312,7 @@ __device__ static void bucket_pairs(const int *__restrict__ topk, int T, int K, 
 /* One wavefront, after bucket_pairs (cnt final): the chunk list of the groups (pf_chunk_list;
    group g is the g-th expert with pairs, in expert order, as bucket_pairs numbers them);
    experts 4t..4t+3 of lane t. */
-__device__ static void chunks_of_counts(const int *cnt, int E, int max_chunks, int *chunk_grp,
+__device__ static void chunks_of_counts(const int *cnt, int E, int ch, int max_chunks, int *chunk_grp,
                                         int *chunk_m0) {
     static_assert(MAX_E / WAVE == 4, "four experts per lane");
     const int t = threadIdx.x;
@@ -334,7 +334,7 @@ __device__ static void chunks_of_counts(const int *cnt, int E, int max_chunks, i
         g[k] = gi;
         gi += c[k] > 0;
     }
-    pf_chunk_list(c, g, max_chunks, chunk_grp, chunk_m0);
+    pf_chunk_list(c, g, ch, max_chunks, chunk_grp, chunk_m0);
 }
 
 /* grid (ceil(E/RPW), T), 256 threads. Every workgroup of a token computes the token's RMSNorm
@@ -1350,7 +1350,7 @@ __global__ __launch_bounds__(64 * route_rows(NQ)) void k_route_fast(
     int *__restrict__ pair_pos, int *__restrict__ list_tok, int *__restrict__ list_pair,
     int *__restrict__ grp_expert, int *__restrict__ grp_off, int *__restrict__ grp_cnt,
     int *__restrict__ n_groups, _Float16 *__restrict__ xh, _Float16 *__restrict__ xl,
-    int max_chunks, int *__restrict__ chunk_grp, int *__restrict__ chunk_m0) {
+    int ch, int max_chunks, int *__restrict__ chunk_grp, int *__restrict__ chunk_m0) {
     extern __shared__ __align__(16) float smem[];   /* float4 accesses: 16-byte aligned */
     __shared__ int flag_s;
     __shared__ uint64_t tab[32];
@@ -1479,7 +1479,7 @@ __global__ __launch_bounds__(64 * route_rows(NQ)) void k_route_fast(
     __syncthreads();
     bucket_pairs(tk_all, T, K, E, mask, base, cnt, pair_pos, list_tok, list_pair, grp_expert,
                  grp_off, grp_cnt, n_groups);
-    if (chunk_grp && tid < WAVE) chunks_of_counts(cnt, E, max_chunks, chunk_grp, chunk_m0);
+    if (chunk_grp && tid < WAVE) chunks_of_counts(cnt, E, ch, max_chunks, chunk_grp, chunk_m0);
 }
 
 /* ================================================================ routing, T > 16 */
@@ -1655,13 +1655,13 @@ __global__ __launch_bounds__(1024) void k_bucket(
     const int *__restrict__ topk, int T, int K, int E, int *__restrict__ pair_pos,
     int *__restrict__ list_tok, int *__restrict__ list_pair, int *__restrict__ grp_expert,
     int *__restrict__ grp_off, int *__restrict__ grp_cnt, int *__restrict__ n_groups,
-    int max_chunks, int *__restrict__ chunk_grp, int *__restrict__ chunk_m0) {
+    int ch, int max_chunks, int *__restrict__ chunk_grp, int *__restrict__ chunk_m0) {
     __shared__ unsigned long long mask[(BUCKET_MAX_T / 64) * MAX_E];
     __shared__ int base[MAX_E], cnt[MAX_E];
     bucket_pairs(topk, T, K, E, mask, base, cnt, pair_pos, list_tok, list_pair, grp_expert,
                  grp_off, grp_cnt, n_groups);
     /* cnt is final since bucket_pairs' last barrier */
-    if (chunk_grp && threadIdx.x < WAVE) chunks_of_counts(cnt, E, max_chunks, chunk_grp, chunk_m0);
+    if (chunk_grp && threadIdx.x < WAVE) chunks_of_counts(cnt, E, ch, max_chunks, chunk_grp, chunk_m0);
 }
 
 /* ================================================================ expert GEMVs */
@@ -2395,7 +2395,7 @@ static size_t moe_ws_carve(cpg_moe_ws *ws, uint8_t *base, int D, int E, int K, i
                            int max_T, int cnt_D, int cnt_T) {
     const size_t TK = (size_t)max_T * K;
     enum { N = 23 };
-    const size_t mc = (size_t)cpg_prefill_max_chunks(max_T, K, E);
+    const size_t mc = (size_t)cpg_prefill_chunks_upto(max_T, K, E);
     const size_t sz[N] = {(SMALL_T + 1) * 4, (size_t)cnt_T * (cnt_D / 64) * 4, 16,
                           sizeof(moe1_state), 4,
                           (size_t)max_T * D * 4, (size_t)max_T * E * 4, TK * 4,
@@ -2603,9 +2603,10 @@ static int route_fast(const cpg_moe_layer *L, const float *x, const float *attn,
        (in the expert scratch) and the chunk list */
     _Float16 *xh = planes ? (_Float16 *)ws->gu : nullptr;
     const int mc = planes ? cpg_prefill_max_chunks(T, L->K, E) : 0;
+    const int ch = cpg_prefill_chunk(T, L->K, E);
 #define ROUTE_FAST_ARGS x, attn, L->ln2, L->wgate, T, D, E, L->K, L->eps, force, ws->xn, ws->rec, ws->ctr, \
         tk, wt, ws->stat, select, bucket, ws->pair_pos, ws->list_tok, ws->list_pair, ws->grp_expert, ws->grp_off,  \
-        ws->grp_cnt, ws->n_groups, xh, xh ? xh + (size_t)T * D : nullptr, mc, \
+        ws->grp_cnt, ws->n_groups, xh, xh ? xh + (size_t)T * D : nullptr, ch, mc, \
         planes ? ws->chunk_grp : nullptr, ws->chunk_m0
     switch (D / 256) {
     case 1: LAUNCH(CPG_KT_ROUTE, k_route_fast<1>, grid, block, smem, ROUTE_FAST_ARGS); break;
@@ -2878,16 +2879,21 @@ static int moe_forward(const cpg_moe_layer *L, const float *x, const float *attn
     int *tk_d = topk ? topk : ws->topk;
     float *wt_d = wt ? wt : ws->wt;
 
-    /* many tokens: the expert products as MFMA grouped GEMMs (prefill.hip) */
+    const bool fast = T <= SMALL_T && !xn && !router && g_route_mode != CPG_ROUTE_EXACT &&
+                      fast_shape(D);
+    /* The expert products as MFMA grouped GEMMs (prefill.hip): from PREFILL_MIN_T tokens, and
+       from two where the routing is the certified one, which writes their planes and whose
+       selections they read (the batch GEMVs against them, us per layer with the routing: 2 tokens
+       Q4_0 43.5, 41.7, 4 tokens 62.9, 47.4, Q8_0 68.2, 51.3, 7 tokens 90.2, 57.1). A call that asks for xn or the router's logits keeps
+       the GEMVs below PREFILL_MIN_T: its outputs are those of one token at a time, bit for bit. */
     const bool mfma = cpg_prefill_shape_ok(D, F) &&
                       cpg_prefill_scratch_bytes(T, D, K, F) <= (size_t)T * K * 2 * KS * F * 4 &&
                       (g_expert_mode == CPG_EXPERTS_MFMA ||
-                       (g_expert_mode == CPG_EXPERTS_AUTO && T >= PREFILL_MIN_T));
+                       (g_expert_mode == CPG_EXPERTS_AUTO &&
+                        (T >= PREFILL_MIN_T || (fast && T >= 2 && cpg_prefill_sel_ok(T, K, E)))));
     bool prepared = false;      /* chunk list and xn planes formed by the routing step */
 
     /* routing, selection, bucketing */
-    const bool fast = T <= SMALL_T && !xn && !router && g_route_mode != CPG_ROUTE_EXACT &&
-                      fast_shape(D);
     const bool one = fast && T == 1 && one_token_shape(D, K, F) && E * CR_P <= GW * 64;
     if (one && g_fused) {
         const int rc = moe1(L, x, attn, topk, wt, mlp, xres, ws);
@@ -2928,7 +2934,8 @@ static int moe_forward(const cpg_moe_layer *L, const float *x, const float *attn
         LAUNCH(CPG_KT_SELECT, k_select, dim3(T), dim3(64), 0, lg_d, E, K, tk_d, wt_d);
         LAUNCH(CPG_KT_SELECT, k_bucket, dim3(1), dim3(1024), 0, tk_d, T, K, E, ws->pair_pos,
                ws->list_tok, ws->list_pair, ws->grp_expert, ws->grp_off, ws->grp_cnt,
-               ws->n_groups, cpg_prefill_max_chunks(T, K, E), mfma ? ws->chunk_grp : nullptr,
+               ws->n_groups, cpg_prefill_chunk(T, K, E), cpg_prefill_max_chunks(T, K, E),
+               mfma ? ws->chunk_grp : nullptr,
                ws->chunk_m0);
         prepared = mfma;
     }

@@ -28,8 +28,8 @@
  * tokens is three chunks); a workgroup of 4 wavefronts computes 128 rows of each of its
  * matrices for one chunk (gate/up: 128 rows of Wg and the same rows of Wu, so SwiGLU pairs
  * are in one lane; down: 128 rows of Wd), each wavefront 32 rows for every non-empty token
- * tile of 16 (a chunk of 20 tokens costs 2 tiles, not 4). Batches of at most 16 tokens (one
- * token tile per chunk) use a variant with 64 gate/up rows per workgroup and a ring of four
+ * tile of 16 (a chunk of 20 tokens costs 2 tiles, not 4). Calls whose experts have few tokens
+ * (cpg_prefill_chunk) take chunks of one token tile and use a variant with 64 gate/up rows per workgroup and a ring of four
  * stages: there the VALU weight conversion, not the MFMAs, sets each wavefront's pace, and
  * twice the workgroups spread it over the CUs. The activations are split into
  * hi/lo f16 planes once per call (k_split_hilo for xn; the gate/up epilogue writes h split).
@@ -44,7 +44,7 @@
 
 /* One wavefront: the chunk list over the groups the routing step formed (pf_chunk_list), for
    routing steps that do not form it themselves; lane t takes groups 4t..4t+3 (E <= 256). */
-__global__ __launch_bounds__(64) void k_chunks(const int *__restrict__ grp_cnt, int E,
+__global__ __launch_bounds__(64) void k_chunks(const int *__restrict__ grp_cnt, int E, int ch,
                                                int max_chunks, int *__restrict__ chunk_grp,
                                                int *__restrict__ chunk_m0) {
     int cnt[4], grp[4];
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(64) void k_chunks(const int *__restrict__ grp_cnt, 
         grp[j] = 4 * threadIdx.x + j;
         cnt[j] = grp[j] < E ? grp_cnt[grp[j]] : 0;
     }
-    pf_chunk_list(cnt, grp, max_chunks, chunk_grp, chunk_m0);
+    pf_chunk_list(cnt, grp, ch, max_chunks, chunk_grp, chunk_m0);
 }
 
 /* grid rows, 256 threads: hi[r] = f16(x[r]), lo[r] = f16(x[r] - hi[r]) for rows of n floats
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void k_split_hilo(const float *__restrict__ x,
    workgroup (4 wavefronts) computes 128 rows of each of its matrices for the chunk; a
    wavefront 32 rows of each (GU: gate rows, up rows: four 16-row B tiles; down: two). */
 #define PF_NT 256
-/* batches of at most 16 tokens: ring depth, rows of each matrix per workgroup (gate/up,
+/* chunks of one token tile: ring depth, rows of each matrix per workgroup (gate/up,
    down), blocks per stage; measured at 16 tokens (gate/up, down us): 128 rows in rings of 4
    38.4, 16.6; 64 rows 29.3, 20.1; 64 rows in rings of 6 30.9, 22.4; stages of 4 blocks in
    rings of 3 28.3 (gate/up, against 28.0 with stages of 2), in rings of 4 32.7 */
@@ -107,6 +107,7 @@ __global__ __launch_bounds__(256) void k_split_hilo(const float *__restrict__ x,
 #define PF_SMALL_RW_GU 64
 #define PF_SMALL_RW_DN 128
 #define PF_SMALL_KB 2
+#define PF_SUM 4            /* pf_loop: stages whose sums are taken together, one token tile */
 #define R_Q_FITS(q, p) ((q) * ((p) - 2) < 64)   /* the stage wait's vmcnt fits its field */
 
 template <int ENC, bool GU, int TT_ = PF_CHUNK / 16, int P_ = 2, int RW_ = 128, int KB_ = 2>
@@ -241,8 +242,29 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *const (&asr
         boff[n] = (seg * KB * 64 + rs) * R::PB + (ENC == CPG_ENC_Q4 ? 8 * (g & 1) : 8 * g);
         soff[n] = (seg * KB * 64 + rs) * 2;
     }
+    /* one token tile: the sums are taken PF_SUM stages at a time and added up, which takes a fifth
+       off the error of one chain over all blocks (a layer at 16 tokens 3.5e-7 -> 2.8e-7 against 64
+       bits; more tiles have no registers for it) */
+    constexpr bool PARTS = R::TT == 1;
+    f32x4_t tot[PARTS ? R::NBT : 1][PARTS ? NMT : 1];
+    if constexpr (PARTS) {
+#pragma unroll
+        for (int n = 0; n < R::NBT; n++)
+#pragma unroll
+            for (int mt = 0; mt < NMT; mt++) tot[n][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
     for (int st = 0; st < R::P - 1; st++) issue(st);
     for (int s = 0; s < S; s++) {
+        if constexpr (PARTS) {
+            if (s % PF_SUM == 0)
+#pragma unroll
+                for (int n = 0; n < R::NBT; n++)
+#pragma unroll
+                    for (int mt = 0; mt < NMT; mt++) {
+                        tot[n][mt] += acc[n][mt];
+                        acc[n][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+        }
         asm volatile("" ::: "memory");
         /* stage s has landed when at most the later stages' loads are in flight: Q per stage
            for a wavefront that loads A tiles, Q - 2 * KB for one that does not */
@@ -289,6 +311,12 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *const (&asr
                     for (int i = 0; i < 4; i++) acc[n][mt][i] = fmaf(d, t[mt][i], acc[n][mt][i]);
             }
         }
+    }
+    if constexpr (PARTS) {
+#pragma unroll
+        for (int n = 0; n < R::NBT; n++)
+#pragma unroll
+            for (int mt = 0; mt < NMT; mt++) acc[n][mt] += tot[n][mt];
     }
     /* no load may still write this workgroup's LDS when it ends */
     asm volatile("" ::: "memory");
@@ -394,7 +422,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
         if (grp < 0) return;
         e = grp_expert[grp];
         const int off = grp_off[grp], m0 = chunk_m0[c];
-        m = min(PF_CHUNK, grp_cnt[grp] - m0);
+        m = min(16 * TT, grp_cnt[grp] - m0);
         if (tid < PF_CHUNK) {
             const int i = min(tid, m - 1);
             arow[tid] = GU ? list[off + m0 + i] : off + m0 + i;
@@ -618,13 +646,29 @@ __global__ __launch_bounds__(256) void k_pair_combine(const float *__restrict__ 
 
 /* ---------------------------------------------------------------- host */
 
-/* the most chunks T tokens with K experts each over E experts can form */
-int cpg_prefill_max_chunks(int T, int K, int E) {
+static int max_chunks(int T, int K, int E, int ch) {
     const int pairs = T * K;
     const int groups = pairs < E ? pairs : E;
-    const int n = (pairs + PF_CHUNK - 1) / PF_CHUNK + groups;
+    const int n = (pairs + ch - 1) / ch + groups;
     return (n + 7) / 8 * 8;                      /* k_pf_gemm places chunk c on XCD c % 8 */
 }
+
+/* Tokens per chunk of T tokens with K experts each: one tile of 16 while the experts have 8 tokens
+   each on average, so that nearly every expert is one chunk: the one-tile GEMMs' deeper ring and
+   smaller workgroups then keep more of the weights in flight (us per layer with the routing,
+   chunks of 64 and of 16: 45 tokens Q4_0 122.7, 120.7, Q8_0 skewed 148.3, 135.0; 96 tokens 125.9,
+   126.1 and 170.8, 161.2). Above, an expert's second chunk reads its weights again: 160 tokens
+   132.7, 134.2 and 187.2, 185.6; 256 tokens Q4_0 154, 170. */
+int cpg_prefill_chunk(int T, int K, int E) {
+    return T <= 16 || T * K <= 8 * E ? 16 : PF_CHUNK;
+}
+
+/* the most chunks T tokens with K experts each over E experts can form */
+int cpg_prefill_max_chunks(int T, int K, int E) {
+    return max_chunks(T, K, E, cpg_prefill_chunk(T, K, E));
+}
+
+int cpg_prefill_chunks_upto(int T, int K, int E) { return max_chunks(T, K, E, 16); }
 
 bool cpg_prefill_shape_ok(int D, int F) {
     return D % 128 == 0 && F % 128 == 0;
@@ -648,8 +692,8 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
     _Float16 *hh = xl + (size_t)T * D, *hl = hh + (size_t)T * K * F;
     if (!prepared) {
         if (!sel)
-            LAUNCH(CPG_KT_SELECT, k_chunks, dim3(1), dim3(64), 0, grp_cnt, E, mc, chunk_grp,
-                   chunk_m0);
+            LAUNCH(CPG_KT_SELECT, k_chunks, dim3(1), dim3(64), 0, grp_cnt, E,
+                   cpg_prefill_chunk(T, K, E), mc, chunk_grp, chunk_m0);
         LAUNCH(CPG_KT_SELECT, k_split_hilo<false>, dim3(T), dim3(256), 0, xn, D, xh, xl);
     }
     const uint8_t *ex = (const uint8_t *)L->experts;
@@ -673,8 +717,8 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
         return 0;
     };
     int rc;
-    if (T <= 16) {
-        /* every expert group holds at most T <= 16 tokens: one token tile, a deeper ring */
+    if (cpg_prefill_chunk(T, K, E) == 16) {
+        /* chunks of one token tile: a deeper ring */
         using RG = PfRing<ENC, true, 1, PF_SMALL_RING, PF_SMALL_RW_GU, PF_SMALL_KB>;
         using RD = PfRing<ENC, false, 1, PF_SMALL_RING, PF_SMALL_RW_DN, PF_SMALL_KB>;
         rc = gemms(k_pf_gemm<ENC, true, 1, PF_SMALL_RING, PF_SMALL_RW_GU, PF_SMALL_KB>,
@@ -682,7 +726,6 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
                    k_pf_gemm<ENC, false, 1, PF_SMALL_RING, PF_SMALL_RW_DN, PF_SMALL_KB>,
                    (size_t)RD::P * RD::STAGE, RD::RW);
     } else {
-        if (sel) { cpg_set_error("prefill_experts: selections need T <= 16"); return -1; }
         using RG = PfRing<ENC, true>;
         using RD = PfRing<ENC, false>;
         rc = gemms(k_pf_gemm<ENC, true>, (size_t)RG::P * RG::STAGE, RG::RW,

@@ -198,11 +198,12 @@ int cpg_moe_ws_exact_routings(cpg_moe_ws *ws);
 int cpg_moe_route_mode(int mode);
 
 /* Expert computation of cpg_moe_forward for T tokens.
- *   CPG_EXPERTS_AUTO (default): from 8 tokens the MFMA grouped GEMMs (f16 MFMA on the exact
- *     quantised weights with the block scale folded in as exact hi + lo halves, activations
- *     split into f16 hi + lo, fp32 accumulation), below that the grouped dequant-fused GEMVs
- *     (whose results do not depend on the batch a token is in); one token always the
- *     one-token GEMVs.
+ *   CPG_EXPERTS_AUTO (default): the MFMA grouped GEMMs (f16 MFMA on the exact quantised
+ *     weights, the block scale applied in fp32, activations split into f16 hi + lo, fp32
+ *     accumulation) from 8 tokens, and from 2 where neither xn nor the router's logits are asked
+ *     for; the grouped dequant-fused GEMVs for 2 to 7 tokens with either (there a token's
+ *     outputs are those of one token with either, bit for bit); one token always the one-token
+ *     GEMVs. Up to 16 tokens the experts' sums do not depend on the batch a token is in.
  *   CPG_EXPERTS_GEMV / CPG_EXPERTS_MFMA: always the one path for T > 1 (for testing). */
 #define CPG_EXPERTS_AUTO 0
 #define CPG_EXPERTS_GEMV 1

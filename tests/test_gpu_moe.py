@@ -584,6 +584,41 @@ def test_moe_small_mfma_vs_oracle(cpg, oracle, small, T):
         assert e <= SPLIT_TOL
 
 
+@pytest.mark.parametrize("T", [2, 7, 16])
+def test_moe_small_certified_batch_invariance(small, T):
+    """Certified calls of 2 to 16 tokens (the one-tile GEMMs, reading the selections): a token's
+    outputs do not depend on the batch it is in, bit for bit, and agree with the grouped GEMVs
+    within rounding."""
+    import cachepotato_amd as C
+    from cachepotato_amd import synth
+    x = synth.inputs(small.spec, 7000, 16)
+    ref = small.forward(x, outputs=False)
+    got = small.forward(x[16 - T:], outputs=False)
+    for k in ("topk", "wt", "mlp"):
+        assert np.array_equal(got[k].view(np.uint32), ref[k][16 - T:].view(np.uint32)), k
+    with expert_mode(C.EXPERTS_GEMV):
+        gemv = small.forward(x[16 - T:], outputs=False)
+    assert np.array_equal(got["topk"], gemv["topk"])
+    assert rel_err(got["mlp"], gemv["mlp"]) <= SPLIT_TOL
+
+
+@pytest.mark.parametrize("T", [17, 32, 33])
+def test_moe_small_crowded_experts_vs_oracle(cpg, oracle, small, T):
+    """Every token takes the same experts, so each has T tokens: chunks of 16 (17 = one row past a
+    chunk, 32 = the last call with them at 16 experts) and chunks of 64 (33), against the
+    oracle."""
+    from cachepotato_amd import synth
+    spec = small.spec
+    x = np.repeat(synth.inputs(spec, 7100, 1), T, 0)
+    x = (x + 1e-3 * synth.inputs(spec, 7200, T)).astype(np.float32)
+    got = small.forward(x)
+    want = oracle.moe(spec, small.wgate_host, synth.ln2(spec), small.host_mats, x, threads=8)
+    assert np.array_equal(got["topk"], want["topk"])
+    assert np.bincount(got["topk"].ravel()).max() > 16
+    for t in range(T):
+        assert rel_err(got["mlp"][t], want["mlp"][t]) <= SPLIT_TOL, t
+
+
 # ------------------------------------------------------------------ full-size properties
 
 def test_moe_batch_invariance_and_determinism(full_q4):
