@@ -147,20 +147,26 @@ struct PfRing {
     __device__ static int apos(int r, int c) { return c ^ ((r / (16 / PP)) % PP); }
 };
 
-/* One global_load_lds_dwordx4: 16 bytes from src per lane into LDS at lds_dst + 16 * lane
-   (lds_dst the same for the whole wavefront). Written as inline asm: the compiler, which
+/* One global_load_lds_dwordx4: 16 bytes from base + voff per lane into LDS at byte lds + 16 * lane
+   (base and lds the same for the whole wavefront). Written as inline asm: the compiler, which
    cannot tell the ring's slots apart, would otherwise wait for every such load in flight
    before each LDS read. The waits are the caller's (wait_vm_lgkm), and the memory clobber
    keeps the compiler's own LDS accesses on their side of it. */
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"     /* m0 is written on purpose */
-__device__ static inline void lds_dma16(const void *src, const void *lds_dst) {
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(
-        (uint32_t)(uintptr_t)(const void __attribute__((address_space(3))) *)lds_dst);
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                 :: "v"(src), "s"(m0) : "memory", "m0");
+__device__ static inline void lds_dma16(const uint8_t *base, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop
+
+/* a pointer that is the same in every lane, in scalar registers */
+__device__ static inline const uint8_t *uniform_ptr(const void *p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v),
+                   hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (const uint8_t *)((uint64_t)hi << 32 | lo);
+}
 
 /* s_waitcnt vmcnt(N) lgkmcnt(0) (gfx9 encoding; expcnt left at its maximum) */
 template <int N> __device__ static inline void wait_vm_lgkm() {
@@ -203,33 +209,44 @@ __device__ static inline half8_t weight_q(uint2 pw, int g) {
    UP: the lo plane is 2^11 times larger (split_f16_up), and is multiplied by q * 2^-11, exact
    in f16: four more instructions per B tile and block. */
 template <class R, int NMT, bool UP = false>
-__device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *const (&asrc_h)[R::KB],
-                               const _Float16 *const (&asrc_l)[R::KB],
-                               const uint8_t *wsrc, size_t wstep, const uint8_t *ssrc,
-                               f32x4_t (*acc)[R::TT]) {
+__device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _Float16 *xl,
+                               const uint32_t (&aoff)[R::KB], const uint8_t *wsrc,
+                               const uint8_t *ssrc, f32x4_t (*acc)[R::TT]) {
     static_assert(NMT <= R::TT, "token tiles");
     constexpr int ENC = R::ENCODING;
     constexpr int KB = R::KB;
     const int l = threadIdx.x & 63, g = l >> 4;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   /* wavefront-uniform */
-    auto issue = [&](int st) {
-        uint8_t *slot = ring + (st % R::P) * R::STAGE;
-        st = min(st, S - 1);            /* past the end: a valid stage into a free slot */
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+        (uint32_t)(uintptr_t)(const void __attribute__((address_space(3))) *)ring);
+    /* the next stage to load: its sources (scalar pointers; a lane's part is a 32-bit offset) and
+       its slot. Past the end: the last stage again, into a free slot. */
+    const uint8_t *ph = uniform_ptr(xh), *pl = uniform_ptr(xl), *pw = uniform_ptr(wsrc),
+                  *ps = uniform_ptr(ssrc);
+    int left = S - 1;
+    uint32_t put = 0;
+    auto issue = [&]() __attribute__((always_inline)) {
+        const uint32_t dst = lds0 + put;
         if (w < NMT) {                  /* empty token tiles are not loaded */
 #pragma unroll
             for (int i = 0; i < KB; i++) {
-                lds_dma16(asrc_h[i] + st * 32 * KB, slot + 1024 * (KB * w + i));
-                lds_dma16(asrc_l[i] + st * 32 * KB, slot + R::A_BYTES + 1024 * (KB * w + i));
+                lds_dma16(ph, aoff[i], dst + 1024 * (KB * w + i));
+                lds_dma16(pl, aoff[i], dst + R::A_BYTES + 1024 * (KB * w + i));
             }
         }
 #pragma unroll
         for (int i = 0; i < R::WI; i++)
             if (R::WB >= 1024 * (i + 1) || l * 16 < R::WB - 1024 * i)
-                lds_dma16(wsrc + (size_t)st * wstep + 1024 * i + 16 * l,
-                          slot + 2 * R::A_BYTES + w * R::WB + 1024 * i);
+                lds_dma16(pw, 1024 * i + 16 * l, dst + 2 * R::A_BYTES + w * R::WB + 1024 * i);
         if (l * 16 < R::SB)
-            lds_dma16(ssrc + (size_t)st * 128 * KB + 16 * l,
-                      slot + 2 * R::A_BYTES + R::W_BYTES + w * R::SB);
+            lds_dma16(ps, 16 * l, dst + 2 * R::A_BYTES + R::W_BYTES + w * R::SB);
+        const uint32_t on = left > 0;
+        left--;
+        ph += on * (64 * KB);
+        pl += on * (64 * KB);
+        pw += on * (KB * 64 * R::PB);
+        ps += on * (128 * KB);
+        put = put + R::STAGE == R::P * R::STAGE ? 0 : put + R::STAGE;
     };
     /* this lane's B rows: segment and row within it, per tile */
     int boff[R::NBT], soff[R::NBT];
@@ -253,7 +270,8 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *const (&asr
 #pragma unroll
             for (int mt = 0; mt < NMT; mt++) tot[n][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    for (int st = 0; st < R::P - 1; st++) issue(st);
+    for (int st = 0; st < R::P - 1; st++) issue();
+    uint32_t get = 0;
     for (int s = 0; s < S; s++) {
         if constexpr (PARTS) {
             if (s % PF_SUM == 0)
@@ -272,8 +290,9 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *const (&asr
         else wait_vm_lgkm<(R::Q - 2 * KB) * (R::P - 2)>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        issue(s + R::P - 1);
-        const uint8_t *slot = ring + (s % R::P) * R::STAGE;
+        issue();
+        const uint8_t *slot = ring + get;
+        get = get + R::STAGE == R::P * R::STAGE ? 0 : get + R::STAGE;
         const _Float16 *ah = (const _Float16 *)slot, *al = (const _Float16 *)(slot + R::A_BYTES);
         const uint8_t *wl = slot + 2 * R::A_BYTES;
         const uint16_t *sl = (const uint16_t *)(wl + R::W_BYTES);
@@ -437,13 +456,11 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
        scale bytes of the stage */
     /* A load i of the wavefront fills rows 16w + i * 64/PP .. (PP lanes per row): this lane's
        row and the logical piece that belongs at its position */
-    const _Float16 *ash[R::KB], *asl[R::KB];
+    uint32_t aoff[R::KB];            /* bytes (T K F halves are far below 2^32 of them) */
 #pragma unroll
     for (int i = 0; i < R::KB; i++) {
         const int ar = 16 * w + i * (64 / R::PP) + l / R::PP;
-        const size_t ao = (size_t)arow[ar] * n_in + 8 * R::apos(ar, l % R::PP);
-        ash[i] = xh + ao;
-        asl[i] = xl + ao;
+        aoff[i] = 2 * ((uint32_t)arow[ar] * n_in + 8 * R::apos(ar, l % R::PP));
     }
     const uint8_t *M0 = experts + (size_t)e * exp_stride + mat0;
     const int wseg = w * R::WB / (R::KB * 64 * R::PB), wofs = w * R::WB % (R::KB * 64 * R::PB);
@@ -459,16 +476,15 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
 #pragma unroll
         for (int mt = 0; mt < TT; mt++)
             for (int i = 0; i < 4; i++) acc[n][mt][i] = 0.0f;
-    const size_t wstep = (size_t)R::KB * 64 * R::PB;
     const int S = nb / R::KB;
     if constexpr (TT == 1) {
-        pf_loop<R, 1>(ring, S, ash, asl, wsrc, wstep, ssrc, acc);
+        pf_loop<R, 1>(ring, S, xh, xl, aoff, wsrc, ssrc, acc);
     } else {
         switch (nmt) {
-        case 1: pf_loop<R, 1>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
-        case 2: pf_loop<R, 2>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
-        case 3: pf_loop<R, 3>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
-        default: pf_loop<R, 4>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
+        case 1: pf_loop<R, 1>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
+        case 2: pf_loop<R, 2>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
+        case 3: pf_loop<R, 3>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
+        default: pf_loop<R, 4>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
         }
     }
     if constexpr (GU) {
@@ -535,14 +551,13 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, g = l >> 4;
     const int m0 = blockIdx.y * ct, m = min(ct, T - m0), nmt = (m + 15) / 16;
     const int r0 = blockIdx.x * RW, nb = n_in / 32, b0 = blockIdx.z * nbs;
-    const _Float16 *ash[KB], *asl[KB];
+    uint32_t aoff[KB];
 #pragma unroll
     for (int i = 0; i < KB; i++) {
         const int ar = 16 * w + i * (64 / R::PP) + l / R::PP;
-        const size_t ao = (size_t)(m0 + min(ar, m - 1)) * n_in + 32 * b0 + 8 * R::apos(ar, l % R::PP);
-        ash[i] = xh + ao;
-        asl[i] = xl + ao;
+        aoff[i] = 2 * ((uint32_t)min(ar, m - 1) * n_in + 8 * R::apos(ar, l % R::PP));
     }
+    const size_t a0 = (size_t)m0 * n_in + 32 * b0;
     const int wseg = w * R::WB / (KB * 64 * R::PB), wofs = w * R::WB % (KB * 64 * R::PB);
     const int sseg = w * R::SB / (KB * 128), sofs = w * R::SB % (KB * 128);
     const uint8_t *wsrc = W + ((size_t)((r0 >> 6) + wseg) * nb + b0) * 64 * R::PB + wofs;
@@ -553,19 +568,18 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
 #pragma unroll
         for (int mt = 0; mt < TT; mt++)
             for (int i = 0; i < 4; i++) acc[n][mt][i] = 0.0f;
-    const size_t wstep = (size_t)KB * 64 * R::PB;
     const int S = nbs / KB;
     if constexpr (TT == 1) {
-        pf_loop<R, 1, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc);
+        pf_loop<R, 1, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc);
     } else if constexpr (TT == 2) {
-        if (nmt == 1) pf_loop<R, 1, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc);
-        else pf_loop<R, 2, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc);
+        if (nmt == 1) pf_loop<R, 1, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc);
+        else pf_loop<R, 2, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc);
     } else {
         switch (nmt) {
-        case 1: pf_loop<R, 1, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
-        case 2: pf_loop<R, 2, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
-        case 3: pf_loop<R, 3, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
-        default: pf_loop<R, 4, true>(ring, S, ash, asl, wsrc, wstep, ssrc, acc); break;
+        case 1: pf_loop<R, 1, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc); break;
+        case 2: pf_loop<R, 2, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc); break;
+        case 3: pf_loop<R, 3, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc); break;
+        default: pf_loop<R, 4, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc); break;
         }
     }
     float *o = out + ((size_t)blockIdx.z * T + m0) * n_out + r0 + RW / 4 * w + (l & 15);
