@@ -151,6 +151,33 @@ __device__ static inline void split_hilo8(float4 v0, float4 v1, half8_t &h, half
     }
 }
 
+/* One global_load_lds_dwordx4: 16 bytes from base + voff per lane into LDS at byte lds + 16 * lane
+   (base and lds the same for the whole wavefront). Written as inline asm: the compiler, which
+   cannot tell the ring's slots apart, would otherwise wait for every such load in flight
+   before each LDS read. The waits are the caller's (wait_vm_lgkm), and the memory clobber
+   keeps the compiler's own LDS accesses on their side of it. */
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"     /* m0 is written on purpose */
+__device__ static inline void lds_dma16(const uint8_t *base, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+/* a pointer that is the same in every lane, in scalar registers */
+__device__ static inline const uint8_t *uniform_ptr(const void *p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v),
+                   hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (const uint8_t *)((uint64_t)hi << 32 | lo);
+}
+
+/* s_waitcnt vmcnt(N) lgkmcnt(0) (gfx9 encoding; expcnt left at its maximum) */
+template <int N> __device__ static inline void wait_vm_lgkm() {
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
+}
+
 #define PF_CHUNK 64         /* prefill: tokens per chunk of an expert group (4 MFMA tiles) */
 
 /* One wavefront, all 64 lanes: the prefill chunk list, the (group, first token m0) of every

@@ -29,9 +29,9 @@
  * matrices for one chunk (gate/up: 128 rows of Wg and the same rows of Wu, so SwiGLU pairs
  * are in one lane; down: 128 rows of Wd), each wavefront 32 rows for every non-empty token
  * tile of 16 (a chunk of 20 tokens costs 2 tiles, not 4). Calls whose experts have few tokens
- * (cpg_prefill_chunk) take chunks of one token tile and use a variant with 64 gate/up rows per workgroup and a ring of four
- * stages: there the VALU weight conversion, not the MFMAs, sets each wavefront's pace, and
- * twice the workgroups spread it over the CUs. The activations are split into
+ * (cpg_prefill_chunk) take chunks of one token tile and use variants with 64 gate/up rows per
+ * workgroup (PF_FEW_PAIRS): there the VALU weight conversion, not the MFMAs, sets each
+ * wavefront's pace, and twice the workgroups spread it over the CUs. The activations are split into
  * hi/lo f16 planes once per call (k_split_hilo for xn; the gate/up epilogue writes h split).
  * Both operands reach the MFMAs through a ring of stages in LDS filled by direct
  * global-to-LDS loads (k_pf_gemm; k_dense for the dense projections).
@@ -39,6 +39,7 @@
 #include "cpg_internal.h"
 #include "cpg_gemv.h"
 #include "cpg_mfma.h"
+#include <type_traits>
 
 /* ---------------------------------------------------------------- chunk list */
 
@@ -96,26 +97,36 @@ __global__ __launch_bounds__(256) void k_split_hilo(const float *__restrict__ x,
    Every wavefront issues the same number Q of loads per stage, so "stage s has landed" is
    vmcnt <= Q * (P - 2) for each wavefront, followed by a barrier for the others' loads. The
    barrier is s_barrier alone: __syncthreads() would wait for every load in flight. The
-   workgroup (4 wavefronts) computes 128 rows of each of its matrices for the chunk; a
-   wavefront 32 rows of each (GU: gate rows, up rows: four 16-row B tiles; down: two). */
+   workgroup (4 wavefronts) computes RW rows of each of its matrices for the chunk; a
+   wavefront RW/4 rows of each (RW 128, GU: gate rows, up rows: four 16-row B tiles; down: two).
+   KG > 1 (one token tile): KG groups of four wavefronts, each taking KB / KG blocks of every
+   stage for all the rows; group 0 adds the groups' sums in order at the end. */
 #define PF_NT 256
-/* chunks of one token tile: ring depth, rows of each matrix per workgroup (gate/up,
-   down), blocks per stage; measured at 16 tokens (gate/up, down us): 128 rows in rings of 4
-   38.4, 16.6; 64 rows 29.3, 20.1; 64 rows in rings of 6 30.9, 22.4; stages of 4 blocks in
-   rings of 3 28.3 (gate/up, against 28.0 with stages of 2), in rings of 4 32.7 */
-#define PF_SMALL_RING 4
+/* chunks of one token tile: rows of each matrix per workgroup (gate/up, down; measured at 16 tokens
+   with rings of 4, gate/up, down us: 128 rows 38.4, 16.6; 64 rows 29.3, 20.1). Up to PF_FEW_PAIRS
+   pairs there are at most a few workgroups per CU and the length of each one's chain of stages
+   counts: eight wavefronts in two groups, each taking half the blocks of a stage of four, in a ring
+   of two; above, four wavefronts, stages of two blocks and a ring of three (us per layer with the
+   routing, in that order: 2 tokens Q4_0 33.6, 40.2; 4 tokens 42.3, 45.4, Q8_0 48.1, 48.8; 8 tokens
+   56.3, 56.8; 16 tokens skewed 56.9, 57.9, Q8_0 78.3, 76.0; 45 tokens 121.8, 122.7 and 160.9, 158.2;
+   a ring of four in place of three: 16 tokens 60.5, 78.9, 45 tokens 122.9, 162.1; four groups and
+   stages of eight: 4 tokens 41.2, Q8_0 61.5, 8 tokens 61.1) */
 #define PF_SMALL_RW_GU 64
 #define PF_SMALL_RW_DN 128
-#define PF_SMALL_KB 2
+#define PF_FEW_PAIRS 64
 #define PF_SUM 4            /* pf_loop: stages whose sums are taken together, one token tile */
 #define R_Q_FITS(q, p) ((q) * ((p) - 2) < 64)   /* the stage wait's vmcnt fits its field */
 
-template <int ENC, bool GU, int TT_ = PF_CHUNK / 16, int P_ = 2, int RW_ = 128, int KB_ = 2>
+template <int ENC, bool GU, int TT_ = PF_CHUNK / 16, int P_ = 2, int RW_ = 128, int KB_ = 2, int KG_ = 1>
 struct PfRing {
     static constexpr int ENCODING = ENC;
     static constexpr bool GATE_UP = GU;
     static constexpr int TT = TT_;                            /* token tiles of 16 at most */
     static constexpr int KB = KB_;                            /* blocks of 32 per stage */
+    static constexpr int KG = KG_;                            /* groups of 4 wavefronts */
+    static constexpr int NT = 256 * KG_;                      /* threads */
+    static constexpr int KBW = KB_ / KG_;                     /* blocks of a stage per group */
+    static constexpr int AI = KG_ == 1 ? KB_ : 1;             /* A loads of each plane per wave */
     static constexpr int PB = ENC == CPG_ENC_Q4 ? 16 : 32;   /* payload bytes per row-block */
     static constexpr int RW = RW_;                            /* rows of each matrix */
     static constexpr int TPM = RW / 64;                       /* B tiles per matrix per wave */
@@ -126,53 +137,27 @@ struct PfRing {
     static constexpr int W_BYTES = NSEG * KB * 64 * PB;
     static constexpr int S_BYTES = NSEG * KB * 128;
     static constexpr int STAGE = 2 * A_BYTES + W_BYTES + S_BYTES;
-    static constexpr int WB = W_BYTES / 4;                    /* weight bytes per wavefront */
+    static constexpr int WB = W_BYTES / (4 * KG);             /* weight bytes per wavefront */
     static constexpr int WI = (WB + 1023) / 1024;             /* their loads */
-    static constexpr int SB = S_BYTES / 4;                    /* scale bytes per wavefront */
-    static constexpr int Q = 2 * KB + WI + 1;                 /* loads per stage per wavefront */
+    static constexpr int SB = S_BYTES / (4 * KG);             /* scale bytes per wavefront */
+    static constexpr int QA = KG == 1 ? 2 * KB : 1;           /* A loads per stage per wavefront */
+    static constexpr int Q = QA + WI + 1;                     /* loads per stage per wavefront */
     /* ring depth: chunks of up to 64 tokens (TT = 4) use 2, the next stage loading while
        this one is computed. Stages of two blocks with two slots (37-52 KiB) let three
        workgroups share a CU (the register limit) and halve the barriers of one-block stages;
        measured: gate/up 134 us with one-block stages in three slots, 144 with two-block
        stages in three slots (two workgroups per CU), 125 with two in two; deeper rings were
        slower still, as fewer workgroups then hide each other's barriers and LDS latency.
-       Chunks of one token tile (batches of up to 16 tokens) compute little per stage and
-       wait for its loads: their ring is deeper (pf_small_ring). */
+       Chunks of one token tile: PF_FEW_PAIRS. */
     static constexpr int P = P_;
     static_assert(RW % 64 == 0 && P >= 2 && WB % 16 == 0 && SB % 16 == 0 && SB <= 1024 && PP <= 16 &&
-                      TT >= 1 && TT <= PF_CHUNK / 16 && R_Q_FITS(2 * KB + WI + 1, P),
+                      TT >= 1 && TT <= PF_CHUNK / 16 && R_Q_FITS(2 * KB + WI + 1, P) &&
+                      KB % KG == 0 && (KG == 1 || (TT == 1 && 2 * KB == 4 * KG)),
                   "ring geometry");
     /* the position of logical piece c of A row r: rows 16 * 4 / PP apart share banks, so the
        16 rows of an MFMA operand read land in distinct banks */
     __device__ static int apos(int r, int c) { return c ^ ((r / (16 / PP)) % PP); }
 };
-
-/* One global_load_lds_dwordx4: 16 bytes from base + voff per lane into LDS at byte lds + 16 * lane
-   (base and lds the same for the whole wavefront). Written as inline asm: the compiler, which
-   cannot tell the ring's slots apart, would otherwise wait for every such load in flight
-   before each LDS read. The waits are the caller's (wait_vm_lgkm), and the memory clobber
-   keeps the compiler's own LDS accesses on their side of it. */
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"     /* m0 is written on purpose */
-__device__ static inline void lds_dma16(const uint8_t *base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :: "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-/* a pointer that is the same in every lane, in scalar registers */
-__device__ static inline const uint8_t *uniform_ptr(const void *p) {
-    const uint64_t v = (uint64_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v),
-                   hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (const uint8_t *)((uint64_t)hi << 32 | lo);
-}
-
-/* s_waitcnt vmcnt(N) lgkmcnt(0) (gfx9 encoding; expcnt left at its maximum) */
-template <int N> __device__ static inline void wait_vm_lgkm() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
-}
 
 /* One lane's B operand of one block as exact f16 integers q, in natural k order: the nibble
    mask (Q4, after a shift to the lane group's nibbles) or nothing (Q8) leaves each byte u, a
@@ -210,7 +195,7 @@ __device__ static inline half8_t weight_q(uint2 pw, int g) {
    in f16: four more instructions per B tile and block. */
 template <class R, int NMT, bool UP = false>
 __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _Float16 *xl,
-                               const uint32_t (&aoff)[R::KB], const uint8_t *wsrc,
+                               const uint32_t (&aoff)[R::AI], const uint8_t *wsrc,
                                const uint8_t *ssrc, f32x4_t (*acc)[R::TT]) {
     static_assert(NMT <= R::TT, "token tiles");
     constexpr int ENC = R::ENCODING;
@@ -221,13 +206,16 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
         (uint32_t)(uintptr_t)(const void __attribute__((address_space(3))) *)ring);
     /* the next stage to load: its sources (scalar pointers; a lane's part is a 32-bit offset) and
        its slot. Past the end: the last stage again, into a free slot. */
-    const uint8_t *ph = uniform_ptr(xh), *pl = uniform_ptr(xl), *pw = uniform_ptr(wsrc),
+    const int w4 = w & 3, kg = w >> 2;           /* the wavefront of its group, the group */
+    const uint8_t *ph = uniform_ptr(R::KG > 1 && w >= R::KB ? xl : xh), *pl = uniform_ptr(xl), *pw = uniform_ptr(wsrc),
                   *ps = uniform_ptr(ssrc);
     int left = S - 1;
     uint32_t put = 0;
     auto issue = [&]() __attribute__((always_inline)) {
         const uint32_t dst = lds0 + put;
-        if (w < NMT) {                  /* empty token tiles are not loaded */
+        if constexpr (R::KG > 1) {      /* one KiB of one plane per wavefront */
+            lds_dma16(ph, aoff[0], dst + 1024 * w);
+        } else if (w < NMT) {           /* empty token tiles are not loaded */
 #pragma unroll
             for (int i = 0; i < KB; i++) {
                 lds_dma16(ph, aoff[i], dst + 1024 * (KB * w + i));
@@ -254,7 +242,7 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
     for (int n = 0; n < R::NBT; n++) {
         /* tile n: matrix n / TPM (GU: gate, then up), rows RW/4 * w + 16 * (n % TPM) of it;
            the workgroup's RW rows of a matrix are its segments TPM * matrix .. */
-        const int r = R::RW * (n / R::TPM) + R::RW / 4 * w + 16 * (n % R::TPM) + (l & 15);
+        const int r = R::RW * (n / R::TPM) + R::RW / 4 * w4 + 16 * (n % R::TPM) + (l & 15);
         const int seg = r >> 6, rs = r & 63;
         boff[n] = (seg * KB * 64 + rs) * R::PB + (ENC == CPG_ENC_Q4 ? 8 * (g & 1) : 8 * g);
         soff[n] = (seg * KB * 64 + rs) * 2;
@@ -286,8 +274,8 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
         asm volatile("" ::: "memory");
         /* stage s has landed when at most the later stages' loads are in flight: Q per stage
            for a wavefront that loads A tiles, Q - 2 * KB for one that does not */
-        if (w < NMT) wait_vm_lgkm<R::Q * (R::P - 2)>();
-        else wait_vm_lgkm<(R::Q - 2 * KB) * (R::P - 2)>();
+        if (R::KG > 1 || w < NMT) wait_vm_lgkm<R::Q * (R::P - 2)>();
+        else wait_vm_lgkm<(R::Q - R::QA) * (R::P - 2)>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         issue();
@@ -297,7 +285,8 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
         const uint8_t *wl = slot + 2 * R::A_BYTES;
         const uint16_t *sl = (const uint16_t *)(wl + R::W_BYTES);
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
+        for (int kq = 0; kq < R::KBW; kq++) {
+            const int kb = R::KG > 1 ? kg * R::KBW + kq : kq;
             half8_t a_hi[NMT], a_lo[NMT];
 #pragma unroll
             for (int mt = 0; mt < NMT; mt++) {
@@ -340,6 +329,25 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
     /* no load may still write this workgroup's LDS when it ends */
     asm volatile("" ::: "memory");
     wait_vm_lgkm<0>();
+    if constexpr (R::KG > 1) {                   /* the groups' sums: group 0 adds the others in order */
+        float *red = (float *)ring;
+        __syncthreads();                         /* every load has landed, every stage is read */
+        if (kg > 0)
+#pragma unroll
+            for (int n = 0; n < R::NBT; n++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    red[(((kg - 1) * R::NBT + n) * 4 + i) * 256 + 64 * w4 + l] = acc[n][0][i];
+        __syncthreads();
+        if (kg == 0)
+#pragma unroll
+            for (int q = 1; q < R::KG; q++)
+#pragma unroll
+                for (int n = 0; n < R::NBT; n++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        acc[n][0][i] += red[(((q - 1) * R::NBT + n) * 4 + i) * 256 + 64 * w4 + l];
+    }
 }
 
 /* grid (rows / RW, max_chunks), PF_NT threads, dynamic LDS PfRing::P * PfRing::STAGE,
@@ -351,8 +359,8 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
      (row stride n_out) for the pair of each position.
    TT < 4 (a ring for TT token tiles): every chunk holds at most 16 * TT tokens (the host
    guarantees it: batches of at most 16 * TT tokens, as a token's K experts are distinct). */
-template <int ENC, bool GU, int TT = PF_CHUNK / 16, int P = 2, int RW = 128, int KB = 2>
-__global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ? 3 : 1))) void k_pf_gemm(
+template <int ENC, bool GU, int TT = PF_CHUNK / 16, int P = 2, int RW = 128, int KB = 2, int KG = 1>
+__global__ __launch_bounds__(PF_NT *KG) __attribute__((amdgpu_waves_per_eu(TT == 4 ? 3 : 1))) void k_pf_gemm(
     const uint8_t *__restrict__ experts, size_t exp_stride, size_t mat0, size_t mat_bytes,
     size_t payload_plane, int n_in, int n_out, const int *__restrict__ chunk_grp,
     const int *__restrict__ chunk_m0, const int *__restrict__ grp_expert,
@@ -361,7 +369,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
     const _Float16 *__restrict__ xl, _Float16 *__restrict__ hh, _Float16 *__restrict__ hl,
     float *__restrict__ y, const int *__restrict__ sel, int npairs, int K, int E,
     int *__restrict__ ngroups) {
-    using R = PfRing<ENC, GU, TT, P, RW, KB>;
+    using R = PfRing<ENC, GU, TT, P, RW, KB, KG>;
     extern __shared__ __align__(16) uint8_t ring[];
     __shared__ int arow[PF_CHUNK], orow[PF_CHUNK];
     __shared__ uint64_t tab[32];
@@ -370,7 +378,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
        (gridDim.y is a multiple of 8) */
     const int nx = gridDim.x, id = blockIdx.x + nx * blockIdx.y, sidx = id >> 3;
     const int c = 8 * (sidx / nx) + (id & 7);
-    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, g = l >> 4;
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, w4 = w & 3, g = l >> 4;
     const int r0 = (sidx % nx) * RW, nb = n_in / 32;
     int e, m;
     if (TT == 1 && sel) {
@@ -456,10 +464,10 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
        scale bytes of the stage */
     /* A load i of the wavefront fills rows 16w + i * 64/PP .. (PP lanes per row): this lane's
        row and the logical piece that belongs at its position */
-    uint32_t aoff[R::KB];            /* bytes (T K F halves are far below 2^32 of them) */
+    uint32_t aoff[R::AI];            /* bytes (T K F halves are far below 2^32 of them) */
 #pragma unroll
-    for (int i = 0; i < R::KB; i++) {
-        const int ar = 16 * w + i * (64 / R::PP) + l / R::PP;
+    for (int i = 0; i < R::AI; i++) {
+        const int ar = (KG > 1 ? w % KB : 16 / (64 / R::PP) * w + i) * (64 / R::PP) + l / R::PP;
         aoff[i] = 2 * ((uint32_t)arow[ar] * n_in + 8 * R::apos(ar, l % R::PP));
     }
     const uint8_t *M0 = experts + (size_t)e * exp_stride + mat0;
@@ -487,6 +495,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
         default: pf_loop<R, 4>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
         }
     }
+    if (KG > 1 && w >= 4) return;                /* group 0 holds the sums */
     if constexpr (GU) {
 #pragma unroll
         for (int half = 0; half < R::TPM; half++)
@@ -499,7 +508,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
                         const float hv =
                             swiglu_t(acc[half][mt][i], acc[R::TPM + half][mt][i], tab);
                         const f16pair p = split_f16(hv);
-                        const size_t o = (size_t)orow[r] * n_out + r0 + RW / 4 * w +
+                        const size_t o = (size_t)orow[r] * n_out + r0 + RW / 4 * w4 +
                                          16 * half + (l & 15);
                         hh[o] = p.hi;
                         hl[o] = p.lo;
@@ -514,7 +523,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
                 for (int i = 0; i < 4; i++) {
                     const int r = mt * 16 + 4 * g + i;
                     if (r < m)
-                        y[(size_t)orow[r] * n_out + r0 + RW / 4 * w + 16 * n + (l & 15)] =
+                        y[(size_t)orow[r] * n_out + r0 + RW / 4 * w4 + 16 * n + (l & 15)] =
                             acc[n][mt][i];
                 }
     }
@@ -712,19 +721,19 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
     }
     const uint8_t *ex = (const uint8_t *)L->experts;
     const size_t es = cpg_expert_bytes(ENC, D, F), mg = cpg_matrix_bytes(ENC, F, D);
-    auto gemms = [&](auto gu_kernel, size_t ring_gu, int rw_gu, auto dn_kernel, size_t ring_dn,
-                     int rw_dn) {
+    auto gemms = [&](int nt, auto gu_kernel, size_t ring_gu, int rw_gu, auto dn_kernel,
+                     size_t ring_dn, int rw_dn) {
         if (ring_gu > 64 * 1024)
             CPG_HIP(hipFuncSetAttribute((const void *)gu_kernel,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)ring_gu));
         if (ring_dn > 64 * 1024)
             CPG_HIP(hipFuncSetAttribute((const void *)dn_kernel,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)ring_dn));
-        LAUNCH(CPG_KT_GATEUP, gu_kernel, dim3(F / rw_gu, mc), dim3(PF_NT), ring_gu, ex, es,
+        LAUNCH(CPG_KT_GATEUP, gu_kernel, dim3(F / rw_gu, mc), dim3(nt), ring_gu, ex, es,
                (size_t)0, mg, cpg_payload_plane(ENC, F, D), D, F, chunk_grp, chunk_m0,
                grp_expert, grp_off, grp_cnt, list_tok, xh, xl, hh, hl, (float *)nullptr, sel,
                T * K, K, E, ngroups);
-        LAUNCH(CPG_KT_DOWN, dn_kernel, dim3(D / rw_dn, mc), dim3(PF_NT), ring_dn, ex, es, 2 * mg,
+        LAUNCH(CPG_KT_DOWN, dn_kernel, dim3(D / rw_dn, mc), dim3(nt), ring_dn, ex, es, 2 * mg,
                mg, cpg_payload_plane(ENC, D, F), F, D, chunk_grp, chunk_m0, grp_expert, grp_off,
                grp_cnt, list_pair, hh, hl, (_Float16 *)nullptr, (_Float16 *)nullptr, y, sel,
                T * K, K, E, (int *)nullptr);
@@ -732,17 +741,21 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
     };
     int rc;
     if (cpg_prefill_chunk(T, K, E) == 16) {
-        /* chunks of one token tile: a deeper ring */
-        using RG = PfRing<ENC, true, 1, PF_SMALL_RING, PF_SMALL_RW_GU, PF_SMALL_KB>;
-        using RD = PfRing<ENC, false, 1, PF_SMALL_RING, PF_SMALL_RW_DN, PF_SMALL_KB>;
-        rc = gemms(k_pf_gemm<ENC, true, 1, PF_SMALL_RING, PF_SMALL_RW_GU, PF_SMALL_KB>,
-                   (size_t)RG::P * RG::STAGE, RG::RW,
-                   k_pf_gemm<ENC, false, 1, PF_SMALL_RING, PF_SMALL_RW_DN, PF_SMALL_KB>,
-                   (size_t)RD::P * RD::STAGE, RD::RW);
+        /* chunks of one token tile */
+        auto tile = [&](auto few) {
+            constexpr int P = few ? 2 : 3, KB = few ? 4 : 2, KG = few ? 2 : 1;
+            using RG = PfRing<ENC, true, 1, P, PF_SMALL_RW_GU, KB, KG>;
+            using RD = PfRing<ENC, false, 1, P, PF_SMALL_RW_DN, KB, KG>;
+            return gemms(RG::NT, k_pf_gemm<ENC, true, 1, P, PF_SMALL_RW_GU, KB, KG>,
+                         (size_t)RG::P * RG::STAGE, RG::RW,
+                         k_pf_gemm<ENC, false, 1, P, PF_SMALL_RW_DN, KB, KG>,
+                         (size_t)RD::P * RD::STAGE, RD::RW);
+        };
+        rc = T * K <= PF_FEW_PAIRS ? tile(std::true_type{}) : tile(std::false_type{});
     } else {
         using RG = PfRing<ENC, true>;
         using RD = PfRing<ENC, false>;
-        rc = gemms(k_pf_gemm<ENC, true>, (size_t)RG::P * RG::STAGE, RG::RW,
+        rc = gemms(PF_NT, k_pf_gemm<ENC, true>, (size_t)RG::P * RG::STAGE, RG::RW,
                    k_pf_gemm<ENC, false>, (size_t)RD::P * RD::STAGE, RD::RW);
     }
     if (rc) return rc;
