@@ -1547,97 +1547,112 @@ __global__ __launch_bounds__(256) void k_rmsnorm_tok(
     }
 }
 
-#define RL_TOK 16           /* k_router_tok: tokens per workgroup */
-#define RL_ROWS 16          /* router rows per workgroup */
+#define RC_TOK 4            /* k_router_chain: tokens per workgroup */
+#define RC_ROWS 16          /* router rows per workgroup */
+#define RC_KC 128           /* columns per stage */
+#define RC_RING 4           /* stages in LDS: 40 KiB, four workgroups per CU */
+#define RC_C (RC_KC / 16)   /* float4 of a row read at once: a quarter of a stage */
 
-/* step b: grid (ceil(T/16), ceil(E/16)), 256 threads. Thread (i, r) = (tid % 16, tid / 16)
-   runs the chain of token t0+i and router row e0+r: logits[t][e] = the reference's serial
-   chain of separately rounded products (kernels.c:75-95), one chain per lane, so the GPU's
-   lanes together hold all T * E chains. A stage puts KC columns (128, or 64 where D is not a
-   multiple of 128) of the 16 tokens' xn and of the 16 rows in LDS (row stride KC + 4 floats,
-   so the 16 rows a wavefront reads as float4 fall in distinct banks; the 4 lanes of a token
-   and the 16 lanes of a row read the same address). Each thread loads KC/64 float4 of each
-   per stage, two stages ahead into two register sets in a loop unrolled by two with no exit
-   between the halves (a branch there would make the compiler copy registers whose loads are
-   in flight): a stage of 128 columns is long enough to cover the loads' latency, one of 64
-   was not (each stage waited for its loads). A chain's stage is unrolled whole, so its LDS
-   reads issue together and wait once. Tokens and rows past the ends read clamped (valid)
-   addresses and are not stored. */
-template <int KC>
-__global__ __launch_bounds__(256) void k_router_tok(
-    const float *__restrict__ xn, const float *__restrict__ wgate, int T, int D, int E,
-    float *__restrict__ logits) {
-    constexpr int LX = KC + 4, NI = KC / 64;     /* float4 items per thread and array */
-    static_assert(NI == 1 || NI == 2, "stage width");
-    __shared__ __align__(16) float xs[2][RL_TOK * LX];
-    __shared__ __align__(16) float ws[2][RL_ROWS * LX];
-    const int tid = threadIdx.x, i = tid & 15, r = tid >> 4;
-    const int t0 = blockIdx.x * RL_TOK, e0 = blockIdx.y * RL_ROWS;
-    const int nt = min(RL_TOK, T - t0), ne = min(RL_ROWS, E - e0), S = D / KC;
-    /* this thread's stage items q < NI: item tid + 256 q = (row, float4 column) of the
-       16 x KC/4 tile, for xn and for the router rows, named (an array of them would be kept
-       in scratch) */
-#define RK_ITEM(q)                                                                          \
-    const int lr##q = (tid + 256 * (q)) / (KC / 4), lc##q = (tid + 256 * (q)) % (KC / 4);    \
-    const float *xp##q = xn + (size_t)(t0 + min(lr##q, nt - 1)) * D + 4 * lc##q;            \
-    const float *wp##q = wgate + (size_t)(e0 + min(lr##q, ne - 1)) * D + 4 * lc##q;          \
-    const int so##q = lr##q * LX + 4 * lc##q;                                               \
-    float4 ax##q, aw##q, bx##q, bw##q;
-#define RK_EACH(M) { M(0) } if constexpr (NI > 1) { M(1) }
-    RK_ITEM(0)
-    RK_ITEM(1)
-    float acc = 0.0f;
-    auto chain = [&](int b) {
-        const float4 *xr = (const float4 *)(xs[b] + i * LX), *wr = (const float4 *)(ws[b] + r * LX);
+/* step b: logits[t][e] = the reference's serial chain of separately rounded products
+   (kernels.c:75-95), one chain per lane, so that the GPU's lanes together hold all T * E chains;
+   D a multiple of 128. One wavefront per workgroup: grid (ceil(T/4), ceil(E/16)), 64 threads, lane
+   (i, r) = (l / 16, l % 16) the chain of token t0+i and router row e0+r. The
+   16 rows and the 4 tokens' xn stream through a ring of stages of 128 columns in LDS, filled by
+   direct loads (ten of 1 KiB, two rows each; 16-byte piece c of router row r sits at piece
+   c ^ r, so that the 16 rows that a quarter of the wavefront reads fall in distinct banks; its
+   token's piece is one address). A wavefront waits for its own loads only and has no barrier; it
+   reads a quarter of a stage ahead of the additions, and each product is formed three additions
+   before its own, in the slots that the dependent additions leave (in source order each addition
+   waited for its product as well as for the sum).
+   Tokens and rows past the ends read clamped (valid) addresses and are not stored.
+
+   What bounds it: the chain, 2048 dependent additions, and with four workgroups on a CU the LDS
+   reads (two 16-byte reads per lane and four products). Against 16 tokens x 16 rows in a workgroup of
+   four wavefronts, stages through registers and a barrier each, us: 45 tokens 17.8 -> 14.6,
+   160 tokens 18.4 -> 16.0, 512 tokens 20.3 -> 19.9. */
+__global__ __launch_bounds__(64) void k_router_chain(const float *__restrict__ xn,
+                                                     const float *__restrict__ wgate, int T, int D,
+                                                     int E, float *__restrict__ logits) {
+    constexpr int ROWB = RC_KC * 4, STAGE = (RC_ROWS + RC_TOK) * ROWB, NL = STAGE / 1024;
+    static_assert(ROWB == 512 && NL * (RC_RING - 1) < 64, "two rows per load, vmcnt");
+    __shared__ __align__(16) uint8_t ring[RC_RING * STAGE];
+    const int l = threadIdx.x, i = l >> 4, r = l & 15;
+    const int t0 = blockIdx.x * RC_TOK, e0 = blockIdx.y * RC_ROWS, S = D / RC_KC;
+    const uint8_t *pw = uniform_ptr(wgate + (size_t)e0 * D), *px = uniform_ptr(xn + (size_t)t0 * D);
+    uint32_t off[NL];                            /* bytes from the stage's first column */
 #pragma unroll
-        for (int k = 0; k < KC / 4; k++) {
-            const float4 xv = xr[k], wv = wr[k];
-            acc = __fadd_rn(acc, __fmul_rn(wv.x, xv.x));
-            acc = __fadd_rn(acc, __fmul_rn(wv.y, xv.y));
-            acc = __fadd_rn(acc, __fmul_rn(wv.z, xv.z));
-            acc = __fadd_rn(acc, __fmul_rn(wv.w, xv.w));
+    for (int n = 0; n < NL; n++) {
+        const int row = 2 * n + (l >> 5), p = l & 31;
+        off[n] = row < RC_ROWS ? 4 * (uint32_t)min(row, E - 1 - e0) * D + 16 * (p ^ row)
+                               : 4 * (uint32_t)min(row - RC_ROWS, T - 1 - t0) * D + 16 * p;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+        (uint32_t)(uintptr_t)(const void __attribute__((address_space(3))) *)ring);
+    uint32_t put = 0, get = 0;
+    int left = S - 1;
+    auto issue = [&]() __attribute__((always_inline)) {   /* past the end: the last stage again */
+#pragma unroll
+        for (int n = 0; n < NL; n++)
+            lds_dma16(2 * n < RC_ROWS ? pw : px, off[n], lds0 + put + 1024 * n);
+        const uint32_t on = left > 0 ? ROWB : 0;
+        left--;
+        pw += on;
+        px += on;
+        put = put + STAGE == RC_RING * STAGE ? 0 : put + STAGE;
+    };
+    /* chunk c of the stage at ring + at: this lane's RC_C float4 of its router row and token */
+    float4 wa[RC_C], xa[RC_C], wb[RC_C], xb[RC_C];
+    auto read = [&](float4 (&wv)[RC_C], float4 (&xv)[RC_C], uint32_t at, int c)
+        __attribute__((always_inline)) {
+        const uint8_t *wr = ring + at + r * ROWB, *xr = ring + at + (RC_ROWS + i) * ROWB;
+#pragma unroll
+        for (int k = 0; k < RC_C; k++) {
+            wv[k] = *(const float4 *)(wr + 16 * ((RC_C * c + k) ^ r));
+            xv[k] = *(const float4 *)(xr + 16 * (RC_C * c + k));
         }
     };
-#define RK_LOAD(set, q, st)                                                                 \
-    set##x##q = *(const float4 *)(xp##q + min((st), S - 1) * KC);                           \
-    set##w##q = *(const float4 *)(wp##q + min((st), S - 1) * KC);
-#define RK_PUT(set, q, buf)                                                                 \
-    *(float4 *)(xs[buf] + so##q) = set##x##q;                                               \
-    *(float4 *)(ws[buf] + so##q) = set##w##q;
-#define RK_LA0(q) RK_LOAD(a, q, 0)
-#define RK_LB1(q) RK_LOAD(b, q, 1)
-#define RK_LA2(q) RK_LOAD(a, q, 2)
-#define RK_LB3(q) RK_LOAD(b, q, st + 3)
-#define RK_LA4(q) RK_LOAD(a, q, st + 4)
-#define RK_PA0(q) RK_PUT(a, q, 0)
-#define RK_PB1(q) RK_PUT(b, q, 1)
-    RK_EACH(RK_LA0)
-    RK_EACH(RK_LB1)
-    RK_EACH(RK_PA0)
-    RK_EACH(RK_LA2)
-    __syncthreads();
-    for (int st = 0; st < S; st += 2) {
-        chain(0);                                /* stage st in buffer 0 */
-        RK_EACH(RK_PB1)                          /* stage st + 1 */
-        RK_EACH(RK_LB3)
-        __syncthreads();
-        if (st + 1 < S) chain(1);                /* stage st + 1 in buffer 1 */
-        RK_EACH(RK_PA0)                          /* stage st + 2 */
-        RK_EACH(RK_LA4)
-        __syncthreads();
+    float acc = 0.0f;
+    auto chain = [&](const float4 (&wv)[RC_C], const float4 (&xv)[RC_C]) __attribute__((always_inline)) {
+        float p0 = __fmul_rn(wv[0].x, xv[0].x), p1 = __fmul_rn(wv[0].y, xv[0].y),
+              p2 = __fmul_rn(wv[0].z, xv[0].z), p3 = __fmul_rn(wv[0].w, xv[0].w);
+#pragma unroll
+        for (int k = 1; k < RC_C; k++)
+            asm volatile("v_add_f32 %0, %0, %1\n\tv_mul_f32 %1, %5, %9\n\t"
+                         "v_add_f32 %0, %0, %2\n\tv_mul_f32 %2, %6, %10\n\t"
+                         "v_add_f32 %0, %0, %3\n\tv_mul_f32 %3, %7, %11\n\t"
+                         "v_add_f32 %0, %0, %4\n\tv_mul_f32 %4, %8, %12"
+                         : "+&v"(acc), "+&v"(p0), "+&v"(p1), "+&v"(p2), "+&v"(p3)
+                         : "v"(wv[k].x), "v"(wv[k].y), "v"(wv[k].z), "v"(wv[k].w), "v"(xv[k].x),
+                           "v"(xv[k].y), "v"(xv[k].z), "v"(xv[k].w));
+        acc = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(acc, p0), p1), p2), p3);
+    };
+    auto next = [&](uint32_t at) { return at + STAGE == RC_RING * STAGE ? 0 : at + STAGE; };
+    for (int st = 0; st < RC_RING - 1; st++) issue();
+    wait_vm_lgkm<NL * (RC_RING - 2)>();
+    asm volatile("" ::: "memory");
+    read(wa, xa, 0, 0);
+    for (int s = 0; s < S; s++) {
+        /* every read of stage s - 1 has been used: its slot is free */
+        issue();
+        read(wb, xb, get, 1);
+        asm volatile("" ::: "memory");           /* the reads stay ahead of the chain */
+        chain(wa, xa);
+        read(wa, xa, get, 2);
+        asm volatile("" ::: "memory");
+        chain(wb, xb);
+        read(wb, xb, get, 3);
+        asm volatile("" ::: "memory");
+        chain(wa, xa);
+        get = next(get);
+        wait_vm_lgkm<NL * (RC_RING - 2)>();      /* stage s + 1 has landed */
+        asm volatile("" ::: "memory");
+        read(wa, xa, get, 0);
+        asm volatile("" ::: "memory");
+        chain(wb, xb);
     }
-#undef RK_ITEM
-#undef RK_EACH
-#undef RK_LOAD
-#undef RK_PUT
-#undef RK_LA0
-#undef RK_LB1
-#undef RK_LA2
-#undef RK_LB3
-#undef RK_LA4
-#undef RK_PA0
-#undef RK_PB1
-    if (i < nt && r < ne) logits[(size_t)(t0 + i) * E + e0 + r] = acc;
+    asm volatile("" ::: "memory");
+    wait_vm_lgkm<0>();                           /* no load may still write this LDS */
+    if (t0 + i < T && e0 + r < E) logits[(size_t)(t0 + i) * E + e0 + r] = acc;
 }
 
 /* grid T, 64 threads: softmax and top-K of one token */
@@ -2914,7 +2929,7 @@ static int moe_forward(const cpg_moe_layer *L, const float *x, const float *attn
                wt_d, ws->pair_pos, ws->list_tok, ws->list_pair, ws->grp_expert, ws->grp_off,
                ws->grp_cnt, ws->n_groups);
     } else {
-        if (D % 64) { cpg_set_error("routing of %d tokens needs D %% 64 == 0", T); return -1; }
+        if (D % RC_KC) { cpg_set_error("routing of %d tokens needs D %% %d == 0", T, RC_KC); return -1; }
         if (D % 4 || D > 4 * 256 * RN_V4) {
             cpg_set_error("routing of %d tokens needs D %% 4 == 0 and D <= %d", T, 4 * 256 * RN_V4);
             return -1;
@@ -2924,13 +2939,9 @@ static int moe_forward(const cpg_moe_layer *L, const float *x, const float *attn
         _Float16 *xh = mfma ? (_Float16 *)ws->gu : nullptr;
         LAUNCH(CPG_KT_ROUTE, k_rmsnorm_tok, dim3(T), dim3(256), sizeof(float) * (size_t)D, x,
                attn, L->ln2, D, L->eps, xn_d, xh, xh ? xh + (size_t)T * D : nullptr);
-        const dim3 rgrid((T + RL_TOK - 1) / RL_TOK, (E + RL_ROWS - 1) / RL_ROWS);
-        if (D % 128 == 0)
-            LAUNCH(CPG_KT_ROUTE, k_router_tok<128>, rgrid, dim3(256), 0, xn_d, L->wgate, T, D, E,
-                   lg_d);
-        else
-            LAUNCH(CPG_KT_ROUTE, k_router_tok<64>, rgrid, dim3(256), 0, xn_d, L->wgate, T, D, E,
-                   lg_d);
+        LAUNCH(CPG_KT_ROUTE, k_router_chain,
+               dim3((T + RC_TOK - 1) / RC_TOK, (E + RC_ROWS - 1) / RC_ROWS), dim3(64), 0, xn_d,
+               L->wgate, T, D, E, lg_d);
         LAUNCH(CPG_KT_SELECT, k_select, dim3(T), dim3(64), 0, lg_d, E, K, tk_d, wt_d);
         LAUNCH(CPG_KT_SELECT, k_bucket, dim3(1), dim3(1024), 0, tk_d, T, K, E, ws->pair_pos,
                ws->list_tok, ws->list_pair, ws->grp_expert, ws->grp_off, ws->grp_cnt,
