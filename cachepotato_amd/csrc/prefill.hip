@@ -771,7 +771,10 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
 /* The dense product's launch for T tokens: blocks of 32 per stage (two where the row has an
    even number), token tiles of 16 and chunks (a workgroup's tokens, spread evenly: 96 tokens are
    two chunks of 48, not 64 and 32), and the split of the k range, doubled while every part keeps
-   at least 8 blocks and the grid stays within 1024 workgroups. */
+   at least 8 blocks and the grid stays within 1024 workgroups (640 with 128 and more blocks per row,
+   whose many parts cost more where they are summed than their shorter loops give: output
+   projection and sum of its parts at 96 tokens 13.0 + 5.3 -> 10.6 + 3.9 us with 8 parts for 16, 512
+   tokens 28.4 + 5.1 and 28.8 + 4.9 with 2 for 4; q|k|v at 96 tokens 13.2 with 4 parts, 14.6 with 2). */
 struct dense_geo {
     int kb, tt, tpc, chunks, ks;                 /* tt: the kernel's tiles; tpc: a chunk's */
 };
@@ -786,7 +789,7 @@ static dense_geo dense_geometry(int T, int n_in, int n_out) {
     const int base = n_out / DENSE_RW * d.chunks;
     d.ks = 1;
     while (d.ks < 16 && nb % (2 * d.ks * d.kb) == 0 && nb / (2 * d.ks) >= 8 &&
-           base * 2 * d.ks <= 1024)
+           base * 2 * d.ks <= (nb >= 128 ? 640 : 1024))
         d.ks *= 2;
     return d;
 }
