@@ -676,14 +676,15 @@ static int max_chunks(int T, int K, int E, int ch) {
     return (n + 7) / 8 * 8;                      /* k_pf_gemm places chunk c on XCD c % 8 */
 }
 
-/* Tokens per chunk of T tokens with K experts each: one tile of 16 while the experts have 8 tokens
-   each on average, so that nearly every expert is one chunk: the one-tile GEMMs' deeper ring and
-   smaller workgroups then keep more of the weights in flight (us per layer with the routing,
-   chunks of 64 and of 16: 45 tokens Q4_0 122.7, 120.7, Q8_0 skewed 148.3, 135.0; 96 tokens 125.9,
-   126.1 and 170.8, 161.2). Above, an expert's second chunk reads its weights again: 160 tokens
-   132.7, 134.2 and 187.2, 185.6; 256 tokens Q4_0 154, 170. */
+/* Tokens per chunk of T tokens with K experts each: one tile of 16 while the experts have at most 11
+   tokens each on average, so that most experts are one chunk: the one-tile GEMMs' smaller
+   workgroups then keep more of the weights in flight (us per layer with the routing, chunks of 64 and
+   of 16, 128 experts top-8: 45 tokens Q4_0 122.7, 120.7, Q8_0 skewed 148.3, 135.0; 96 tokens 125.9,
+   126.1 and 170.8, 161.2; 144 tokens Q8_0 184.5, 173.0; 160 tokens Q8_0 184.9, 179.3, skewed 181.1,
+   182.8, Q4_0 skewed 138.8, 137.5). Above, the second chunks of crowded experts read their weights
+   again: 192 tokens 188.5, 184.4, skewed 185.2, 195.5, Q4_0 133.5, 134.8; 256 tokens 142, 155. */
 int cpg_prefill_chunk(int T, int K, int E) {
-    return T <= 16 || T * K <= 8 * E ? 16 : PF_CHUNK;
+    return T <= 16 || T * K <= 11 * E ? 16 : PF_CHUNK;
 }
 
 /* the most chunks T tokens with K experts each over E experts can form */

@@ -602,11 +602,11 @@ def test_moe_small_certified_batch_invariance(small, T):
     assert rel_err(got["mlp"], gemv["mlp"]) <= SPLIT_TOL
 
 
-@pytest.mark.parametrize("T", [17, 32, 33])
+@pytest.mark.parametrize("T", [17, 32, 44, 45])
 def test_moe_small_crowded_experts_vs_oracle(cpg, oracle, small, T):
     """Every token takes the same experts, so each has T tokens: chunks of 16 (17 = one row past a
-    chunk, 32 = the last call with them at 16 experts) and chunks of 64 (33), against the
-    oracle."""
+    chunk, 32 = two whole ones, 44 = the last call with them at 16 experts, top-4) and a chunk of
+    64 (45), against the oracle."""
     from cachepotato_amd import synth
     spec = small.spec
     x = np.repeat(synth.inputs(spec, 7100, 1), T, 0)
