@@ -106,11 +106,14 @@ __global__ __launch_bounds__(256) void k_split_hilo(const float *__restrict__ x,
    with rings of 4, gate/up, down us: 128 rows 38.4, 16.6; 64 rows 29.3, 20.1). Up to PF_FEW_PAIRS
    pairs there are at most a few workgroups per CU and the length of each one's chain of stages
    counts: eight wavefronts in two groups, each taking half the blocks of a stage of four, in a ring
-   of two; above, four wavefronts, stages of two blocks and a ring of three (us per layer with the
-   routing, in that order: 2 tokens Q4_0 33.6, 40.2; 4 tokens 42.3, 45.4, Q8_0 48.1, 48.8; 8 tokens
-   56.3, 56.8; 16 tokens skewed 56.9, 57.9, Q8_0 78.3, 76.0; 45 tokens 121.8, 122.7 and 160.9, 158.2;
-   a ring of four in place of three: 16 tokens 60.5, 78.9, 45 tokens 122.9, 162.1; four groups and
-   stages of eight: 4 tokens 41.2, Q8_0 61.5, 8 tokens 61.1) */
+   of two (us per layer with the routing, against four wavefronts and a ring of three: 2 tokens Q4_0
+   33.6, 40.2; 4 tokens 42.3, 45.4, Q8_0 48.1, 48.8; 8 tokens 56.3, 56.8; four groups and stages of
+   eight: 4 tokens 41.2, Q8_0 61.5). Above, four wavefronts and stages of two blocks. There a ring of
+   two lets eight workgroups share a CU, where the weight conversion (Q4_0 with many experts) or
+   nothing but latency (Q8_0 with few) sets the pace; a ring of three keeps more in flight where the
+   loads do. Rings of two and three: up to 2 PF_FEW_PAIRS Q4_0 10 tokens 60.0, 58.7, 16 skewed 58.4,
+   58.4; Q8_0 73.5, 76.6 and 69.2, 75.5; more pairs Q4_0 20 tokens 97.9, 102.3, 45 tokens 110.8, 118.3,
+   96 tokens 116.3, 122.7, 160 tokens 132.0, 129.6; Q8_0 45 tokens 166.7, 155.0, 96 skewed 164.7, 156.8 */
 #define PF_SMALL_RW_GU 64
 #define PF_SMALL_RW_DN 128
 #define PF_FEW_PAIRS 64
@@ -743,8 +746,8 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
     int rc;
     if (cpg_prefill_chunk(T, K, E) == 16) {
         /* chunks of one token tile */
-        auto tile = [&](auto few) {
-            constexpr int P = few ? 2 : 3, KB = few ? 4 : 2, KG = few ? 2 : 1;
+        auto tile = [&](auto groups, auto ring) {
+            constexpr int KG = groups, P = ring, KB = 2 * KG;
             using RG = PfRing<ENC, true, 1, P, PF_SMALL_RW_GU, KB, KG>;
             using RD = PfRing<ENC, false, 1, P, PF_SMALL_RW_DN, KB, KG>;
             return gemms(RG::NT, k_pf_gemm<ENC, true, 1, P, PF_SMALL_RW_GU, KB, KG>,
@@ -752,7 +755,13 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
                          k_pf_gemm<ENC, false, 1, P, PF_SMALL_RW_DN, KB, KG>,
                          (size_t)RD::P * RD::STAGE, RD::RW);
         };
-        rc = T * K <= PF_FEW_PAIRS ? tile(std::true_type{}) : tile(std::false_type{});
+        using std::integral_constant;
+        if (T * K <= PF_FEW_PAIRS)
+            rc = tile(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+        else if ((ENC == CPG_ENC_Q4) == (T * K > 2 * PF_FEW_PAIRS))
+            rc = tile(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+        else
+            rc = tile(integral_constant<int, 1>{}, integral_constant<int, 3>{});
     } else {
         using RG = PfRing<ENC, true>;
         using RD = PfRing<ENC, false>;
