@@ -1319,9 +1319,14 @@ __global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ qk
         }
         return;
     }
-    const int n = pos + 1, tiles = (n + AP - 1) / AP, tps = (tiles + ASPLIT_NS - 1) / ASPLIT_NS;
-    const int ns = (tiles + tps - 1) / tps, j0 = sp * tps * AP;
+    const int n = pos + 1, tiles = (n + AP - 1) / AP;
+    int tps = 1, ns = tiles;
+    if (tiles > ASPLIT_NS) {                     /* no division ahead of the loads of a short context */
+        tps = (tiles + ASPLIT_NS - 1) / ASPLIT_NS;
+        ns = (tiles + tps - 1) / tps;
+    }
     if (sp >= ns) return;
+    const int j0 = sp * tps * AP;
     const int jend = min(n, j0 + tps * AP), kvw = KV * AHD, half = AHD / 2;
     const bool has_new = pos < jend;             /* this split (the last) holds the new row */
     /* ---- every load first */
