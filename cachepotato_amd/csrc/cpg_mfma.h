@@ -164,12 +164,17 @@ __device__ static inline void lds_dma16(const uint8_t *base, uint32_t voff, uint
 }
 #pragma clang diagnostic pop
 
-/* a pointer that is the same in every lane, in scalar registers */
+/* a pointer that is the same in every lane, in scalar registers. A vector memory instruction may
+   read a scalar register five wait states after a v_readfirstlane wrote it; the compiler keeps
+   that distance for its own loads only, not for those of inline assembly (lds_dma16), so it is
+   kept here. */
 __device__ static inline const uint8_t *uniform_ptr(const void *p) {
     const uint64_t v = (uint64_t)p;
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v),
                    hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (const uint8_t *)((uint64_t)hi << 32 | lo);
+    uint64_t u = (uint64_t)hi << 32 | lo;
+    asm("s_nop 4" : "+s"(u));
+    return (const uint8_t *)u;
 }
 
 /* s_waitcnt vmcnt(N) lgkmcnt(0) (gfx9 encoding; expcnt left at its maximum) */
