@@ -22,6 +22,15 @@ def oracle():
 
 
 @pytest.fixture(scope="session")
+def reference_built():
+    """Skips the tests that need the reference engine where it is not built (oracle/Makefile builds
+    it where the reference's sources are)."""
+    from oracle.bindings import REF_SO
+    if not os.path.exists(REF_SO):
+        pytest.skip("oracle/_ref/libref.so is not built")
+
+
+@pytest.fixture(scope="session")
 def cpg():
     """The product library, initialised on GPU 0 (gpu tests only)."""
     import cachepotato_amd as C

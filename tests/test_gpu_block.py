@@ -33,7 +33,7 @@ def model_file(tmp_path_factory):
 
 
 @pytest.fixture(scope="module")
-def ref_lib():
+def ref_lib(reference_built):
     from oracle.bindings import REF_SO, Reference
     Reference(threads=1)        # start the reference pool (scalar Q4 numerics)
     return Q.bind(ctypes.CDLL(REF_SO), extra=False)

@@ -86,7 +86,7 @@ def compare(got, want):
         assert [g[k] for k in keys] == [w[k] for k in keys]
 
 
-def test_chat_turns_match_reference(cpg, tok_dir):
+def test_chat_turns_match_reference(cpg, tok_dir, reference_built):
     from oracle.refrun import spawn_chat
     fd, path = model_fd("chat")
     try:
@@ -132,7 +132,7 @@ def patch_im_end_row(fd, path, X, D):
     os.pwrite(fd, int(crc).to_bytes(8, "little"), hdr["off_r"] + 4 + 43 * ri + 35)
 
 
-def test_chat_stops_at_im_end(cpg, tok_dir):
+def test_chat_stops_at_im_end(cpg, tok_dir, reference_built):
     """A turn ends at <|im_end|>, which is neither handed to the callback nor fed back, and the
     next turn continues after it. The synthetic weights never produce it, so its head row is
     made to win: a copy of the row of the token greedy decoding emits 10 steps in, its scales

@@ -45,7 +45,7 @@ def memfd_model(cfg, name):
 
 
 @pytest.fixture(scope="module")
-def reference():
+def reference(reference_built):
     from oracle.bindings import Reference
     return Reference(threads=1)      # scalar Q4 numerics (kernels.c:524-539)
 
@@ -109,7 +109,7 @@ def test_qwen3_shaped_two_layers_greedy_tokens(cpg, reference, encs):
     assert same == 64 and agree >= 0.98
 
 
-def test_qwen3_30b_a3b_full_model_greedy_tokens(cpg):
+def test_qwen3_30b_a3b_full_model_greedy_tokens(cpg, reference_built):
     """The whole random-init Qwen3-30B-A3B-shaped model (48 layers, the full geometry, Q4_0
     experts and attention, Q8_0 embedding and head; 17.5 GB in HBM): a 128-token prompt of
     seeded ids, then 256 greedy steps through the public API with the graph-replayed step,

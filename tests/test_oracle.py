@@ -20,7 +20,7 @@ needs_ref = pytest.mark.skipif(not HAVE_REF, reason="oracle/_ref/libref.so not b
 
 
 @pytest.fixture(scope="module")
-def ref():
+def ref(reference_built):
     from oracle.bindings import Reference
     return Reference(threads=8)
 
