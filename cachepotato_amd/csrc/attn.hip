@@ -20,9 +20,9 @@
  *                    reference's serial loops (fp32, ~1e-7 to 1e-6 relative).
  *   k_gemv           attn = Wo . ao.
  * From DENSE_MIN_T tokens on, both projections run as MFMA GEMMs instead (k_dense and
- * k_sum_parts of prefill.hip): k_rmsnorm_rows_hilo writes ln1's output as the hi + lo f16
+ * k_sum_parts of prefill.hip): k_rmsnorm_rows_planes writes ln1's output as the
  * planes of the q|k|v product, k_qk_norm_rope adds that product's k parts as it reads them,
- * and the attention core writes the planes of the Wo product; exact f16 weight integers, fp32
+ * and the attention core writes the planes of the Wo product; exact weight integers, fp32
  * accumulation with the block scale applied in fp32, the k range split into parts summed in a
  * fixed order. The projections accumulate in fp32 in a different order than the CPU GEMVs
  * (within ~1e-6 relative), which is what separates this path from the reference's bits.
@@ -68,12 +68,12 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float *__restrict__ 
     }
 }
 
-/* the same rows as k_rmsnorm_rows, written as the hi/lo f16 planes of the dense MFMA
-   product (split_f16_up: hi = f16(v), lo = f16((v - hi) 2^11)) instead of fp32 */
-__global__ __launch_bounds__(256) void k_rmsnorm_rows_hilo(const float *__restrict__ x,
-                                                           const float *__restrict__ g, int D,
-                                                           float eps, _Float16 *__restrict__ hi,
-                                                           _Float16 *__restrict__ lo) {
+/* the same rows as k_rmsnorm_rows, written as the planes of the dense MFMA product instead of
+   fp32 */
+template <int FMT>
+__global__ __launch_bounds__(256) void k_rmsnorm_rows_planes(const float *__restrict__ x,
+                                                             const float *__restrict__ g, int D,
+                                                             float eps, cpg_planes pl) {
     __shared__ double part[4];
     const int t = blockIdx.x, tid = threadIdx.x;
     const float inv = rms_inv_row(x + (size_t)t * D, D, eps, part);
@@ -83,16 +83,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows_hilo(const float *__restri
         const float4 v = x4[i], gv = g4[i];
         const float o[4] = {__fmul_rn(__fmul_rn(v.x, inv), gv.x), __fmul_rn(__fmul_rn(v.y, inv), gv.y),
                             __fmul_rn(__fmul_rn(v.z, inv), gv.z), __fmul_rn(__fmul_rn(v.w, inv), gv.w)};
-        typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-        half4_t h, l;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const f16pair p = split_f16_up(o[j]);
-            h[j] = p.hi;
-            l[j] = p.lo;
-        }
-        *(half4_t *)(hi + (size_t)t * D + 4 * i) = h;
-        *(half4_t *)(lo + (size_t)t * D + 4 * i) = l;
+        planes_put<FMT>(pl, (size_t)t * D + 4 * i, o);
     }
 }
 
@@ -544,8 +535,8 @@ __device__ static inline float half_sum(float v) {
        is key 4g + j for j < 4 and 16 + 4g + j - 4 after), B = value rows read in that key
        order from LDS, where a value tile is laid out as [key / 4][dim][key % 4] so that a
        lane's four consecutive keys of one dimension are one 8-byte read.
-   ns == 1: out = O / l, written as ao (fp32) or, aoh not null, as the hi/lo planes of the
-   output projection. ns > 1: split z's O, M and l are left in pacc / pml at row (z*T + t)*H + h
+   ns == 1: out = O / l, written as ao (fp32; FMT CPG_PL_NONE) or as the planes pl of the output
+   projection. ns > 1: split z's O, M and l are left in pacc / pml at row (z*T + t)*H + h
    for k_attn_merge. The sums run in another order than the reference's two-pass softmax
    (qwen3_moe.c:127-157) and the products carry 22-bit operands, so the output agrees to
    rounding. Dynamic LDS: amma_lds_bytes().
@@ -632,12 +623,12 @@ __device__ __forceinline__ static void amma_store(const float4 (&kv)[4], const f
     }
 }
 
-template <int QS>
+template <int QS, int FMT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_mma(
     const float *__restrict__ q, const float *__restrict__ kc, const float *__restrict__ vc, int H,
     int KV, int T, int pos0_arg, const int *__restrict__ pos_dev, int lim,
     int ns, float *__restrict__ pacc, float2 *__restrict__ pml, float *__restrict__ ao,
-    _Float16 *__restrict__ aoh, _Float16 *__restrict__ aol) {
+    cpg_planes pl) {
     constexpr int HD = 128;
     extern __shared__ __align__(16) _Float16 smh[];   /* two tile buffers (amma_store) */
     const int tid = threadIdx.x, l = tid & 63, g = l >> 4, c = l & 15;
@@ -649,10 +640,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const int tl = min(T, t0 + TB) - 1;          /* the last token of the block */
     auto put = [&](int t, int h, int d, float v) {
         const size_t e = ((size_t)t * H + h) * HD + d;
-        if (aoh) {
-            const f16pair p = split_f16_up(v);
-            aoh[e] = p.hi;
-            aol[e] = p.lo;
+        if constexpr (FMT != CPG_PL_NONE) {
+            const float one[1] = {v};
+            planes_put<FMT>(pl, e, one);
         } else {
             ao[e] = v;
         }
@@ -849,11 +839,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 /* grid ceil(T * H / 8), 256 threads: row (t, h) of k_attn_mma's ns splits (the same H, KV, T,
    position, lim and TB) merged by 32 threads, a float4 of the head each: with M the largest
    M_z, w_z = exp2(M_z - M) and L = sum_z w_z l_z, out = (sum_z w_z O_z) / L, splits in order.
-   Written as ao or, aoh not null, as hi/lo planes; NaN for a block past the cache. */
+   Written as ao (FMT CPG_PL_NONE) or as planes; NaN for a block past the cache. */
+template <int FMT>
 __global__ __launch_bounds__(256) void k_attn_merge(
     const float *__restrict__ pacc, const float2 *__restrict__ pml, int H, int T, int TB, int ns,
-    int pos0_arg, const int *__restrict__ pos_dev, int lim, float *__restrict__ ao,
-    _Float16 *__restrict__ aoh, _Float16 *__restrict__ aol) {
+    int pos0_arg, const int *__restrict__ pos_dev, int lim, float *__restrict__ ao, cpg_planes pl) {
     const int row = blockIdx.x * 8 + (threadIdx.x >> 5), l32 = threadIdx.x & 31;
     if (row >= T * H) return;
     const int t0 = row / H / TB * TB;
@@ -887,10 +877,9 @@ __global__ __launch_bounds__(256) void k_attn_merge(
     }
     a = make_float4(__fdiv_rn(a.x, L), __fdiv_rn(a.y, L), __fdiv_rn(a.z, L), __fdiv_rn(a.w, L));
     const size_t e = (size_t)row * 128 + 4 * l32;
-    if (aoh) {
-        const f16pair2 p = split_f16x2_up(a.x, a.y), r = split_f16x2_up(a.z, a.w);
-        *(uint2 *)(aoh + e) = make_uint2(p.hi, r.hi);
-        *(uint2 *)(aol + e) = make_uint2(p.lo, r.lo);
+    if constexpr (FMT != CPG_PL_NONE) {
+        const float o[4] = {a.x, a.y, a.z, a.w};
+        planes_put<FMT>(pl, e, o);
     } else {
         *(float4 *)(ao + e) = a;
     }
@@ -918,8 +907,7 @@ __global__ __launch_bounds__(256) void k_attn_blk(const float *__restrict__ q,
                                                   int HD, int T, int pos0_arg,
                                                   const int *__restrict__ pos_dev, int lim,
                                                   float *__restrict__ ao,
-                                                  _Float16 *__restrict__ aoh,
-                                                  _Float16 *__restrict__ aol) {
+                                                  cpg_planes pl) {
     constexpr int RS = R / 16, DPT = 128 * R / 256 / 4;   /* float4 of values per thread (HD 128) */
     extern __shared__ __align__(16) float sm[];
     const int LQ = HD + 4;
@@ -1046,18 +1034,11 @@ __global__ __launch_bounds__(256) void k_attn_blk(const float *__restrict__ q,
             if (4 * (vd + i) < HD) {
                 const float r4[4] = {__fdiv_rn(acc[i].x, l), __fdiv_rn(acc[i].y, l),
                                      __fdiv_rn(acc[i].z, l), __fdiv_rn(acc[i].w, l)};
-                if (aoh) {                       /* the output projection's hi/lo planes */
-                    typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-                    const size_t e = ((size_t)t * H + h) * HD + 4 * (vd + i);
-                    half4_t hv, lv;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const f16pair p = split_f16_up(r4[j]);
-                        hv[j] = p.hi;
-                        lv[j] = p.lo;
-                    }
-                    *(half4_t *)(aoh + e) = hv;
-                    *(half4_t *)(aol + e) = lv;
+                const size_t e = ((size_t)t * H + h) * HD + 4 * (vd + i);
+                if (pl.fmt == CPG_PL_BF16) {     /* the output projection's planes */
+                    planes_put<CPG_PL_BF16>(pl, e, r4);
+                } else if (pl.fmt == CPG_PL_F16UP) {
+                    planes_put<CPG_PL_F16UP>(pl, e, r4);
                 } else {
                     *(float4 *)(o + 4 * (vd + i)) = make_float4(r4[0], r4[1], r4[2], r4[3]);
                 }
@@ -1565,7 +1546,8 @@ struct cpg_attn_ws {
 /* from this many tokens on the q|k|v and output projections run on MFMA (k_dense) instead of
    k_gemv, whose passes of four tokens each convert the whole matrix again. With the norm and the
    sums of the parts, which k_gemv has inside, over 700 positions, Q4_0, us: 2 tokens 17.0 in four
-   launches against 16.2 in two, 3 tokens 17.3 against 21.2, 21 tokens (Q8_0) 21.1 against 96.2 */
+   launches (two planes of f16) against 16.2 in two, 3 tokens 18.3 against 21.2, 21 tokens (Q8_0) 22.4
+   against 96.2 */
 #define DENSE_MIN_T 3
 
 static int g_attn_mode = CPG_ATTN_SPLIT;     /* the per-head kernel where split does not apply */
@@ -1655,8 +1637,7 @@ extern "C" void cpg_attn_ws_destroy(cpg_attn_ws *ws) {
 /* k_attn_mma over the T tokens whose q heads are in ws->q and whose keys are in the cache, and
    k_attn_merge where the keys are split */
 static int launch_attn_mma(const cpg_attn_layer *A, cpg_attn_ws *ws, int T, int pos0,
-                           const int *pos_dev, int lim, float *kc, float *vc, _Float16 *aoh,
-                           _Float16 *aol) {
+                           const int *pos_dev, int lim, float *kc, float *vc, cpg_planes pl) {
     const int H = A->H, KV = A->KV, G = H / KV;
     const int qs = T * G > AMMA_QS1_ROWS ? 2 : 1, TB = 64 * qs / G;
     const int blocks = KV * ((T + TB - 1) / TB);
@@ -1673,19 +1654,23 @@ static int launch_attn_mma(const cpg_attn_layer *A, cpg_attn_ws *ws, int T, int 
     const int tiles = pos_dev ? ns : (pos0 + T + AMT - 1) / AMT;
     if (tiles == 1) ns = 1;
     const size_t sm = amma_lds_bytes();
-    const void *kf = qs == 2 ? (const void *)k_attn_mma<2> : (const void *)k_attn_mma<1>;
-    CPG_HIP(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
+    /* up to 32 tokens (three planes, CPG_PL_BF16) qs is 1: T G <= 32 * 16 */
+    auto kernel = pl.fmt == CPG_PL_BF16  ? k_attn_mma<1, CPG_PL_BF16>
+                  : pl.fmt == CPG_PL_NONE ? (qs == 2 ? k_attn_mma<2, CPG_PL_NONE> : k_attn_mma<1, CPG_PL_NONE>)
+                  : qs == 2               ? k_attn_mma<2, CPG_PL_F16UP>
+                                          : k_attn_mma<1, CPG_PL_F16UP>;
+    auto merge = pl.fmt == CPG_PL_BF16  ? k_attn_merge<CPG_PL_BF16>
+                 : pl.fmt == CPG_PL_NONE ? k_attn_merge<CPG_PL_NONE>
+                                         : k_attn_merge<CPG_PL_F16UP>;
+    if (pl.fmt == CPG_PL_BF16 && qs != 1) { cpg_set_error("k_attn_mma: %d tokens as three planes", T); return -1; }
+    CPG_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
     const dim3 grid(KV, (T + TB - 1) / TB, ns < tiles ? ns : tiles);
-    if (qs == 2)
-        hipLaunchKernelGGL(k_attn_mma<2>, grid, dim3(256), sm, g_cpg.stream, ws->q, kc, vc, H, KV,
-                           T, pos0, pos_dev, lim, ns, ws->pacc, ws->pml, ws->ao, aoh, aol);
-    else
-        hipLaunchKernelGGL(k_attn_mma<1>, grid, dim3(256), sm, g_cpg.stream, ws->q, kc, vc, H, KV,
-                           T, pos0, pos_dev, lim, ns, ws->pacc, ws->pml, ws->ao, aoh, aol);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), sm, g_cpg.stream, ws->q, kc, vc, H, KV, T, pos0,
+                       pos_dev, lim, ns, ws->pacc, ws->pml, ws->ao, pl);
     CPG_LAUNCH_CHECK("k_attn_mma");
     if (ns > 1) {
-        hipLaunchKernelGGL(k_attn_merge, dim3((T * H + 7) / 8), dim3(256), 0, g_cpg.stream,
-                           ws->pacc, ws->pml, H, T, TB, ns, pos0, pos_dev, lim, ws->ao, aoh, aol);
+        hipLaunchKernelGGL(merge, dim3((T * H + 7) / 8), dim3(256), 0, g_cpg.stream,
+                           ws->pacc, ws->pml, H, T, TB, ns, pos0, pos_dev, lim, ws->ao, pl);
         CPG_LAUNCH_CHECK("k_attn_merge");
     }
     return 0;
@@ -1717,16 +1702,17 @@ static int attn_forward(const cpg_attn_layer *A, const float *x, int T, int pos0
     hipStream_t s = g_cpg.stream;
     const bool dense = T >= DENSE_MIN_T && ws->dense;
     int rc;
-    /* dense: ln1 writes the hi/lo planes of the product directly, the q|k|v product's k parts
-       are summed by k_qk_norm_rope as it reads them, and the attention core writes the planes
+    /* dense: ln1 writes the planes of the product directly, the q|k|v product's k parts are
+       summed by k_qk_norm_rope as it reads them, and the attention core writes the planes
        of the output projection's input (the scratch's planes are free again by then) */
     const float *qparts = ws->qkv;
     int qks = 1;
-    _Float16 *ph = (_Float16 *)ws->dense;
     if (dense) {
-        hipLaunchKernelGGL(k_rmsnorm_rows_hilo, dim3(T), dim3(256), 0, s, x, A->ln1, D, A->eps,
-                           ph, ph + (size_t)T * D);
-        CPG_LAUNCH_CHECK("k_rmsnorm_rows_hilo");
+        const cpg_planes pl = cpg_dense_planes(T, D, ws->dense);
+        hipLaunchKernelGGL(pl.fmt == CPG_PL_BF16 ? k_rmsnorm_rows_planes<CPG_PL_BF16>
+                                                 : k_rmsnorm_rows_planes<CPG_PL_F16UP>,
+                           dim3(T), dim3(256), 0, s, x, A->ln1, D, A->eps, pl);
+        CPG_LAUNCH_CHECK("k_rmsnorm_rows_planes");
         rc = cpg_dense_from_planes(A->enc, A->wqkv, D, nqkv, T, ws->dense, ws->qkv, 0, &qparts,
                                    &qks);
     } else {
@@ -1761,9 +1747,10 @@ static int attn_forward(const cpg_attn_layer *A, const float *x, int T, int pos0
                            KV, HD, A->eps, pos0, pos_dev, lim, ws->q, kc, vc, ws->stat);
         CPG_LAUNCH_CHECK("k_qk_norm_rope");
         const int G = H / KV;
-        _Float16 *aoh = dense ? ph : nullptr, *aol = dense ? ph + (size_t)T * H * HD : nullptr;
+        const cpg_planes pl = dense ? cpg_dense_planes(T, H * HD, ws->dense)
+                                    : cpg_planes{nullptr, 0, CPG_PL_NONE};
         if (attn_mma_shape(H, KV, HD) && T >= AMMA_MIN_T) {
-            rc = launch_attn_mma(A, ws, T, pos0, pos_dev, lim, kc, vc, aoh, aol);
+            rc = launch_attn_mma(A, ws, T, pos0, pos_dev, lim, kc, vc, pl);
             if (rc) return rc;
             planes = dense;
         } else if (G <= 32 && 32 % G == 0 && HD <= 128) {
@@ -1777,12 +1764,10 @@ static int attn_forward(const cpg_attn_layer *A, const float *x, int T, int pos0
                 CPG_HIP(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
             if (r16)
                 hipLaunchKernelGGL(k_attn_blk<16>, dim3(KV, (T + TB - 1) / TB), dim3(256), sm, s,
-                                   ws->q, kc, vc, H, KV, HD, T, pos0, pos_dev, lim, ws->ao, aoh,
-                                   aol);
+                                   ws->q, kc, vc, H, KV, HD, T, pos0, pos_dev, lim, ws->ao, pl);
             else
                 hipLaunchKernelGGL(k_attn_blk<32>, dim3(KV, (T + TB - 1) / TB), dim3(256), sm, s,
-                                   ws->q, kc, vc, H, KV, HD, T, pos0, pos_dev, lim, ws->ao, aoh,
-                                   aol);
+                                   ws->q, kc, vc, H, KV, HD, T, pos0, pos_dev, lim, ws->ao, pl);
             CPG_LAUNCH_CHECK("k_attn_blk");
             planes = dense;
         } else {

@@ -86,6 +86,20 @@ hipEvent_t *cpg_timing_pair(int slot);
         CPG_LAUNCH_CHECK(#kern);                                                          \
     } while (0)
 
+/* Activations as the MFMA GEMMs read them: planes of 16-bit pieces, `stride` elements apart, whose
+   products with the exact weight integers are added in fp32 (split_f16, split_f16_up, split_bf16x3
+   of cpg_mfma.h). */
+#define CPG_PL_NONE -1
+#define CPG_PL_F16 0        /* two planes: hi = f16(x), lo = f16(x - hi) */
+#define CPG_PL_F16UP 1      /* two planes: hi = f16(x), lo = f16((x - hi) 2^11) */
+#define CPG_PL_BF16 2       /* three planes of bf16, their sum x itself: fp32's 24 bits and its range */
+struct cpg_planes {
+    uint16_t *p;
+    size_t stride;
+    int fmt;
+};
+__host__ __device__ static inline int cpg_plane_count(int fmt) { return fmt == CPG_PL_BF16 ? 3 : 2; }
+
 /* prefill.hip: the MFMA grouped expert GEMMs for many tokens */
 int cpg_prefill_max_chunks(int T, int K, int E);
 /* the most chunks of any call of up to T tokens, and the tokens per chunk of a call of T */
@@ -96,9 +110,10 @@ bool cpg_prefill_shape_ok(int D, int F);
    prepared: the routing step has written the chunk list (pf_chunk_list) and the planes of
    xn; otherwise they are formed here from grp_cnt and xn. */
 size_t cpg_prefill_scratch_bytes(int T, int D, int K, int F);
-/* prefill.hip: the dense MFMA product from hi/lo planes already at the start of scratch
-   (T rows of n_in halves each, hi then lo as split_f16_up forms them); with sum == 0 and more than one k part the parts
+/* prefill.hip: the dense MFMA product from planes already at the start of scratch
+   (cpg_dense_planes: T rows of n_in each); with sum == 0 and more than one k part the parts
    are left in *parts (ks of them, T * n_out floats each, to be added in order) */
+cpg_planes cpg_dense_planes(int T, int n_in, void *scratch);
 int cpg_dense_from_planes(int enc, const void *w, int n_in, int n_out, int T, void *scratch,
                           float *out, int sum, const float **parts, int *ks);
 /* sel not null (cpg_prefill_sel_ok): the GEMMs take each expert's pairs from the T * K
@@ -111,8 +126,8 @@ int cpg_prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const fl
                         int *chunk_m0, void *scratch, float *y, float *mlp, float *xres,
                         const float *attn, int prepared, const int *sel, int *ngroups);
 /* out (T rows of n_out) = W . x for a row-tiled Q4_0/Q8_0 matrix W on MFMA, the k range split
-   into parts summed in a fixed order; scratch: cpg_dense_scratch_bytes (the hi/lo f16 planes of
-   x and the parts) */
+   into parts summed in a fixed order; scratch: cpg_dense_scratch_bytes (the planes of x and the
+   parts) */
 bool cpg_dense_shape_ok(int n_in, int n_out);
 size_t cpg_dense_scratch_bytes(int T, int n_in, int n_out);
 int cpg_dense_mfma(int enc, const void *w, int n_in, int n_out, const float *x, int T,

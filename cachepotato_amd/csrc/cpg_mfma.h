@@ -5,8 +5,10 @@
  * i = 0..3. The weights are the B operand: a lane's 8 k-slots of one block are 8 exact small
  * integers q (Q4: -8..7, Q8: -127..127) of row l%16, converted to f16 without rounding; the
  * block's fp16 scale is applied in fp32 to the block's product. The activations are the A
- * operand, split x = hi + lo with hi = f16(x) and lo = f16(x - hi) (22 significant bits),
- * both halves multiplied. A Q4 lane group g takes the low (g < 2) or high (g >= 2) nibbles of
+ * operand, split x = hi + lo with hi = f16(x) and lo = f16(x - hi) (22 significant bits from
+ * |x| = 2^-2 on, below that what an absolute 2^-25 leaves; infinite beyond 65504), both halves
+ * multiplied; or, on v_mfma_f32_16x16x32_bf16 (the same layout), in three bf16 pieces (split_bf16x3),
+ * the weights then exact bf16 integers. A Q4 lane group g takes the low (g < 2) or high (g >= 2) nibbles of
  * payload bytes 8(g%2)..8(g%2)+7, which hold elements 8g..8g+7 (byte i holds elements i and
  * i+16); a Q8 lane group takes bytes 8g..8g+7. */
 #ifndef CPG_MFMA_H
@@ -58,10 +60,41 @@ __device__ static inline f16pair split_f16_up(float x) {
     const _Float16 h = (_Float16)x;
     return {h, (_Float16)((x - (float)h) * 0x1p11f)};
 }
-__device__ static inline f16pair2 split_f16x2_up(float x, float y) {
-    const f16pair a = split_f16_up(x), b = split_f16_up(y);
-    return {__builtin_bit_cast(uint32_t, half2_t{a.hi, b.hi}),
-            __builtin_bit_cast(uint32_t, half2_t{a.lo, b.lo})};
+
+/* x in three bf16 pieces a + b + c = x, each the leading 8 bits of what the ones before leave:
+   fp32's 24 significant bits over fp32's range (an infinity is a alone). */
+struct bf16x3 {
+    uint16_t a, b, c;
+};
+__device__ static inline bf16x3 split_bf16x3(float x) {
+    const uint32_t a = __float_as_uint(x) & 0xFFFF0000u;
+    const float r = fabsf(x) == INFINITY ? 0.0f : x - __uint_as_float(a);
+    const uint32_t b = __float_as_uint(r) & 0xFFFF0000u;
+    const float s = r - __uint_as_float(b);
+    return {(uint16_t)(a >> 16), (uint16_t)(b >> 16), (uint16_t)(__float_as_uint(s) >> 16)};
+}
+
+/* N consecutive values (1 or 4) at element e of planes of format FMT */
+template <int FMT, int N>
+__device__ static inline void planes_put(const cpg_planes &pl, size_t e, const float (&v)[N]) {
+    typedef uint16_t words_t __attribute__((ext_vector_type(N)));
+    words_t a, b, c;
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        if (FMT == CPG_PL_BF16) {
+            const bf16x3 s = split_bf16x3(v[j]);
+            a[j] = s.a;
+            b[j] = s.b;
+            c[j] = s.c;
+        } else {
+            const f16pair s = FMT == CPG_PL_F16UP ? split_f16_up(v[j]) : split_f16(v[j]);
+            a[j] = __builtin_bit_cast(uint16_t, s.hi);
+            b[j] = __builtin_bit_cast(uint16_t, s.lo);
+        }
+    }
+    *(words_t *)(pl.p + e) = a;
+    *(words_t *)(pl.p + pl.stride + e) = b;
+    if (FMT == CPG_PL_BF16) *(words_t *)(pl.p + 2 * pl.stride + e) = c;
 }
 
 __device__ static inline half8_t pairs_to_half8(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3,

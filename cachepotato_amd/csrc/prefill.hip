@@ -32,7 +32,7 @@
  * (cpg_prefill_chunk) take chunks of one token tile and use variants with 64 gate/up rows per
  * workgroup (PF_FEW_PAIRS): there the VALU weight conversion, not the MFMAs, sets each
  * wavefront's pace, and twice the workgroups spread it over the CUs. The activations are split into
- * hi/lo f16 planes once per call (k_split_hilo for xn; the gate/up epilogue writes h split).
+ * hi/lo f16 planes once per call (k_split_planes for xn; the gate/up epilogue writes h split).
  * Both operands reach the MFMAs through a ring of stages in LDS filled by direct
  * global-to-LDS loads (k_pf_gemm; k_dense for the dense projections).
  */
@@ -57,26 +57,15 @@ __global__ __launch_bounds__(64) void k_chunks(const int *__restrict__ grp_cnt, 
     pf_chunk_list(cnt, grp, ch, max_chunks, chunk_grp, chunk_m0);
 }
 
-/* grid rows, 256 threads: hi[r] = f16(x[r]), lo[r] = f16(x[r] - hi[r]) for rows of n floats
-   (n % 8 == 0); UP: lo is kept 2^11 times larger, as the dense product takes it (split_f16_up) */
-template <bool UP>
-__global__ __launch_bounds__(256) void k_split_hilo(const float *__restrict__ x, int n,
-                                                    _Float16 *__restrict__ hi,
-                                                    _Float16 *__restrict__ lo) {
+/* grid rows, 256 threads: rows of n floats (n % 4 == 0) as planes */
+template <int FMT>
+__global__ __launch_bounds__(256) void k_split_planes(const float *__restrict__ x, int n,
+                                                      cpg_planes pl) {
     const size_t r = blockIdx.x;
-    for (int c = threadIdx.x; c < n / 8; c += 256) {
-        const float4 v0 = *(const float4 *)(x + r * n + 8 * c);
-        const float4 v1 = *(const float4 *)(x + r * n + 8 * c + 4);
-        const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-        half8_t h, l;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const f16pair p = UP ? split_f16_up(v[j]) : split_f16(v[j]);
-            h[j] = p.hi;
-            l[j] = p.lo;
-        }
-        *(half8_t *)(hi + r * n + 8 * c) = h;
-        *(half8_t *)(lo + r * n + 8 * c) = l;
+    for (int c = threadIdx.x; c < n / 4; c += 256) {
+        const float4 v = *(const float4 *)(x + r * n + 4 * c);
+        const float o[4] = {v.x, v.y, v.z, v.w};
+        planes_put<FMT>(pl, r * n + 4 * c, o);
     }
 }
 
@@ -120,13 +109,16 @@ __global__ __launch_bounds__(256) void k_split_hilo(const float *__restrict__ x,
 #define PF_SUM 4            /* pf_loop: stages whose sums are taken together, one token tile */
 #define R_Q_FITS(q, p) ((q) * ((p) - 2) < 64)   /* the stage wait's vmcnt fits its field */
 
-template <int ENC, bool GU, int TT_ = PF_CHUNK / 16, int P_ = 2, int RW_ = 128, int KB_ = 2, int KG_ = 1>
+template <int ENC, bool GU, int TT_ = PF_CHUNK / 16, int P_ = 2, int RW_ = 128, int KB_ = 2, int KG_ = 1,
+          int FMT_ = CPG_PL_F16>
 struct PfRing {
     static constexpr int ENCODING = ENC;
     static constexpr bool GATE_UP = GU;
     static constexpr int TT = TT_;                            /* token tiles of 16 at most */
     static constexpr int KB = KB_;                            /* blocks of 32 per stage */
     static constexpr int KG = KG_;                            /* groups of 4 wavefronts */
+    static constexpr int FMT = FMT_;                          /* the activations' planes */
+    static constexpr int NA = FMT_ == CPG_PL_BF16 ? 3 : 2;
     static constexpr int NT = 256 * KG_;                      /* threads */
     static constexpr int KBW = KB_ / KG_;                     /* blocks of a stage per group */
     static constexpr int AI = KG_ == 1 ? KB_ : 1;             /* A loads of each plane per wave */
@@ -139,11 +131,11 @@ struct PfRing {
     static constexpr int A_BYTES = TT * 16 * 32 * KB * 2;     /* one activation plane */
     static constexpr int W_BYTES = NSEG * KB * 64 * PB;
     static constexpr int S_BYTES = NSEG * KB * 128;
-    static constexpr int STAGE = 2 * A_BYTES + W_BYTES + S_BYTES;
+    static constexpr int STAGE = NA * A_BYTES + W_BYTES + S_BYTES;
     static constexpr int WB = W_BYTES / (4 * KG);             /* weight bytes per wavefront */
     static constexpr int WI = (WB + 1023) / 1024;             /* their loads */
     static constexpr int SB = S_BYTES / (4 * KG);             /* scale bytes per wavefront */
-    static constexpr int QA = KG == 1 ? 2 * KB : 1;           /* A loads per stage per wavefront */
+    static constexpr int QA = KG == 1 ? NA * KB : 1;          /* A loads per stage per wavefront */
     static constexpr int Q = QA + WI + 1;                     /* loads per stage per wavefront */
     /* ring depth: chunks of up to 64 tokens (TT = 4) use 2, the next stage loading while
        this one is computed. Stages of two blocks with two slots (37-52 KiB) let three
@@ -154,8 +146,8 @@ struct PfRing {
        Chunks of one token tile: PF_FEW_PAIRS. */
     static constexpr int P = P_;
     static_assert(RW % 64 == 0 && P >= 2 && WB % 16 == 0 && SB % 16 == 0 && SB <= 1024 && PP <= 16 &&
-                      TT >= 1 && TT <= PF_CHUNK / 16 && R_Q_FITS(2 * KB + WI + 1, P) &&
-                      KB % KG == 0 && (KG == 1 || (TT == 1 && 2 * KB == 4 * KG)),
+                      TT >= 1 && TT <= PF_CHUNK / 16 && R_Q_FITS(NA * KB + WI + 1, P) &&
+                      KB % KG == 0 && (KG == 1 || (TT == 1 && NA * KB == 4 * KG)),
                   "ring geometry");
     /* the position of logical piece c of A row r: rows 16 * 4 / PP apart share banks, so the
        16 rows of an MFMA operand read land in distinct banks */
@@ -188,16 +180,41 @@ __device__ static inline half8_t weight_q(uint2 pw, int g) {
     return q;
 }
 
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+/* The same weights as exact bf16 integers, Q4's 16 times larger (the caller scales by 2^-4): bytes
+   with their bias turned into a sign (Q4: the nibble in the byte's upper half), converted as
+   signed integers of at most 8 significant bits, whose fp32 upper halves are the bf16 numbers. */
+template <int ENC> __device__ static inline bf16x8_t weight_q_bf16(uint2 pw, int g) {
+    uint32_t src[2] = {pw.x, pw.y};
+    if (ENC == CPG_ENC_Q4) {
+        const int sh = 4 - (g >> 1) * 4;
+        src[0] = (src[0] << sh) & 0xF0F0F0F0u;
+        src[1] = (src[1] << sh) & 0xF0F0F0F0u;
+    }
+    uint4 q;
+    uint32_t *o = (uint32_t *)&q;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t s = src[i >> 1] ^ 0x80808080u;
+        const float x = (float)(int8_t)(s >> (16 * (i & 1))), y = (float)(int8_t)(s >> (16 * (i & 1) + 8));
+        o[i] = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u);
+    }
+    return __builtin_bit_cast(bf16x8_t, q);
+}
+
 /* the k loop of one chunk for NMT token tiles: per block, t = A_hi[mt] . q[n] + A_lo[mt] . q[n]
    (two MFMAs, the second accumulating onto the first) and acc[n][mt] += d[n] * t in fp32,
    blocks in order. Measured against the B operand w = q * d as an exact f16 pair hi + lo
    (three MFMAs accumulating across blocks, 22 instructions per lane to form hi and lo from
    a block's 8 weights, against 12 for q here plus 4 fused multiply-adds per token tile):
    gate/up 112.7 -> 103.5 us, down 60.2 -> 57.6 us at 512 tokens.
-   UP: the lo plane is 2^11 times larger (split_f16_up), and is multiplied by q * 2^-11, exact
-   in f16: four more instructions per B tile and block. */
-template <class R, int NMT, bool UP = false>
-__device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _Float16 *xl,
+   CPG_PL_F16UP: the lo plane is 2^11 times larger, and is multiplied by q * 2^-11, exact in f16:
+   four more instructions per B tile and block. CPG_PL_BF16: the smallest plane's product first
+   (weight_q_bf16).
+   x: the first plane at the chunk's first token and block, the others xs elements apart. */
+template <class R, int NMT>
+__device__ static void pf_loop(uint8_t *ring, int S, const uint16_t *x, size_t xs,
                                const uint32_t (&aoff)[R::AI], const uint8_t *wsrc,
                                const uint8_t *ssrc, f32x4_t (*acc)[R::TT]) {
     static_assert(NMT <= R::TT, "token tiles");
@@ -210,31 +227,32 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
     /* the next stage to load: its sources (scalar pointers; a lane's part is a 32-bit offset) and
        its slot. Past the end: the last stage again, into a free slot. */
     const int w4 = w & 3, kg = w >> 2;           /* the wavefront of its group, the group */
-    const uint8_t *ph = uniform_ptr(R::KG > 1 && w >= R::KB ? xl : xh), *pl = uniform_ptr(xl), *pw = uniform_ptr(wsrc),
-                  *ps = uniform_ptr(ssrc);
+    const uint8_t *pa[R::NA], *pw = uniform_ptr(wsrc), *ps = uniform_ptr(ssrc);
+#pragma unroll
+    for (int p = 0; p < R::NA; p++) pa[p] = uniform_ptr(x + (R::KG > 1 ? w / R::KB : p) * xs);
     int left = S - 1;
     uint32_t put = 0;
     auto issue = [&]() __attribute__((always_inline)) {
         const uint32_t dst = lds0 + put;
         if constexpr (R::KG > 1) {      /* one KiB of one plane per wavefront */
-            lds_dma16(ph, aoff[0], dst + 1024 * w);
+            lds_dma16(pa[0], aoff[0], dst + 1024 * w);
         } else if (w < NMT) {           /* empty token tiles are not loaded */
 #pragma unroll
-            for (int i = 0; i < KB; i++) {
-                lds_dma16(ph, aoff[i], dst + 1024 * (KB * w + i));
-                lds_dma16(pl, aoff[i], dst + R::A_BYTES + 1024 * (KB * w + i));
-            }
+            for (int i = 0; i < KB; i++)
+#pragma unroll
+                for (int p = 0; p < R::NA; p++)
+                    lds_dma16(pa[p], aoff[i], dst + p * R::A_BYTES + 1024 * (KB * w + i));
         }
 #pragma unroll
         for (int i = 0; i < R::WI; i++)
             if (R::WB >= 1024 * (i + 1) || l * 16 < R::WB - 1024 * i)
-                lds_dma16(pw, 1024 * i + 16 * l, dst + 2 * R::A_BYTES + w * R::WB + 1024 * i);
+                lds_dma16(pw, 1024 * i + 16 * l, dst + R::NA * R::A_BYTES + w * R::WB + 1024 * i);
         if (l * 16 < R::SB)
-            lds_dma16(ps, 16 * l, dst + 2 * R::A_BYTES + R::W_BYTES + w * R::SB);
+            lds_dma16(ps, 16 * l, dst + R::NA * R::A_BYTES + R::W_BYTES + w * R::SB);
         const uint32_t on = left > 0;
         left--;
-        ph += on * (64 * KB);
-        pl += on * (64 * KB);
+#pragma unroll
+        for (int p = 0; p < R::NA; p++) pa[p] += on * (64 * KB);
         pw += on * (KB * 64 * R::PB);
         ps += on * (128 * KB);
         put = put + R::STAGE == R::P * R::STAGE ? 0 : put + R::STAGE;
@@ -276,7 +294,7 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
         }
         asm volatile("" ::: "memory");
         /* stage s has landed when at most the later stages' loads are in flight: Q per stage
-           for a wavefront that loads A tiles, Q - 2 * KB for one that does not */
+           for a wavefront that loads A tiles, Q - QA for one that does not */
         if (R::KG > 1 || w < NMT) wait_vm_lgkm<R::Q * (R::P - 2)>();
         else wait_vm_lgkm<(R::Q - R::QA) * (R::P - 2)>();
         __builtin_amdgcn_s_barrier();
@@ -284,38 +302,48 @@ __device__ static void pf_loop(uint8_t *ring, int S, const _Float16 *xh, const _
         issue();
         const uint8_t *slot = ring + get;
         get = get + R::STAGE == R::P * R::STAGE ? 0 : get + R::STAGE;
-        const _Float16 *ah = (const _Float16 *)slot, *al = (const _Float16 *)(slot + R::A_BYTES);
-        const uint8_t *wl = slot + 2 * R::A_BYTES;
+        const uint8_t *wl = slot + R::NA * R::A_BYTES;
         const uint16_t *sl = (const uint16_t *)(wl + R::W_BYTES);
 #pragma unroll
         for (int kq = 0; kq < R::KBW; kq++) {
             const int kb = R::KG > 1 ? kg * R::KBW + kq : kq;
-            half8_t a_hi[NMT], a_lo[NMT];
+            uint4 a[R::NA][NMT];
 #pragma unroll
             for (int mt = 0; mt < NMT; mt++) {
                 const int r = mt * 16 + (l & 15);
-                const int o = r * 32 * KB + 8 * R::apos(r, 4 * kb + g);
-                a_hi[mt] = *(const half8_t *)(ah + o);
-                a_lo[mt] = *(const half8_t *)(al + o);
+                const int o = 2 * (r * 32 * KB + 8 * R::apos(r, 4 * kb + g));
+#pragma unroll
+                for (int p = 0; p < R::NA; p++) a[p][mt] = *(const uint4 *)(slot + p * R::A_BYTES + o);
             }
 #pragma unroll
             for (int n = 0; n < R::NBT; n++) {
                 WRaw r;
                 r.w = *(const uint2 *)(wl + boff[n] + kb * 64 * R::PB);
                 r.d = *(const uint16_t *)((const uint8_t *)sl + soff[n] + kb * 128);
-                const half8_t q = weight_q<ENC>(r.w, g);
-                half8_t ql = q;
-                if (UP) ql *= (_Float16)0x1p-11f;
-                const float d = scale_f32(r.d);
+                float d = scale_f32(r.d);
                 f32x4_t t[NMT];
 #pragma unroll
-                for (int mt = 0; mt < NMT; mt++) {
-                    const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-                    t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_hi[mt], q, z, 0, 0, 0);
-                }
+                for (int mt = 0; mt < NMT; mt++) t[mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (R::FMT == CPG_PL_BF16) {
+                    const bf16x8_t q = weight_q_bf16<ENC>(r.w, g);
+                    if (ENC == CPG_ENC_Q4) d *= 0x1p-4f;
 #pragma unroll
-                for (int mt = 0; mt < NMT; mt++)
-                    t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_lo[mt], ql, t[mt], 0, 0, 0);
+                    for (int p = R::NA - 1; p >= 0; p--)
+#pragma unroll
+                        for (int mt = 0; mt < NMT; mt++)
+                            t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                __builtin_bit_cast(bf16x8_t, a[p][mt]), q, t[mt], 0, 0, 0);
+                } else {
+                    const half8_t q = weight_q<ENC>(r.w, g);
+                    half8_t ql = q;
+                    if (R::FMT == CPG_PL_F16UP) ql *= (_Float16)0x1p-11f;
+#pragma unroll
+                    for (int p = 0; p < R::NA; p++)
+#pragma unroll
+                        for (int mt = 0; mt < NMT; mt++)
+                            t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                __builtin_bit_cast(half8_t, a[p][mt]), p ? ql : q, t[mt], 0, 0, 0);
+                }
 #pragma unroll
                 for (int mt = 0; mt < NMT; mt++)
 #pragma unroll
@@ -489,13 +517,13 @@ __global__ __launch_bounds__(PF_NT *KG) __attribute__((amdgpu_waves_per_eu(TT ==
             for (int i = 0; i < 4; i++) acc[n][mt][i] = 0.0f;
     const int S = nb / R::KB;
     if constexpr (TT == 1) {
-        pf_loop<R, 1>(ring, S, xh, xl, aoff, wsrc, ssrc, acc);
+        pf_loop<R, 1>(ring, S, (const uint16_t *)xh, xl - xh, aoff, wsrc, ssrc, acc);
     } else {
         switch (nmt) {
-        case 1: pf_loop<R, 1>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
-        case 2: pf_loop<R, 2>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
-        case 3: pf_loop<R, 3>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
-        default: pf_loop<R, 4>(ring, S, xh, xl, aoff, wsrc, ssrc, acc); break;
+        case 1: pf_loop<R, 1>(ring, S, (const uint16_t *)xh, xl - xh, aoff, wsrc, ssrc, acc); break;
+        case 2: pf_loop<R, 2>(ring, S, (const uint16_t *)xh, xl - xh, aoff, wsrc, ssrc, acc); break;
+        case 3: pf_loop<R, 3>(ring, S, (const uint16_t *)xh, xl - xh, aoff, wsrc, ssrc, acc); break;
+        default: pf_loop<R, 4>(ring, S, (const uint16_t *)xh, xl - xh, aoff, wsrc, ssrc, acc); break;
         }
     }
     if (KG > 1 && w >= 4) return;                /* group 0 holds the sums */
@@ -536,29 +564,30 @@ __global__ __launch_bounds__(PF_NT *KG) __attribute__((amdgpu_waves_per_eu(TT ==
 
 #define DENSE_RW 64         /* rows per workgroup. Measured at 64, 128 and 256 (q|k|v, output
                                projection with the sums of their parts, us): 512 tokens Q4_0 77.8,
-                               80.1, 87.1; 96 tokens 38, 39, 41; 21 tokens Q8_0 21.9, 22.7, - */
+                               80.1, 87.1; 96 tokens 38, 39, 41; 21 tokens Q8_0, two planes, 21.9, 22.7, - */
 
 /* grid (n_out / DENSE_RW, chunks, ks), PF_NT threads, dynamic LDS PfRing::P * PfRing::STAGE: one
    row-tiled matrix W (n_out rows of n_in) times the ct <= 16 TT tokens from blockIdx.y * ct of
-   the hi/lo planes xh/xl (T rows of n_in, lo 2^11 times larger), over the nbs blocks of 32 from
+   the planes pl of format FMT (T rows of n_in), over the nbs blocks of 32 from
    blockIdx.z * nbs (nbs a multiple of KB); written to out[(blockIdx.z * T + t) * n_out + row],
    one part per blockIdx.z.
 
    The expert GEMMs' k loop over a ring of stages in LDS (pf_loop), each wavefront 16 rows for
-   the chunk's token tiles. Few tokens are bound by the launch and one trip through the ring (up
-   to 32 tokens a ring of four stages, all of a part's loads in flight at once), many by the MFMAs
+   the chunk's token tiles. Few tokens are bound by the launch and one trip through the ring (one
+   token tile a ring of four stages, all of a part's loads in flight at once; two a ring of three,
+   which leaves LDS for three workgroups per CU: 21 tokens q|k|v 8.2 us, with four 10.0), many by the MFMAs
    and the LDS reads of their operands (per block and wavefront 2 token-tile operands for 2 MFMAs).
    Against a k loop through registers (weights two stages ahead, a barrier a block): q|k|v and
    output projection, Q4_0, us: 512 tokens 49.2 + 35.2 -> 36.6 + 26.8, 96 tokens 18.0 + 14.5 ->
-   14.7 + 12.6; and against k_gemv's passes of four tokens: 21 tokens Q8_0 46.8 + 49.4 -> 7.5 +
-   6.3, 4 tokens Q4_0 12.0 + 13.6 -> 6.0 + 5.2. */
-template <int ENC, int TT, int P, int KB>
+   14.7 + 12.6; and against k_gemv's passes of four tokens: 21 tokens Q8_0 46.8 + 49.4 -> 8.3 +
+   6.8, 4 tokens Q4_0 12.0 + 13.6 -> 6.2 + 5.4 (two planes of f16 instead of three of bf16: 7.6 + 6.4
+   and 5.8 + 4.9, without fp32's range). */
+template <int ENC, int TT, int P, int KB, int FMT>
 __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ? 3 : 1))) void k_dense(
     const uint8_t *__restrict__ W, size_t payload_plane, int n_in, int n_out, int T, int ct,
-    int nbs, const _Float16 *__restrict__ xh, const _Float16 *__restrict__ xl,
-    float *__restrict__ out) {
+    int nbs, cpg_planes pl, float *__restrict__ out) {
     constexpr int RW = DENSE_RW;
-    using R = PfRing<ENC, false, TT, P, RW, KB>;
+    using R = PfRing<ENC, false, TT, P, RW, KB, 1, FMT>;
     extern __shared__ __align__(16) uint8_t ring[];
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, g = l >> 4;
     const int m0 = blockIdx.y * ct, m = min(ct, T - m0), nmt = (m + 15) / 16;
@@ -582,16 +611,16 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(TT == 4 ?
             for (int i = 0; i < 4; i++) acc[n][mt][i] = 0.0f;
     const int S = nbs / KB;
     if constexpr (TT == 1) {
-        pf_loop<R, 1, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc);
+        pf_loop<R, 1>(ring, S, pl.p + a0, pl.stride, aoff, wsrc, ssrc, acc);
     } else if constexpr (TT == 2) {
-        if (nmt == 1) pf_loop<R, 1, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc);
-        else pf_loop<R, 2, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc);
+        if (nmt == 1) pf_loop<R, 1>(ring, S, pl.p + a0, pl.stride, aoff, wsrc, ssrc, acc);
+        else pf_loop<R, 2>(ring, S, pl.p + a0, pl.stride, aoff, wsrc, ssrc, acc);
     } else {
         switch (nmt) {
-        case 1: pf_loop<R, 1, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc); break;
-        case 2: pf_loop<R, 2, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc); break;
-        case 3: pf_loop<R, 3, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc); break;
-        default: pf_loop<R, 4, true>(ring, S, xh + a0, xl + a0, aoff, wsrc, ssrc, acc); break;
+        case 1: pf_loop<R, 1>(ring, S, pl.p + a0, pl.stride, aoff, wsrc, ssrc, acc); break;
+        case 2: pf_loop<R, 2>(ring, S, pl.p + a0, pl.stride, aoff, wsrc, ssrc, acc); break;
+        case 3: pf_loop<R, 3>(ring, S, pl.p + a0, pl.stride, aoff, wsrc, ssrc, acc); break;
+        default: pf_loop<R, 4>(ring, S, pl.p + a0, pl.stride, aoff, wsrc, ssrc, acc); break;
         }
     }
     float *o = out + ((size_t)blockIdx.z * T + m0) * n_out + r0 + RW / 4 * w + (l & 15);
@@ -721,7 +750,8 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
         if (!sel)
             LAUNCH(CPG_KT_SELECT, k_chunks, dim3(1), dim3(64), 0, grp_cnt, E,
                    cpg_prefill_chunk(T, K, E), mc, chunk_grp, chunk_m0);
-        LAUNCH(CPG_KT_SELECT, k_split_hilo<false>, dim3(T), dim3(256), 0, xn, D, xh, xl);
+        LAUNCH(CPG_KT_SELECT, k_split_planes<CPG_PL_F16>, dim3(T), dim3(256), 0, xn, D,
+               (cpg_planes{(uint16_t *)xh, (size_t)T * D, CPG_PL_F16}));
     }
     const uint8_t *ex = (const uint8_t *)L->experts;
     const size_t es = cpg_expert_bytes(ENC, D, F), mg = cpg_matrix_bytes(ENC, F, D);
@@ -788,6 +818,15 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
 struct dense_geo {
     int kb, tt, tpc, chunks, ks;                 /* tt: the kernel's tiles; tpc: a chunk's */
 };
+/* Up to 32 tokens the activations keep fp32's bits and range, as in the GEMVs (k_gemv) that fewer
+   tokens take: three planes of bf16. More take two planes of f16. */
+static int dense_format(int T) { return T <= 32 ? CPG_PL_BF16 : CPG_PL_F16UP; }
+static size_t dense_plane_bytes(int T, int n_in) {
+    return cpg_round256((size_t)2 * cpg_plane_count(dense_format(T)) * T * n_in);
+}
+cpg_planes cpg_dense_planes(int T, int n_in, void *scratch) {
+    return {(uint16_t *)scratch, (size_t)T * n_in, dense_format(T)};
+}
 static dense_geo dense_geometry(int T, int n_in, int n_out) {
     const int nb = n_in / 32, tiles = (T + 15) / 16;
     dense_geo d;
@@ -811,23 +850,22 @@ bool cpg_dense_shape_ok(int n_in, int n_out) {
 
 size_t cpg_dense_scratch_bytes(int T, int n_in, int n_out) {
     const int ks = dense_ksplit(T, n_in, n_out);
-    return cpg_round256((size_t)4 * T * n_in) + (ks > 1 ? (size_t)4 * ks * T * n_out : 0);
+    return dense_plane_bytes(T, n_in) + (ks > 1 ? (size_t)4 * ks * T * n_out : 0);
 }
 
-template <int ENC, int TT, int P, int KB> static size_t dense_lds() {
-    using R = PfRing<ENC, false, TT, P, DENSE_RW, KB>;
+template <int ENC, int TT, int P, int KB, int FMT> static size_t dense_lds() {
+    using R = PfRing<ENC, false, TT, P, DENSE_RW, KB, 1, FMT>;
     return (size_t)R::P * R::STAGE;
 }
 
-/* the products from the hi/lo planes already in scratch: out directly (ks == 1) or ks parts
+/* the products from the planes already in scratch: out directly (ks == 1) or ks parts
    of T * n_out floats, left unsummed in *parts when sum is false */
 template <int ENC>
 static int dense_from_planes(const void *w, int n_in, int n_out, int T, void *scratch,
                              float *out, bool sum, const float **parts, int *ks_out) {
     const int ks = dense_ksplit(T, n_in, n_out);
-    const _Float16 *xh = (const _Float16 *)scratch, *xl = xh + (size_t)T * n_in;
-    float *part = ks > 1 ? (float *)((uint8_t *)scratch + cpg_round256((size_t)4 * T * n_in))
-                         : out;
+    const cpg_planes pl = cpg_dense_planes(T, n_in, scratch);
+    float *part = ks > 1 ? (float *)((uint8_t *)scratch + dense_plane_bytes(T, n_in)) : out;
     hipStream_t s = g_cpg.stream;
     const dense_geo d = dense_geometry(T, n_in, n_out);
     auto go = [&](auto kernel, size_t lds) {
@@ -836,16 +874,17 @@ static int dense_from_planes(const void *w, int n_in, int n_out, int T, void *sc
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL(kernel, dim3(n_out / DENSE_RW, d.chunks, ks), dim3(PF_NT), lds, s,
                            (const uint8_t *)w, cpg_payload_plane(ENC, n_out, n_in), n_in, n_out,
-                           T, 16 * d.tpc, n_in / 32 / ks, xh, xl, part);
+                           T, 16 * d.tpc, n_in / 32 / ks, pl, part);
         CPG_LAUNCH_CHECK("k_dense");
         return 0;
     };
-#define DENSE_GO(TT, DEPTH, KB) go(k_dense<ENC, TT, DEPTH, KB>, dense_lds<ENC, TT, DEPTH, KB>())
+#define DENSE_GO(TT, DEPTH, KB, FMT) go(k_dense<ENC, TT, DEPTH, KB, FMT>, dense_lds<ENC, TT, DEPTH, KB, FMT>())
     int rc;
-    if (d.kb == 1) rc = DENSE_GO(4, 2, 1);
-    else if (d.tt == 1) rc = DENSE_GO(1, 4, 2);
-    else if (d.tt == 2) rc = DENSE_GO(2, 4, 2);
-    else rc = DENSE_GO(4, 2, 2);
+    if (pl.fmt == CPG_PL_F16UP)
+        rc = d.kb == 1 ? DENSE_GO(4, 2, 1, CPG_PL_F16UP) : DENSE_GO(4, 2, 2, CPG_PL_F16UP);
+    else if (d.kb == 1) rc = DENSE_GO(4, 2, 1, CPG_PL_BF16);
+    else if (d.tt == 1) rc = DENSE_GO(1, 4, 2, CPG_PL_BF16);
+    else rc = DENSE_GO(2, 3, 2, CPG_PL_BF16);
 #undef DENSE_GO
     if (rc) return rc;
     if (parts) *parts = part;
@@ -862,9 +901,10 @@ static int dense_from_planes(const void *w, int n_in, int n_out, int T, void *sc
 template <int ENC>
 static int dense_mfma(const void *w, int n_in, int n_out, const float *x, int T, void *scratch,
                       float *out) {
-    _Float16 *xh = (_Float16 *)scratch, *xl = xh + (size_t)T * n_in;
-    hipLaunchKernelGGL(k_split_hilo<true>, dim3(T), dim3(256), 0, g_cpg.stream, x, n_in, xh, xl);
-    CPG_LAUNCH_CHECK("k_split_hilo");
+    const cpg_planes pl = cpg_dense_planes(T, n_in, scratch);
+    hipLaunchKernelGGL(pl.fmt == CPG_PL_BF16 ? k_split_planes<CPG_PL_BF16> : k_split_planes<CPG_PL_F16UP>,
+                       dim3(T), dim3(256), 0, g_cpg.stream, x, n_in, pl);
+    CPG_LAUNCH_CHECK("k_split_planes");
     return dense_from_planes<ENC>(w, n_in, n_out, T, scratch, out, true, nullptr, nullptr);
 }
 

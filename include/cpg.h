@@ -217,7 +217,7 @@ int cpg_moe_expert_mode(int mode);
    of at least min(n, CPG_KT_COUNT)), then clears the record. */
 #define CPG_KT_ROUTE 0      /* k_route_fast, k_route_small, k_rmsnorm_tok, k_router_tok */
 #define CPG_KT_SELECT 1     /* k_select_bucket, k_select, k_bucket (exact routing), k_chunks,
-                               k_split_hilo */
+                               k_split_planes */
 #define CPG_KT_GATEUP 2     /* k_gateup1, k_gateup_mm, k_mfma_gateup */
 #define CPG_KT_DOWN 3       /* k_down1, k_down_mm (with the weighted combine), k_mfma_down */
 #define CPG_KT_COMBINE 4    /* k_pair_combine (the prefill path's weighted combine) */

@@ -203,6 +203,41 @@ def test_attn_dense_token_edges_vs_oracle(cpg, oracle, enc, D, T):
         dev.close()
 
 
+@pytest.mark.parametrize("enc,D,T", [(8, 2048, 3), (4, 2048, 21), (8, 2048, 31), (8, 256, 3),
+                                     (4, 256, 31)])
+def test_attn_dense_wide_inputs_vs_oracle(cpg, oracle, enc, D, T):
+    """The projections of 3 to 31 tokens take their inputs over the whole range of fp32: normed
+    inputs beyond f16's largest number 65504, where the gains of one block of 32 are 1e5 and its
+    weights 2^-10 (2048), and attention outputs beyond it (256: head dimension 48, gains of
+    1e6), against the oracle."""
+    from tests.attn_helpers import attn_layer, inputs, DeviceAttn
+    kw = dict(D=2048, H=32, KV=4, HD=128) if D == 2048 else dict(D=D, H=2, KV=1, HD=48)
+    a = attn_layer(enc=enc, **kw)
+    if D == 2048:
+        a["ln1"][:32] *= np.float32(1e5)
+        for m in ("wq", "wk", "wv"):
+            blocks = a[m].reshape(-1, D // 32, 34 if enc == 8 else 18)
+            scale = np.ascontiguousarray(blocks[:, 0, :2]).view(np.float16)
+            blocks[:, 0, :2] = (scale * np.float16(2.0 ** -10)).view(np.uint8)
+    else:
+        a["ln1"] *= np.float32(1e6)
+    cap, kvw = T + 5, a["KV"] * a["HD"]
+    dev = DeviceAttn(a, cap=cap, max_T=T)
+    X = inputs(a["D"], 106, T)
+    kc_o, vc_o = np.zeros((cap, kvw), np.float32), np.zeros((cap, kvw), np.float32)
+    try:
+        got = dev.forward(X, 0)
+        want = oracle.attn(a, X, 0, kc_o, vc_o, threads=8)
+        kc, vc = dev.cache()
+        e = max(rel_err(got[t], want[t]) for t in range(T))
+        say(f"attn wide inputs enc={enc} D={D} T={T}: worst token {e:.2e} k {rel_err(kc, kc_o):.2e}")
+        assert np.abs(vc_o).max() > 65504 if D == 256 else np.abs(vc_o).max() < 65504
+        assert e <= PREFILL_TOL and rel_err(kc, kc_o) <= PREFILL_TOL
+        assert rel_err(vc, vc_o) <= PREFILL_TOL
+    finally:
+        dev.close()
+
+
 def test_attn_device_position_equals_host_position(cpg):
     """cpg_attn_forward_at (position read on the device, as in a replayed graph) computes the
     same bits as cpg_attn_forward at the same positions, cache included; a position whose rows
@@ -279,11 +314,12 @@ def test_attn_decode_long_context_vs_oracle(cpg, oracle, pos, mode):
     assert np.array_equal(kc[:pos].view(np.uint32), kc0[:pos].view(np.uint32))
 
 
-@pytest.mark.parametrize("pos", [511, 512, 4095, 4096, 8191])
+@pytest.mark.parametrize("pos", [511, 512, 4095, 4096, 8191, 8192, 20000, 32767])
 def test_attn_decode_split_groups_vs_oracle(cpg, oracle, pos):
     """The split one-token kernel where its merge changes form: 16 splits (merged at once) and 17
-    (in groups), 128 splits of one tile of 32 and 65 of two, and the last position of the
-    longest context; twice each (the arrival counters are left zero), the position given by
+    (in groups), 128 splits of one tile of 32 and 65 of two, the last position of the longest
+    context a model is opened with, and beyond it several tiles per split: three (257 tiles in 86
+    splits, the last of two), five (the last of one) and eight (the longest cache); twice each (the arrival counters are left zero), the position given by
     the host and read on the device, against the oracle."""
     from tests.attn_helpers import attn_layer, inputs, DeviceAttn
     a = attn_layer(enc=8, D=2048, H=32, KV=4, HD=128)
