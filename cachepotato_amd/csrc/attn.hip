@@ -562,12 +562,10 @@ __device__ static inline float half_sum(float v) {
      with two sets, 61.4 with one; 96 tokens, whole layers with the MoE half, 209 and 207; at
      100 tokens over 2000 positions the two are equal);
    AMMA_WGS: workgroups that the key splits aim at, two per CU (512 tokens over 3584 positions:
-     256 workgroups 238, 512 214, 768 or 1024 224);
-   AMMA_MIN_KEYS: keys per split at least (138 tokens at position 0: 58.7 with 32, 60.0 with
-     64, 65.6 with 128). */
+     256 workgroups 238, 512 214, 768 or 1024 224). A split takes whole tiles, one at least (138
+     tokens at position 0: 58.7 with 32 keys at least, 60.0 with 64, 65.6 with 128). */
 #define AMMA_QS1_ROWS 1024
 #define AMMA_WGS 512
-#define AMMA_MIN_KEYS 32
 
 #define AMMA_BUF (2 * AMT * AMLK + 2 * (AMT / 4) * AMLV)   /* halves of one K/V tile buffer */
 
@@ -1641,10 +1639,9 @@ static int launch_attn_mma(const cpg_attn_layer *A, cpg_attn_ws *ws, int T, int 
     const int H = A->H, KV = A->KV, G = H / KV;
     const int qs = T * G > AMMA_QS1_ROWS ? 2 : 1, TB = 64 * qs / G;
     const int blocks = KV * ((T + TB - 1) / TB);
-    /* the splits are set by the cache's length and not by the position, so that a position
-       given by the host and one read on the device give the same bits */
+    /* the splits are set by the tokens alone, so that the cache's length does not show in the bits,
+       and a position given by the host and one read on the device give the same */
     int ns = AMMA_WGS / blocks;
-    ns = ns < lim / AMMA_MIN_KEYS ? ns : lim / AMMA_MIN_KEYS;
     const size_t cap = ws->mma_rows / ((size_t)T * H);       /* k_attn_merge's partial rows */
     ns = ns < AMMA_MAX_NS ? ns : AMMA_MAX_NS;
     ns = (size_t)ns < cap ? ns : (int)cap;

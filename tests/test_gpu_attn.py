@@ -238,6 +238,28 @@ def test_attn_dense_wide_inputs_vs_oracle(cpg, oracle, enc, D, T):
         dev.close()
 
 
+@pytest.mark.parametrize("T,pos0", [(2, 300), (21, 700), (37, 0)])
+def test_attn_prefill_bits_do_not_depend_on_cache_length(cpg, T, pos0):
+    """The same tokens at the same positions give the same bits in caches of other lengths: as
+    long as the positions, a few rows longer, and much longer."""
+    from tests.attn_helpers import attn_layer, inputs, DeviceAttn
+    a = attn_layer(enc=8, D=2048, H=32, KV=4, HD=128)
+    X = inputs(a["D"], 107, T)
+    kv0 = np.random.default_rng(T).normal(size=(2, pos0, a["KV"] * a["HD"])).astype(np.float32)
+    outs = []
+    for cap in (pos0 + T, pos0 + T + 4, 4096):
+        dev = DeviceAttn(a, cap=cap, max_T=T)
+        try:
+            kc, vc = np.zeros((2, cap, a["KV"] * a["HD"]), np.float32)
+            kc[:pos0], vc[:pos0] = kv0
+            dev.set_cache(kc, vc)
+            outs += [dev.forward(X, pos0), dev.forward_at(X, pos0)]
+        finally:
+            dev.close()
+    for o in outs[1:]:
+        assert np.array_equal(o.view(np.uint32), outs[0].view(np.uint32))
+
+
 def test_attn_device_position_equals_host_position(cpg):
     """cpg_attn_forward_at (position read on the device, as in a replayed graph) computes the
     same bits as cpg_attn_forward at the same positions, cache included; a position whose rows
