@@ -30,7 +30,7 @@
  * are in one lane; down: 128 rows of Wd), each wavefront 32 rows for every non-empty token
  * tile of 16 (a chunk of 20 tokens costs 2 tiles, not 4). Calls whose experts have few tokens
  * (cpg_prefill_chunk) take chunks of one token tile and use variants with 64 gate/up rows per
- * workgroup (PF_FEW_PAIRS): there the VALU weight conversion, not the MFMAs, sets each
+ * workgroup (PF_SMALL_RW_GU): there the VALU weight conversion, not the MFMAs, sets each
  * wavefront's pace, and twice the workgroups spread it over the CUs. The activations are split into
  * hi/lo f16 planes once per call (k_split_planes for xn; the gate/up epilogue writes h split).
  * Both operands reach the MFMAs through a ring of stages in LDS filled by direct
@@ -89,7 +89,9 @@ __global__ __launch_bounds__(256) void k_split_planes(const float *__restrict__ 
    workgroup (4 wavefronts) computes RW rows of each of its matrices for the chunk; a
    wavefront RW/4 rows of each (RW 128, GU: gate rows, up rows: four 16-row B tiles; down: two).
    KG > 1 (one token tile): KG groups of four wavefronts, each taking KB / KG blocks of every
-   stage for all the rows; group 0 adds the groups' sums in order at the end. */
+   stage for all the rows; group 0 adds the groups' sums in order at the end. SUMS = 2 gives one
+   group's sums the order of two groups: stages of the blocks that group 0 and group 1 would take
+   in turn, into a sum each (an even number of stages). */
 #define PF_NT 256
 /* chunks of one token tile: rows of each matrix per workgroup (gate/up, down; measured at 16 tokens
    with rings of 4, gate/up, down us: 128 rows 38.4, 16.6; 64 rows 29.3, 20.1). Up to PF_FEW_PAIRS
@@ -97,20 +99,26 @@ __global__ __launch_bounds__(256) void k_split_planes(const float *__restrict__ 
    counts: eight wavefronts in two groups, each taking half the blocks of a stage of four, in a ring
    of two (us per layer with the routing, against four wavefronts and a ring of three: 2 tokens Q4_0
    33.6, 40.2; 4 tokens 42.3, 45.4, Q8_0 48.1, 48.8; 8 tokens 56.3, 56.8; four groups and stages of
-   eight: 4 tokens 41.2, Q8_0 61.5). Above, four wavefronts and stages of two blocks. There a ring of
-   two lets eight workgroups share a CU, where the weight conversion (Q4_0 with many experts) or
-   nothing but latency (Q8_0 with few) sets the pace; a ring of three keeps more in flight where the
-   loads do. Rings of two and three: up to 2 PF_FEW_PAIRS Q4_0 10 tokens 60.0, 58.7, 16 skewed 58.4,
-   58.4; Q8_0 73.5, 76.6 and 69.2, 75.5; more pairs Q4_0 20 tokens 97.9, 102.3, 45 tokens 110.8, 118.3,
-   96 tokens 116.3, 122.7, 160 tokens 132.0, 129.6; Q8_0 45 tokens 166.7, 155.0, 96 skewed 164.7, 156.8 */
+   eight: 4 tokens 41.2, Q8_0 61.5). More pairs: four wavefronts and stages of two blocks. There a
+   ring of two lets eight workgroups share a CU, where the weight conversion (Q4_0 with many experts)
+   or nothing but latency (Q8_0 with few) sets the pace; a ring of three keeps more in flight where
+   the loads do.
+   Up to 16 tokens the one group sums in the order of two (SUMS = 2), so that a token's bits are the
+   same in every batch of 2 to 16; its 78 registers leave six workgroups per CU, as many as the LDS
+   of a ring of three does (Q4_0), or of two (Q8_0). Ring of two, three, with one sum: Q4_0 10
+   tokens 60.0, 58.7, 16 skewed 58.4, 58.4; Q8_0 73.5, 76.6 and 69.2, 75.5; with two sums, as
+   chosen, Q4_0 60.6 and 58.3, Q8_0 74.2 and 69.7.
+   From 17 tokens, rings of two and three: Q4_0 20 tokens 101, 103, 45 tokens 117, 121, 96 tokens
+   120, 126, 160 tokens 138, 134; Q8_0 45 tokens 167, 155, 96 skewed 165, 156 */
 #define PF_SMALL_RW_GU 64
 #define PF_SMALL_RW_DN 128
 #define PF_FEW_PAIRS 64
+#define PF_RING_PAIRS 128
 #define PF_SUM 4            /* pf_loop: stages whose sums are taken together, one token tile */
 #define R_Q_FITS(q, p) ((q) * ((p) - 2) < 64)   /* the stage wait's vmcnt fits its field */
 
 template <int ENC, bool GU, int TT_ = PF_CHUNK / 16, int P_ = 2, int RW_ = 128, int KB_ = 2, int KG_ = 1,
-          int FMT_ = CPG_PL_F16>
+          int FMT_ = CPG_PL_F16, int SUMS_ = 1>
 struct PfRing {
     static constexpr int ENCODING = ENC;
     static constexpr bool GATE_UP = GU;
@@ -119,6 +127,7 @@ struct PfRing {
     static constexpr int KG = KG_;                            /* groups of 4 wavefronts */
     static constexpr int FMT = FMT_;                          /* the activations' planes */
     static constexpr int NA = FMT_ == CPG_PL_BF16 ? 3 : 2;
+    static constexpr int SUMS = SUMS_;                        /* sums, a stage in turn each */
     static constexpr int NT = 256 * KG_;                      /* threads */
     static constexpr int KBW = KB_ / KG_;                     /* blocks of a stage per group */
     static constexpr int AI = KG_ == 1 ? KB_ : 1;             /* A loads of each plane per wave */
@@ -143,11 +152,12 @@ struct PfRing {
        measured: gate/up 134 us with one-block stages in three slots, 144 with two-block
        stages in three slots (two workgroups per CU), 125 with two in two; deeper rings were
        slower still, as fewer workgroups then hide each other's barriers and LDS latency.
-       Chunks of one token tile: PF_FEW_PAIRS. */
+       Chunks of one token tile: PF_RING_PAIRS. */
     static constexpr int P = P_;
     static_assert(RW % 64 == 0 && P >= 2 && WB % 16 == 0 && SB % 16 == 0 && SB <= 1024 && PP <= 16 &&
                       TT >= 1 && TT <= PF_CHUNK / 16 && R_Q_FITS(NA * KB + WI + 1, P) &&
-                      KB % KG == 0 && (KG == 1 || (TT == 1 && NA * KB == 4 * KG)),
+                      KB % KG == 0 && (KG == 1 || (TT == 1 && NA * KB == 4 * KG)) &&
+                      (SUMS == 1 || (TT == 1 && KG == 1)),
                   "ring geometry");
     /* the position of logical piece c of A row r: rows 16 * 4 / PP apart share banks, so the
        16 rows of an MFMA operand read land in distinct banks */
@@ -272,26 +282,19 @@ __device__ static void pf_loop(uint8_t *ring, int S, const uint16_t *x, size_t x
        off the error of one chain over all blocks (a layer at 16 tokens 3.5e-7 -> 2.8e-7 against 64
        bits; more tiles have no registers for it) */
     constexpr bool PARTS = R::TT == 1;
-    f32x4_t tot[PARTS ? R::NBT : 1][PARTS ? NMT : 1];
+    constexpr int NS = R::SUMS;
+    f32x4_t tot[PARTS ? NS : 1][PARTS ? R::NBT : 1], odd[R::NBT][R::TT];
     if constexpr (PARTS) {
 #pragma unroll
-        for (int n = 0; n < R::NBT; n++)
+        for (int n = 0; n < R::NBT; n++) {
 #pragma unroll
-            for (int mt = 0; mt < NMT; mt++) tot[n][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int u = 0; u < NS; u++) tot[u][n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            odd[n][0] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
     }
     for (int st = 0; st < R::P - 1; st++) issue();
     uint32_t get = 0;
-    for (int s = 0; s < S; s++) {
-        if constexpr (PARTS) {
-            if (s % PF_SUM == 0)
-#pragma unroll
-                for (int n = 0; n < R::NBT; n++)
-#pragma unroll
-                    for (int mt = 0; mt < NMT; mt++) {
-                        tot[n][mt] += acc[n][mt];
-                        acc[n][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                    }
-        }
+    auto stage = [&](f32x4_t (*acc)[R::TT]) __attribute__((always_inline)) {
         asm volatile("" ::: "memory");
         /* stage s has landed when at most the later stages' loads are in flight: Q per stage
            for a wavefront that loads A tiles, Q - QA for one that does not */
@@ -350,12 +353,29 @@ __device__ static void pf_loop(uint8_t *ring, int S, const uint16_t *x, size_t x
                     for (int i = 0; i < 4; i++) acc[n][mt][i] = fmaf(d, t[mt][i], acc[n][mt][i]);
             }
         }
+    };
+    for (int s = 0; s < S; s += NS) {
+        if constexpr (PARTS) {
+            if (s % (PF_SUM * NS) == 0)
+#pragma unroll
+                for (int n = 0; n < R::NBT; n++) {
+                    tot[0][n] += acc[n][0];
+                    acc[n][0] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    if constexpr (NS == 2) {
+                        tot[1][n] += odd[n][0];
+                        odd[n][0] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+                }
+        }
+        stage(acc);
+        if constexpr (NS == 2) stage(odd);
     }
     if constexpr (PARTS) {
 #pragma unroll
-        for (int n = 0; n < R::NBT; n++)
-#pragma unroll
-            for (int mt = 0; mt < NMT; mt++) acc[n][mt] += tot[n][mt];
+        for (int n = 0; n < R::NBT; n++) {
+            acc[n][0] += tot[0][n];
+            if constexpr (NS == 2) acc[n][0] += odd[n][0] + tot[1][n];
+        }
     }
     /* no load may still write this workgroup's LDS when it ends */
     asm volatile("" ::: "memory");
@@ -390,7 +410,7 @@ __device__ static void pf_loop(uint8_t *ring, int S, const uint16_t *x, size_t x
      (row stride n_out) for the pair of each position.
    TT < 4 (a ring for TT token tiles): every chunk holds at most 16 * TT tokens (the host
    guarantees it: batches of at most 16 * TT tokens, as a token's K experts are distinct). */
-template <int ENC, bool GU, int TT = PF_CHUNK / 16, int P = 2, int RW = 128, int KB = 2, int KG = 1>
+template <int ENC, bool GU, int TT = PF_CHUNK / 16, int P = 2, int RW = 128, int KB = 2, int KG = 1, int SUMS = 1>
 __global__ __launch_bounds__(PF_NT *KG) __attribute__((amdgpu_waves_per_eu(TT == 4 ? 3 : 1))) void k_pf_gemm(
     const uint8_t *__restrict__ experts, size_t exp_stride, size_t mat0, size_t mat_bytes,
     size_t payload_plane, int n_in, int n_out, const int *__restrict__ chunk_grp,
@@ -400,7 +420,7 @@ __global__ __launch_bounds__(PF_NT *KG) __attribute__((amdgpu_waves_per_eu(TT ==
     const _Float16 *__restrict__ xl, _Float16 *__restrict__ hh, _Float16 *__restrict__ hl,
     float *__restrict__ y, const int *__restrict__ sel, int npairs, int K, int E,
     int *__restrict__ ngroups) {
-    using R = PfRing<ENC, GU, TT, P, RW, KB, KG>;
+    using R = PfRing<ENC, GU, TT, P, RW, KB, KG, CPG_PL_F16, SUMS>;
     extern __shared__ __align__(16) uint8_t ring[];
     __shared__ int arow[PF_CHUNK], orow[PF_CHUNK];
     __shared__ uint64_t tab[32];
@@ -776,22 +796,28 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
     int rc;
     if (cpg_prefill_chunk(T, K, E) == 16) {
         /* chunks of one token tile */
-        auto tile = [&](auto groups, auto ring) {
-            constexpr int KG = groups, P = ring, KB = 2 * KG;
+        auto tile = [&](auto groups, auto ring, auto sums) {
+            constexpr int KG = groups, P = ring, KB = 2 * KG, SUMS = sums;
             using RG = PfRing<ENC, true, 1, P, PF_SMALL_RW_GU, KB, KG>;
             using RD = PfRing<ENC, false, 1, P, PF_SMALL_RW_DN, KB, KG>;
-            return gemms(RG::NT, k_pf_gemm<ENC, true, 1, P, PF_SMALL_RW_GU, KB, KG>,
+            return gemms(RG::NT, k_pf_gemm<ENC, true, 1, P, PF_SMALL_RW_GU, KB, KG, SUMS>,
                          (size_t)RG::P * RG::STAGE, RG::RW,
-                         k_pf_gemm<ENC, false, 1, P, PF_SMALL_RW_DN, KB, KG>,
+                         k_pf_gemm<ENC, false, 1, P, PF_SMALL_RW_DN, KB, KG, SUMS>,
                          (size_t)RD::P * RD::STAGE, RD::RW);
         };
-        using std::integral_constant;
-        if (T * K <= PF_FEW_PAIRS)
-            rc = tile(integral_constant<int, 2>{}, integral_constant<int, 2>{});
-        else if ((ENC == CPG_ENC_Q4) == (T * K > 2 * PF_FEW_PAIRS))
-            rc = tile(integral_constant<int, 1>{}, integral_constant<int, 2>{});
-        else
-            rc = tile(integral_constant<int, 1>{}, integral_constant<int, 3>{});
+        constexpr std::integral_constant<int, 1> one;
+        constexpr std::integral_constant<int, 2> two;
+        constexpr std::integral_constant<int, 3> three;
+        if (T * K <= PF_FEW_PAIRS) {
+            rc = tile(two, two, one);
+        } else if (T <= 16) {
+            if constexpr (ENC == CPG_ENC_Q4) rc = tile(one, three, two);
+            else rc = tile(one, two, two);
+        } else if ((ENC == CPG_ENC_Q4) == (T * K > PF_RING_PAIRS)) {
+            rc = tile(one, two, one);
+        } else {
+            rc = tile(one, three, one);
+        }
     } else {
         using RG = PfRing<ENC, true>;
         using RD = PfRing<ENC, false>;

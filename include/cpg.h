@@ -203,7 +203,9 @@ int cpg_moe_route_mode(int mode);
  *     accumulation) from 8 tokens, and from 2 where neither xn nor the router's logits are asked
  *     for; the grouped dequant-fused GEMVs for 2 to 7 tokens with either (there a token's
  *     outputs are those of one token with either, bit for bit); one token always the one-token
- *     GEMVs. Up to 16 tokens the experts' sums do not depend on the batch a token is in.
+ *     GEMVs. Among the MFMA calls of 2 to 16 tokens the experts' sums do not depend on the batch
+ *     a token is in, bit for bit; between them, one token, the GEMVs and more than 16 tokens they
+ *     agree to rounding.
  *   CPG_EXPERTS_GEMV / CPG_EXPERTS_MFMA: always the one path for T > 1 (for testing). */
 #define CPG_EXPERTS_AUTO 0
 #define CPG_EXPERTS_GEMV 1

@@ -602,6 +602,30 @@ def test_moe_small_certified_batch_invariance(small, T):
     assert rel_err(got["mlp"], gemv["mlp"]) <= SPLIT_TOL
 
 
+@pytest.mark.parametrize("enc", [4, 8])
+def test_moe_certified_batches_full_width(cpg, oracle, enc):
+    """Certified calls of 2 to 16 tokens at the model's width (D = 2048, F = 768, top-8: 16 and 6 or
+    32 and 12 stages of the one-tile GEMMs, past every ring's depth) against the oracle. A token's
+    outputs do not depend on the batch it is in, bit for bit: up to 8 tokens (64 pairs) two groups
+    of wavefronts sum its blocks, from 9 on one group in their order."""
+    from cachepotato_amd import synth
+    spec = synth.MoESpec(D=2048, E=16, K=8, F=768, enc=enc)
+    m = DeviceMoE(spec, max_T=16)
+    try:
+        x = synth.inputs(spec, 7300, 16)
+        want = oracle.moe(spec, m.wgate_host, synth.ln2(spec), m.host_mats, x, threads=8)
+        got = {T: m.forward(x[:T], outputs=False) for T in (2, 3, 7, 8, 9, 13, 16)}
+        for T, g in got.items():
+            assert np.array_equal(g["topk"], want["topk"][:T]), T
+            e = max(rel_err(g["mlp"][t], want["mlp"][t]) for t in range(T))
+            say(f"certified enc={enc} T={T}: worst token {e:.2e}")
+            assert e <= SPLIT_TOL, T
+            for k in ("topk", "wt", "mlp"):
+                assert np.array_equal(g[k].view(np.uint32), got[16][k][:T].view(np.uint32)), (T, k)
+    finally:
+        m.close()
+
+
 @pytest.mark.parametrize("T", [17, 32, 44, 45])
 def test_moe_small_crowded_experts_vs_oracle(cpg, oracle, small, T):
     """Every token takes the same experts, so each has T tokens: chunks of 16 (17 = one row past a
