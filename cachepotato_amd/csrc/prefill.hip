@@ -109,11 +109,14 @@ __global__ __launch_bounds__(256) void k_split_planes(const float *__restrict__ 
    tokens 60.0, 58.7, 16 skewed 58.4, 58.4; Q8_0 73.5, 76.6 and 69.2, 75.5; with two sums, as
    chosen, Q4_0 60.6 and 58.3, Q8_0 74.2 and 69.7.
    From 17 tokens, rings of two and three: Q4_0 20 tokens 101, 103, 45 tokens 117, 121, 96 tokens
-   120, 126, 160 tokens 138, 134; Q8_0 45 tokens 167, 155, 96 skewed 165, 156 */
+   120, 126, 128 tokens 123, 130, skewed 137, 133, and with more than 8 tokens per expert on average
+   160 tokens 138, 134, 176 tokens 140, 137, skewed 153, 150; Q8_0 20 tokens 137, 138, skewed 100,
+   107, 32 tokens 164, 151, 45 tokens 167, 155, 96 skewed 165, 156, 176 tokens 183, 182 */
 #define PF_SMALL_RW_GU 64
 #define PF_SMALL_RW_DN 128
 #define PF_FEW_PAIRS 64
-#define PF_RING_PAIRS 128
+#define PF_RING_Q4 128      /* pairs from which Q4_0 takes the ring of two, up to 8 tokens per expert */
+#define PF_RING_Q8 160      /* pairs up to which Q8_0 does */
 #define PF_SUM 4            /* pf_loop: stages whose sums are taken together, one token tile */
 #define R_Q_FITS(q, p) ((q) * ((p) - 2) < 64)   /* the stage wait's vmcnt fits its field */
 
@@ -152,7 +155,7 @@ struct PfRing {
        measured: gate/up 134 us with one-block stages in three slots, 144 with two-block
        stages in three slots (two workgroups per CU), 125 with two in two; deeper rings were
        slower still, as fewer workgroups then hide each other's barriers and LDS latency.
-       Chunks of one token tile: PF_RING_PAIRS. */
+       Chunks of one token tile: PF_RING_Q4, PF_RING_Q8. */
     static constexpr int P = P_;
     static_assert(RW % 64 == 0 && P >= 2 && WB % 16 == 0 && SB % 16 == 0 && SB <= 1024 && PP <= 16 &&
                       TT >= 1 && TT <= PF_CHUNK / 16 && R_Q_FITS(NA * KB + WI + 1, P) &&
@@ -731,10 +734,12 @@ static int max_chunks(int T, int K, int E, int ch) {
 /* Tokens per chunk of T tokens with K experts each: one tile of 16 while the experts have at most 11
    tokens each on average, so that most experts are one chunk: the one-tile GEMMs' smaller
    workgroups then keep more of the weights in flight (us per layer with the routing, chunks of 64 and
-   of 16, 128 experts top-8: 45 tokens Q4_0 122.7, 120.7, Q8_0 skewed 148.3, 135.0; 96 tokens 125.9,
-   126.1 and 170.8, 161.2; 144 tokens Q8_0 184.5, 173.0; 160 tokens Q8_0 184.9, 179.3, skewed 181.1,
-   182.8, Q4_0 skewed 138.8, 137.5). Above, the second chunks of crowded experts read their weights
-   again: 192 tokens 188.5, 184.4, skewed 185.2, 195.5, Q4_0 133.5, 134.8; 256 tokens 142, 155. */
+   of 16, 128 experts top-8: 45 tokens Q4_0 123.2, 117.0, Q8_0 skewed 145.9, 132.8; 96 tokens 126.8,
+   119.7 and 168.8, 156.1; 160 tokens Q4_0 136.8, 134.3, Q8_0 185.4, 179.7; 176 tokens 138.1, 137.4
+   and 187.5, 182.0). The second chunks of crowded experts read their weights again, so a skewed
+   choice of experts turns earlier: 160 tokens Q4_0 145.5, 146.0, Q8_0 183.5, 184.7; 176 tokens 149.4,
+   150.3 and 188.0, 191.4. Above, 192 tokens Q8_0 188.5, 184.4, skewed 185.2, 195.5, Q4_0 133.5,
+   134.8; 256 tokens 142, 155. */
 int cpg_prefill_chunk(int T, int K, int E) {
     return T <= 16 || T * K <= 11 * E ? 16 : PF_CHUNK;
 }
@@ -813,7 +818,7 @@ static int prefill_experts(const cpg_moe_layer *L, int T, const float *xn, const
         } else if (T <= 16) {
             if constexpr (ENC == CPG_ENC_Q4) rc = tile(one, three, two);
             else rc = tile(one, two, two);
-        } else if ((ENC == CPG_ENC_Q4) == (T * K > PF_RING_PAIRS)) {
+        } else if (ENC == CPG_ENC_Q4 ? T * K > PF_RING_Q4 && T * K <= 8 * E : T * K <= PF_RING_Q8) {
             rc = tile(one, two, one);
         } else {
             rc = tile(one, three, one);
