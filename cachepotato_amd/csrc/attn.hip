@@ -15,9 +15,10 @@
  *                    to the cache at pos0 + t.
  *   attention        T = 1: k_attn_split (or k_attn_decode); T > 1: k_attn_mma on MFMA for
  *                    head dim 128 and G = H/KV dividing 16, else k_attn_blk or k_attn_core.
- *                    Scores q.k_j / sqrtf(HD), softmax with the glibc-identical expf, the
- *                    weighted sum over positions; the sums run in another order than the
- *                    reference's serial loops (fp32, ~1e-7 to 1e-6 relative).
+ *                    Scores q.k_j / sqrtf(HD), softmax with the glibc-identical expf (k_attn_mma:
+ *                    with the hardware's fp32 power of two, 1 ulp), the weighted sum over
+ *                    positions; the sums run in another order than the reference's serial loops
+ *                    (fp32, ~1e-7 to 1e-6 relative).
  *   k_gemv           attn = Wo . ao.
  * From DENSE_MIN_T tokens on, both projections run as MFMA GEMMs instead (k_dense and
  * k_sum_parts of prefill.hip): k_rmsnorm_rows_planes writes ln1's output as the
@@ -518,12 +519,13 @@ __device__ static inline float half_sum(float v) {
    tokens, over split z of the block's keys, of which there are at most ns (ns == 1: one split
    with all of them; splits past the block's last leave at once). All rows share each tile of
    AMT key positions of kv head kh staged in LDS as hi/lo f16 halves (x = hi + lo, hi = f16(x),
-   lo = f16(x - hi): 22 significant bits), the query rows scaled by 8 log2(e) / sqrt(HD) in
+   lo = f16(x - hi): x to 2^-23 of itself from |x| = 2^-2 on, below that to 2^-25, as lo is then
+   one of f16's subnormals), the query rows scaled by 8 log2(e) / sqrt(HD) in
    double before the split (a scale of the scores rounded to fp32 would bend every softmax by the
    same 2^-24; 8 keeps the halves of a normed query's size). Per tile:
      S^T = K . Q^T on v_mfma_f32_16x16x32_f16 (A = key rows, B = the wavefront's query rows,
        held in registers for the whole call), each product as hi.hi + lo.hi + hi.lo (the lo.lo
-       term, below 2^-22 of the sum, is not formed); lane l then holds the scores of query
+       term, 2^-22 of the product at most, is not formed); lane l then holds the scores of query
        l%16 against keys 16kt + 4(l/16) + i (kt < 2, i < 4), masked where the tile reaches past
        one of the wavefront's positions (key j > the query's position, or past the cache: -inf);
      online softmax per query in powers of two: with M = (the largest score so far) / 8 the
@@ -538,15 +540,17 @@ __device__ static inline float half_sum(float v) {
    ns == 1: out = O / l, written as ao (fp32; FMT CPG_PL_NONE) or as the planes pl of the output
    projection. ns > 1: split z's O, M and l are left in pacc / pml at row (z*T + t)*H + h
    for k_attn_merge. The sums run in another order than the reference's two-pass softmax
-   (qwen3_moe.c:127-157) and the products carry 22-bit operands, so the output agrees to
-   rounding. Dynamic LDS: amma_lds_bytes().
+   (qwen3_moe.c:127-157), and the halves' 2^-25 holds for the probabilities too, of which the
+   largest so far is 1. Error of the attention half against 64 bits, before the splits and the hardware exponential and
+   now: 21 tokens over 700 positions 6.0e-7, 3.7e-7, 128 over 2000 8.4e-7, 4.2e-7, 512 over 3584
+   1.1e-6, 5.5e-7, 96 at position 0 3.1e-7, 3.0e-7. Dynamic LDS: amma_lds_bytes().
 
    What bounds it, at 512 tokens over 4096 positions: per tile and 32 rows of a wavefront 96
    MFMAs of 16 cycles, and beside them the operand reads from LDS and the softmax and staging
    on the VALU. Two sets of rows per wavefront (QS = 2) use each key and value operand read
    from LDS twice; tiles of 32 keys, double-buffered in 72 KiB, let two workgroups share a CU,
    so that one's MFMAs run beside the other's softmax; the splits fill the chip where the
-   query blocks do not. That kernel 365 -> 120 us (MFMAs 32 % of it), and 67 -> 9 at 21 tokens
+   query blocks do not. That kernel 365 -> 118 us (MFMAs busy 37 % of it), and 67 -> 9 at 21 tokens
    over 700 positions, against tiles of 64 keys over one set of rows, one workgroup per CU,
    unsplit, and an exponential in double precision. */
 #define AMT 32              /* k_attn_mma: key positions per tile */

@@ -74,17 +74,18 @@ __global__ __launch_bounds__(256) void k_split_planes(const float *__restrict__ 
 /* The expert GEMMs stream both operands through a ring of P stages in LDS, filled by direct
    global-to-LDS loads (global_load_lds_dwordx4: 16 bytes per lane, a wavefront's 64 lanes
    into 1 KiB of consecutive LDS), so loads in flight hold no registers and a stage is never
-   copied through them. A stage is one block of 32 of the k range:
-     A hi, A lo   the chunk's 64 activation rows, 32 halves each (a 64-byte row per token;
-                  a wavefront's 1 KiB is 16 rows), rows past the chunk repeating its last;
-                  16-byte piece c of row r sits at piece c ^ ((r >> 2) & 3) of its row, so
-                  the 16 rows one MFMA operand read touches fall in distinct LDS banks (rows
-                  64 bytes apart would put rows r and r + 4 in the same banks);
+   copied through them. A stage is KB blocks of 32 of the k range:
+     A planes     the chunk's 16 * TT activation rows, 32 * KB numbers each (64 * KB bytes per
+                  token and plane, NA planes; a wavefront's 1 KiB is 16 / KB rows), rows past the
+                  chunk repeating its last; 16-byte piece c of row r sits at piece apos(r, c) of its
+                  row, so that the 16 rows that one MFMA operand read touches fall in distinct
+                  LDS banks;
      W            NSEG 64-row segments of weight payload (the row-tiled layout keeps a
                   segment's block contiguous: 64 * PB bytes);
-     Sc           their fp16 scales, 128 bytes per segment.
-   Every wavefront issues the same number Q of loads per stage, so "stage s has landed" is
-   vmcnt <= Q * (P - 2) for each wavefront, followed by a barrier for the others' loads. The
+     Sc           their fp16 scales, 128 bytes per segment and block.
+   A wavefront issues the same number of loads in every stage (Q, or Q - QA where its token tile
+   is empty), so "stage s has landed" is that number times P - 2 or fewer in flight, for each
+   wavefront, followed by a barrier for the others' loads. The
    barrier is s_barrier alone: __syncthreads() would wait for every load in flight. The
    workgroup (4 wavefronts) computes RW rows of each of its matrices for the chunk; a
    wavefront RW/4 rows of each (RW 128, GU: gate rows, up rows: four 16-row B tiles; down: two).
@@ -411,8 +412,10 @@ __device__ static void pf_loop(uint8_t *ring, int S, const uint16_t *x, size_t x
      at the token's position in the group list (off + m0 + i), the A operand of the down GEMM.
    down: rows r0..r0+RW-1 of Wd (n_in = F) over hh/hl at the group-list positions; y[pair]
      (row stride n_out) for the pair of each position.
-   TT < 4 (a ring for TT token tiles): every chunk holds at most 16 * TT tokens (the host
-   guarantees it: batches of at most 16 * TT tokens, as a token's K experts are distinct). */
+   TT (a ring for TT token tiles): a chunk holds at most 16 * TT tokens, so the chunk list must have
+   been formed with ch = 16 * TT: its writers and this kernel's dispatch both take
+   cpg_prefill_chunk(T, K, E). With sel there is no list: there an expert's pairs are one chunk, at
+   most 16 as T <= 16 and a token's K experts are distinct. */
 template <int ENC, bool GU, int TT = PF_CHUNK / 16, int P = 2, int RW = 128, int KB = 2, int KG = 1, int SUMS = 1>
 __global__ __launch_bounds__(PF_NT *KG) __attribute__((amdgpu_waves_per_eu(TT == 4 ? 3 : 1))) void k_pf_gemm(
     const uint8_t *__restrict__ experts, size_t exp_stride, size_t mat0, size_t mat_bytes,

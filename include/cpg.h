@@ -217,11 +217,11 @@ int cpg_moe_expert_mode(int mode);
    the kernel's own execution, up to 8192 launches per kernel slot. cpg_moe_timing_read waits
    for them and returns, per slot, the summed milliseconds and the number of launches (arrays
    of at least min(n, CPG_KT_COUNT)), then clears the record. */
-#define CPG_KT_ROUTE 0      /* k_route_fast, k_route_small, k_rmsnorm_tok, k_router_tok */
+#define CPG_KT_ROUTE 0      /* k_route_fast, k_route_small, k_rmsnorm_tok, k_router_chain */
 #define CPG_KT_SELECT 1     /* k_select_bucket, k_select, k_bucket (exact routing), k_chunks,
                                k_split_planes */
-#define CPG_KT_GATEUP 2     /* k_gateup1, k_gateup_mm, k_mfma_gateup */
-#define CPG_KT_DOWN 3       /* k_down1, k_down_mm (with the weighted combine), k_mfma_down */
+#define CPG_KT_GATEUP 2     /* k_gateup1, k_gateup_mm, k_pf_gemm (gate/up) */
+#define CPG_KT_DOWN 3       /* k_down1, k_down_mm (with the weighted combine), k_pf_gemm (down) */
 #define CPG_KT_COMBINE 4    /* k_pair_combine (the prefill path's weighted combine) */
 #define CPG_KT_FUSED 5      /* k_moe1 (one token: routing, experts and combine in one launch) */
 #define CPG_KT_COUNT 6
@@ -263,7 +263,12 @@ void cpg_attn_ws_destroy(cpg_attn_ws *ws);
 /* T new tokens x (T, D) at positions pos0..pos0+T-1 (all device). kc, vc: the cache, cap
    rows of KV*HD floats; rows < pos0 are read, rows pos0..pos0+T-1 written. attn (T, D)
    receives the pre-residual attention output. -1 when pos0 + T exceeds cap, the RoPE table
-   or the workspace (qwen3_moe.c:94-97 refuses such a range). Asynchronous. */
+   or the workspace (qwen3_moe.c:94-97 refuses such a range). Asynchronous.
+   The position as an argument or on the device, the cache's length and the workspace's size do not
+   show in the bits; how many tokens share a call does, to rounding (T = 1, T > 1: other kernels; T
+   > 1: how the sums are split). From 33 tokens the projections take their inputs, and from 2
+   tokens the attention (HD = 128, H/KV a divisor of 16) takes queries, keys and values, as pairs of
+   f16 halves: beyond about 64000 they become infinite. */
 int cpg_attn_forward(const cpg_attn_layer *A, const float *x, int T, int pos0, float *kc,
                      float *vc, int cap, float *attn, cpg_attn_ws *ws);
 

@@ -565,7 +565,8 @@ def test_moe_q4_prefill512_golden(cpg, experts):
 def test_moe_small_mfma_vs_oracle(cpg, oracle, small, T):
     """The MFMA grouped GEMMs forced at small token counts (chunks of 1..64 tokens, Q4 and
     Q8 weights) against the oracle at both reference numerics; up to 16 tokens they run the
-    one-tile kernels (64 gate/up rows per workgroup, a deeper ring)."""
+    one-tile kernels (64 gate/up rows per workgroup; at top-4 up to 64 pairs, so in two groups of
+    wavefronts)."""
     import cachepotato_amd as C
     from cachepotato_amd import synth
     spec = small.spec
