@@ -20,11 +20,12 @@
  *   experts        one token: k_gateup1 (each workgroup ranks and certifies the router
  *                  records itself, then 32 rows of Wg and Wu of its expert, SwiGLU) and
  *                  k_down1 (all K experts' rows of a 64-row tile of Wd, the weighted combine
- *                  and the residual). 2-63 tokens: k_gateup_mm / k_down_mm, one workgroup per
- *                  (row tile, expert group) with the weights in registers and the group's
- *                  tokens 16 at a time on MFMA; the last of a token's K pairs to finish a
- *                  tile adds mlp += wt_j * y_j for that tile in slot order j = 0..K-1
- *                  (qwen3_moe.c:221). From 64 tokens: the MFMA grouped GEMMs of prefill.hip.
+ *                  and the residual). From 8 tokens, and from 2 on the certified routing: the
+ *                  MFMA grouped GEMMs of prefill.hip. 2-7 tokens otherwise: k_gateup_mm /
+ *                  k_down_mm, one workgroup per (row tile, expert group) with the weights in
+ *                  registers and the group's tokens 16 at a time on MFMA; the last of a token's
+ *                  K pairs to finish a tile adds mlp += wt_j * y_j for that tile in slot order
+ *                  j = 0..K-1 (qwen3_moe.c:221).
  * Workgroups of one launch hand results to each other only through agent-scope stores and
  * loads plus an arrival counter (see "cross-workgroup handoff"): a device-scope fence on
  * gfx950 writes back or invalidates a whole XCD's L2, which costs more than the work here.
@@ -51,7 +52,8 @@
    where a row's registers would not fit two wavefronts per SIMD */
 __host__ __device__ constexpr int route_rows(int nq) { return nq >= 16 ? 4 : 8; }
 #define XWAIT_SPINS 4096    /* k_gateup1: polls (of ~512 cycles) for workgroup 0's exact routing */
-#define PREFILL_MIN_T 8     /* from this many tokens the experts run as MFMA grouped GEMMs */
+#define PREFILL_MIN_T 8     /* from this many tokens the experts run as MFMA grouped GEMMs
+                               whatever the routing */
 
 /* ================================================================ serial sums */
 
@@ -2899,8 +2901,9 @@ static int moe_forward(const cpg_moe_layer *L, const float *x, const float *attn
     /* The expert products as MFMA grouped GEMMs (prefill.hip): from PREFILL_MIN_T tokens, and
        from two where the routing is the certified one, which writes their planes and whose
        selections they read (the batch GEMVs against them, us per layer with the routing: 2 tokens
-       Q4_0 43.5, 41.7, 4 tokens 62.9, 47.4, Q8_0 68.2, 51.3, 7 tokens 90.2, 57.1). A call that asks for xn or the router's logits keeps
-       the GEMVs below PREFILL_MIN_T: its outputs are those of one token at a time, bit for bit. */
+       Q4_0 43.5, 33.5, 4 tokens 62.8, 42.5, Q8_0 68.2, 48.0, 7 tokens 90.3, 54.5). A call that asks
+       for xn or the router's logits keeps the GEMVs below PREFILL_MIN_T: its outputs are those of
+       one token at a time, bit for bit. */
     const bool mfma = cpg_prefill_shape_ok(D, F) &&
                       cpg_prefill_scratch_bytes(T, D, K, F) <= (size_t)T * K * 2 * KS * F * 4 &&
                       (g_expert_mode == CPG_EXPERTS_MFMA ||

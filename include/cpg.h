@@ -205,7 +205,8 @@ int cpg_moe_route_mode(int mode);
  *     outputs are those of one token with either, bit for bit); one token always the one-token
  *     GEMVs. Among the MFMA calls of 2 to 16 tokens the experts' sums do not depend on the batch
  *     a token is in, bit for bit; between them, one token, the GEMVs and more than 16 tokens they
- *     agree to rounding.
+ *     agree to rounding. From 2 tokens xn and h are taken as pairs of f16 halves, here and in the
+ *     GEMVs: beyond 65504 they become infinite.
  *   CPG_EXPERTS_GEMV / CPG_EXPERTS_MFMA: always the one path for T > 1 (for testing). */
 #define CPG_EXPERTS_AUTO 0
 #define CPG_EXPERTS_GEMV 1
